@@ -41,7 +41,8 @@ struct GemmArgs {
 };
 
 GemmArgs gemm_args();
-// m_total: for gmode 1, the total rows over all groups (bounds the grid).
+// m_total: for gmode 1, the total rows over all groups (bounds the grid); for
+// gmode 2 the total K over all groups (chooses the tile).
 int gemm_launch(int ta, int tb, int epi, GemmArgs a, long m_total, hipStream_t st, const char* name);
 // Skinny products with n <= 16 columns (the gate projection): Y (T x n, ld n)
 // = X W + b, and G (K x n, ld n) = X^T D with db = column sums of D (db may be

@@ -1,5 +1,5 @@
-// f32 GEMM on the CDNA4 matrix cores (v_mfma_f32_16x16x4_f32), with the
-// operand/epilogue variants the model needs:
+// f32 GEMM on the CDNA4 matrix cores, with the operand/epilogue variants the
+// model needs:
 //
 //   C = alpha * op(A) op(B) (+ bias per column) (+ beta * C)
 //
@@ -18,17 +18,14 @@
 //   - split-K with f32 partials and a deterministic reduction, for the
 //     K = tokens weight-gradient products that have few output tiles.
 //
-// Tiling: 256 threads, a 128 x 128 block tile, k-tiles of 32 double-buffered
-// in LDS, four waves of 64 x 64.  Each operand keeps its global layout in LDS
-// (no transposing stores): a k-contiguous tile is [mn][k] with a 36-float row
-// stride, an mn-contiguous tile is [k][mn].  The MFMA k index is permuted
-// inside every 16-k group (step s, lane l uses k = 4 (l / 16) + s) so every
-// fragment read is one 16-byte ds_read: a [mn][k] read yields four k-steps of
-// one 16-row tile, a [k][mn] read yields one k-step of four tiles whose rows
-// are interleaved by 4.  The epilogue maps rows/columns back accordingly.
-// Plain products whose grid fills whole rounds of the CUs, and the grouped-K
-// expert weight gradients, take a 128 x 256 variant on 8 waves whose operand
-// tiles go from global memory straight into LDS (described at dma_mainloop).
+// The products run on the bf16 matrix cores with every f32 split in three (see
+// "f32 products on the bf16 matrix cores" below): block tiles of 128 x 256 and
+// 128 x 128 staged in LDS (gemm_k) and 64 x 64 with the k range dealt to the
+// block's waves (gemm_small_k); best_tile chooses.  The batched per-chunk
+// products of the chunked delta rule (gemm_batched_k) use
+// v_mfma_f32_16x16x4_f32 with k-tiles of 32 double-buffered in LDS.
+#include <limits.h>
+
 #include <mutex>
 #include <type_traits>
 
@@ -38,9 +35,13 @@
 
 namespace asca {
 
-// Block tiles are (64 WM) x (64 WN) with one 64 x 64 wave tile per wave:
-// 128 x 128 on 4 waves for the large products, 64 x 128 on 2 waves for the
-// 64-row batched per-chunk products of the chunked delta rule.
+// gemm_batched_k's tiles: (64 WM) x (64 WN) with one 64 x 64 wave tile per wave.
+// Each operand keeps its global layout in LDS: a k-contiguous tile is [mn][k]
+// with a 36-float row stride, an mn-contiguous tile is [k][mn].  The MFMA k
+// index is permuted inside every 16-k group (step s, lane l uses
+// k = 4 (l / 16) + s) so every fragment read is one 16-byte ds_read: a [mn][k]
+// read yields four k-steps of one 16-row tile, a [k][mn] read yields one k-step
+// of four tiles whose rows are interleaved by 4.
 constexpr int GM_BM = 128, GM_BN = 128, GM_BK = 32;
 constexpr int GM_LDK = GM_BK + 4;  // [mn][k] tile row stride (floats)
 
@@ -90,52 +91,6 @@ ASCA_DEV void tile_load(float4 (&r)[8 * R / NT], const float* base, long ld, con
     }
 }
 
-// Row offsets (source row * ld) of this thread's mn-rows of a k-contiguous
-// tile; they do not change along K, so they are read once per block.
-template <int R, int NT>
-ASCA_DEV void tile_rows(long (&ro)[8 * R / NT], long ld, const int* rows, long row_off, int mn0, int lim_mn,
-                        int tid) {
-#pragma unroll
-    for (int j = 0; j < 8 * R / NT; ++j) {
-        const int rr = (tid + NT * j) >> 3;
-        ro[j] = rr < lim_mn ? srow(rows, row_off, mn0 + rr) * ld : 0;
-    }
-}
-
-// Row offsets (source row * ld) of this thread's k-rows of an mn-contiguous
-// tile whose storage rows are gathered (rows != null): read one k-tile ahead
-// of its loads, so no load waits on the index read before it.  Rows past the
-// valid extent are clamped to the last valid one.
-template <int R, int NT>
-ASCA_DEV void tile_krows(long (&ro)[8 * R / NT], long ld, const int* rows, long row_off, long k0, long lim_k,
-                         int tid) {
-#pragma unroll
-    for (int j = 0; j < 8 * R / NT; ++j) {
-        const int kr = (tid + NT * j) / (R / 4);
-        ro[j] = (long)rows[row_off + k0 + min((long)kr, lim_k - 1)] * ld;
-    }
-}
-
-// As tile_load for a tile that lies wholly inside the operand (aligned, no
-// edge): unconditional 16-byte loads; a k-contiguous tile takes its row
-// offsets from tile_rows, a gathered mn-contiguous one from tile_krows.
-template <bool KC, int R, int NT>
-ASCA_DEV void tile_load_full(float4 (&r)[8 * R / NT], const float* base, long ld, const int* rows, long row_off,
-                             const long (&ro)[8 * R / NT], int mn0, long k0, int tid) {
-#pragma unroll
-    for (int j = 0; j < 8 * R / NT; ++j) {
-        const int sl = tid + NT * j;
-        if constexpr (KC) {
-            const int kk = 4 * (sl & 7);
-            r[j] = *reinterpret_cast<const float4*>(base + ro[j] + k0 + kk);
-        } else {
-            const int kr = sl / (R / 4), mm = 4 * (sl % (R / 4));
-            const long off = rows ? ro[j] : (row_off + k0 + kr) * ld;
-            r[j] = *reinterpret_cast<const float4*>(base + off + mn0 + mm);
-        }
-    }
-}
-
 template <bool KC, int R, int NT>
 ASCA_DEV void tile_store(const float4 (&r)[8 * R / NT], float* t, int tid) {
 #pragma unroll
@@ -175,453 +130,530 @@ ASCA_DEV void frag_read(float (&f)[4][4], const float* t, int w0, int h, int lan
     }
 }
 
-// As frag_read for NTL 16-row tiles (NTL = 2 or 4): the wave's 16 NTL
-// mn-rows starting at w0.  In the mn-contiguous layout tile x holds the rows
-// w0 + NTL i + x (i = lane % 16), one 8- or 16-byte read per k-step.
-template <bool KC, int R, int NTL>
-ASCA_DEV void frag_read_n(float (&f)[4][NTL], const float* t, int w0, int h, int lane) {
-    if constexpr (NTL == 4) {
-        frag_read<KC, R>(f, t, w0, h, lane);
-    } else if constexpr (KC) {
+// ---------------------------------------------------------------------------
+// f32 products on the bf16 matrix cores.
+//
+// Every operand value is split on its way into LDS into three bf16 values,
+// x = x0 + x1 + x2 with x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1 (each
+// rounded to nearest; a bf16 holds 8 bits, so the three hold all 24 of x and
+// both subtractions are exact).  A product of two splits is six bf16 products
+// (x2 y0, x0 y2, x1 y1, x1 y0, x0 y1, x0 y0), each exact in f32 and summed in
+// the f32 accumulator; the three left out are below 2^-25 of x y.  Six
+// v_mfma_f32_16x16x32_bf16 take 96 cycles where eight
+// v_mfma_f32_16x16x4_f32 take 256 (and those hold the SIMD's VALU besides),
+// and a sum is rounded 6 times per 32 terms instead of 8 times.
+//
+// The bf16 MFMA rounds its sums down (towards minus infinity: mean error -2.6e-8
+// of the rms at K = 512, where the f32 MFMA shows none), and a sum over many
+// rows of such a product (a bias gradient over 16384 tokens) adds these up: its
+// error was 3.7e-6 against 1.2e-6.  So odd rows of a tile are multiplied
+// negated and negated back at the end, which makes every second row's error
+// positive.
+//
+// A value that is not finite, or rounds to infinity in bf16, leaves a
+// non-finite sum wherever it enters: a wave that finds one among its sums
+// computes its tile again with f32 products (split_redo), so infinities and
+// NaN come out as the f32 products give them.
+//
+// LDS image of one operand tile (R rows x 32 k): three planes (x0, x1, x2) of
+// [k / 8][slot][8 bf16], 16 bytes per (row, k / 8), so every fragment read is
+// lane l reading slot l % 16 of k-group l / 16: one conflict-free ds_read_b128.
+// The k-group stride is 32 bytes over a multiple of 256, which keeps the eight
+// lanes of a write phase (two rows x four k-groups) on different banks.
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+// global accesses of 8 and 16 bytes at 4-byte alignment (one instruction)
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+constexpr int SP_BK = 32;
+
+// Elements c .. c + 3 of a run of n (> 0) valid floats, 0 past them: loads at
+// clamped places and no branch, since a conditional load is waited for on its
+// own.  at(i): element i.
+template <class F>
+ASCA_DEV f32x4 ld4_edge(int c, int n, F at) {
+    f32x4 v;
 #pragma unroll
-        for (int x = 0; x < NTL; ++x) {
-            const float4 v =
-                *reinterpret_cast<const float4*>(t + (w0 + 16 * x + (lane & 15)) * GM_LDK + 16 * h + 4 * (lane >> 4));
-            f[0][x] = v.x;
-            f[1][x] = v.y;
-            f[2][x] = v.z;
-            f[3][x] = v.w;
-        }
-    } else {
-        static_assert(NTL == 2, "tile count");
+    for (int e = 0; e < 4; ++e) v[e] = at(min(c + e, n - 1));
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const float2 v =
-                *reinterpret_cast<const float2*>(t + (16 * h + 4 * (lane >> 4) + s) * R + w0 + 2 * (lane & 15));
-            f[s][0] = v.x;
-            f[s][1] = v.y;
+    for (int e = 0; e < 4; ++e) v[e] = c + e < n ? v[e] : 0.0f;
+    return v;
+}
+template <int R>
+constexpr int sp_kg() { return 16 * R + 32; }  // bytes of one k-group of a plane
+template <int R>
+constexpr int sp_plane() { return 4 * sp_kg<R>(); }
+template <int R>
+constexpr int sp_tile() { return 3 * sp_plane<R>(); }
+
+ASCA_DEV unsigned pk_bf16(float a, float b) {
+    return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
+}
+// the three bf16 parts of a and b, a in the low half of each word
+ASCA_DEV void split2(float a, float b, unsigned& w0, unsigned& w1, unsigned& w2) {
+    w0 = pk_bf16(a, b);
+    a -= __uint_as_float(w0 << 16);
+    b -= __uint_as_float(w0 & 0xffff0000u);
+    w1 = pk_bf16(a, b);
+    a -= __uint_as_float(w1 << 16);
+    b -= __uint_as_float(w1 & 0xffff0000u);
+    w2 = pk_bf16(a, b);
+}
+
+// x, negated where `odd` is not zero (a power of two)
+ASCA_DEV float neg_if(float x, int odd) { return odd ? -x : x; }
+
+// A thread's share of one operand tile (R rows x 32 k on NT threads).
+//   KC (k-contiguous, stored [mn][k]): items of 8 consecutive k of one row,
+//     four threads to a row; slot = row.
+//   MC (mn-contiguous, stored [k][mn]): 4 k x W columns; lanes 2i, 2i + 1 hold
+//     the halves of one 8-k group.  Row 4 i + j of each 64 is slot 16 j + i, so
+//     a wave's four 16-slot tiles interleave by 4 and the epilogue finds four
+//     consecutive columns in one lane.
+// Rows past the operand's extent repeat a valid one (KC) or read as 0 (MC);
+// k past the range read as 0.
+// NEG: odd rows are stored negated.
+template <bool KC, bool GATHER, bool NEG, int R, int NT>
+struct SplitTile {
+    static constexpr int NI = KC ? R * 4 / NT : 1, W = R * 8 / NT, NF = R * 32 / NT;
+    const float* p[NI];
+    long ld;
+    int col, kofs;      // MC: column and k of the thread's piece within the tile
+    int idx[4];         // GATHER (MC): storage rows of the next k-tile
+    float x[NF];
+
+    ASCA_DEV void init(const float* base, long ld_, const int* rows, long off, int mn0, int lim_mn, long K_lo,
+                       long K_hi, int tid) {
+        ld = ld_;
+        if constexpr (KC) {
+            kofs = 8 * (tid & 3);
+#pragma unroll
+            for (int j = 0; j < NI; ++j) {
+                const int r = min((tid + NT * j) >> 2, lim_mn - 1);
+                p[j] = base + srow(rows, off, mn0 + r) * ld + K_lo + kofs;
+            }
+        } else {
+            const int lane = tid & 63, w = tid >> 6;
+            constexpr int NB = R / (W == 4 ? 128 : 64);  // column blocks of a wave's width
+            static_assert((NT / 64) == 4 * NB && (W == 2 || W == 4), "tile split");
+            kofs = 8 * (w / NB) + 4 * (lane & 1);
+            if constexpr (W == 4)
+                col = 128 * (w % NB) + 4 * (lane >> 1);
+            else
+                col = 64 * (w % NB) + 4 * ((lane >> 1) & 15) + 2 * (lane >> 5);
+            // a thread whose columns all lie past the extent repeats valid ones
+            const int cc = col < lim_mn ? col : 0;
+            p[0] = base + mn0 + cc + (GATHER ? 0 : (off + K_lo + kofs) * ld);
+            if constexpr (GATHER) next_rows(rows, off, K_lo, K_hi);
         }
     }
-}
-
-// acc (4 x TN tiles of 16 x 16) += the 16-k group whose fragments are fa, fb.
-template <int TN>
-ASCA_DEV void mfma_4xn(f32x4 (&acc)[4][TN], const float (&fa)[4][4], const float (&fb)[4][TN]) {
+    ASCA_DEV void next_rows(const int* rows, long off, long k0, long K_hi) {
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
+        for (int e = 0; e < 4; ++e) idx[e] = rows[off + min(k0 + kofs + e, K_hi - 1)];
+    }
+    // Whether every thread's columns of the tile are all valid or all past the extent.
+    ASCA_DEV static bool whole(int lim_mn) { return KC || lim_mn >= R || lim_mn % W == 0; }
+    // k-tile at K_lo + k.  WHOLE: all of its k are valid and whole(lim_mn).
+    template <bool WHOLE>
+    ASCA_DEV void load(long k, long lim_k, int lim_mn) {
+        if constexpr (KC) {
+            if constexpr (WHOLE) {
 #pragma unroll
-        for (int x = 0; x < 4; ++x)
+                for (int j = 0; j < NI; ++j) {
+                    const f32x4u a = *reinterpret_cast<const f32x4u*>(p[j] + k);
+                    const f32x4u b = *reinterpret_cast<const f32x4u*>(p[j] + k + 4);
 #pragma unroll
-            for (int y = 0; y < TN; ++y)
-                acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[s][x], fb[s][y], acc[x][y], 0, 0, 0);
-}
-
-// ---------------------------------------------------------------------------
-// Direct-to-LDS main loop (128 x 256 block tile, 8 waves of 64 x 64).
-//
-// The operand tiles go from global memory straight into LDS with
-// global_load_lds_dwordx4 (no register staging, no ds_write): each instruction
-// writes 64 lanes x 16 bytes contiguously at M0, and the lane -> global address
-// map is free, so every 1 KB chunk of a stage is laid out exactly as the MFMA
-// fragment reads want it: lane l reads the 16 bytes at chunk + 16 l (linear,
-// no bank conflict, no padding).  A stage is one k-tile of 16:
-//   k-contiguous operand ([mn][k] in memory): chunk c holds mn = 16 c + l % 16,
-//     k = 4 (l / 16) .. +3, i.e. the four k-steps of one 16-row tile;
-//   mn-contiguous operand ([k][mn]): chunk c holds k = 4 (l / 16) + c % 4,
-//     mn = 64 (c / 4) + 4 (l % 16) .. +3, i.e. one k-step of four tiles whose
-//     rows are interleaved by 4 (the same fragment semantics as the register
-//     path, so the epilogue is shared).
-// A (128 mn) has 8 chunks, B (256 mn) 16: wave w loads A chunk w and B chunks
-// 2w, 2w+1.  Three stages: step t waits for its own loads of tile t+1, passes
-// a barrier (every wave's part landed, every wave done reading tile t-1),
-// issues tile t+2 into the stage of tile t-1, reads the fragments of tile t+1
-// and multiplies tile t from registers.  Lanes whose k lies past the K range
-// load from a zero block instead (k tails, grouped K); rows past M or N are
-// clamped into the tile (their results are never stored).
-//
-// The loads are written as inline assembly: the compiler's own tracking of
-// LDS DMA makes every LDS read wait for all outstanding loads.  The loop waits
-// for them itself (s_waitcnt vmcnt(0) before each barrier), and waits for all
-// of them before the kernel ends, so no load lands in LDS after the block.
-constexpr int DMA_STAGES = 3, DMA_BK = 16;
-// bytes of one stage: 8 chunks of A (128 rows) and 4 WN of B (64 WN columns)
-template <int WN>
-constexpr int dma_stage_bytes() { return (8 + 4 * WN) * 1024; }
-
-__device__ float4 g_dma_zero = {0.f, 0.f, 0.f, 0.f};  // read-only source for k past the range
-
-ASCA_DEV void dma16(const float* g, unsigned lds_byte) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_byte), "v"(g) : "memory", "m0");
-}
-ASCA_DEV void dma_wait_all() { __builtin_amdgcn_s_waitcnt(0xF70); }  // vmcnt(0)
-
-// One lane's share of one chunk of an operand: source of the next k-tile.
-struct DmaSrc {
-    const float* p;  // k-contiguous, or mn-contiguous without row gather: source at the next k-tile
-    long step;       // advance per k-tile (floats)
-    long col;        // mn-contiguous: column of the lane's float4
-    int kofs;        // the lane's k within a k-tile
-    int idx;         // mn-contiguous with row gather: storage row of the next k-tile
+                    for (int e = 0; e < 4; ++e) {
+                        x[8 * j + e] = a[e];
+                        x[8 * j + 4 + e] = b[e];
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < NI; ++j) {
+                    const float* q = p[j] + k - kofs;
+                    const int lk = (int)min(lim_k, (long)SP_BK);
+                    const f32x4 a = ld4_edge(kofs, lk, [&](int i) { return q[i]; });
+                    const f32x4 b = ld4_edge(kofs + 4, lk, [&](int i) { return q[i]; });
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        x[8 * j + e] = a[e];
+                        x[8 * j + 4 + e] = b[e];
+                    }
+                }
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (!WHOLE) {
+                    const int lk = (int)min(lim_k, (long)SP_BK), ke = min(kofs + e, lk - 1);
+                    const float* q = GATHER ? p[0] + (long)idx[e] * ld : p[0] + (k + ke - kofs) * ld;
+                    const int cc = col < lim_mn ? col : 0;
+                    const f32x4 a = ld4_edge(col, lim_mn, [&](int i) { return q[i - cc]; });
+#pragma unroll
+                    for (int c = 0; c < W; ++c) x[W * e + c] = kofs + e < lim_k ? a[c] : 0.0f;
+                    continue;
+                }
+                const float* q = GATHER ? p[0] + (long)idx[e] * ld : p[0] + (k + e) * ld;
+                if constexpr (W == 4) {
+                    const f32x4u a = *reinterpret_cast<const f32x4u*>(q);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) x[4 * e + c] = a[c];
+                } else {
+                    const f32x2u a = *reinterpret_cast<const f32x2u*>(q);
+                    x[2 * e] = a[0];
+                    x[2 * e + 1] = a[1];
+                }
+            }
+        }
+    }
+    ASCA_DEV void store(char* t, int tid) const {
+        if constexpr (KC) {
+#pragma unroll
+            for (int j = 0; j < NI; ++j) {
+                const int it = tid + NT * j;
+                char* d = t + (it & 3) * sp_kg<R>() + (it >> 2) * 16;
+                static_assert(NT % 8 == 0, "a thread's rows share their parity");
+                float y[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) y[e] = NEG ? neg_if(x[8 * j + e], tid & 4) : x[8 * j + e];
+                uint4 w0, w1, w2;
+                split2(y[0], y[1], w0.x, w1.x, w2.x);
+                split2(y[2], y[3], w0.y, w1.y, w2.y);
+                split2(y[4], y[5], w0.z, w1.z, w2.z);
+                split2(y[6], y[7], w0.w, w1.w, w2.w);
+                *reinterpret_cast<uint4*>(d) = w0;
+                *reinterpret_cast<uint4*>(d + sp_plane<R>()) = w1;
+                *reinterpret_cast<uint4*>(d + 2 * sp_plane<R>()) = w2;
+            }
+        } else {
+            char* d = t + (kofs >> 3) * sp_kg<R>() + (kofs & 4) * 2 + ((col & ~63) + ((col >> 2) & 15)) * 16;
+#pragma unroll
+            for (int c = 0; c < W; ++c) {
+                const int o = (W == 4 ? c : (col & 2) + c) * 256;
+                constexpr float sg[2] = {1.0f, NEG ? -1.0f : 1.0f};
+                const float f = sg[c & 1];
+                uint2 w0, w1, w2;
+                split2(f * x[c], f * x[W + c], w0.x, w1.x, w2.x);
+                split2(f * x[2 * W + c], f * x[3 * W + c], w0.y, w1.y, w2.y);
+                *reinterpret_cast<uint2*>(d + o) = w0;
+                *reinterpret_cast<uint2*>(d + o + sp_plane<R>()) = w1;
+                *reinterpret_cast<uint2*>(d + o + 2 * sp_plane<R>()) = w2;
+            }
+        }
+    }
 };
 
-template <bool KC>
-ASCA_DEV DmaSrc dma_src(int c, int lane, const float* base, long ld, const int* rows, long row_off, int mn0,
-                        int lim_mn, long K_lo, long K_hi) {
-    DmaSrc d;
-    if constexpr (KC) {
-        int mn = 16 * c + (lane & 15);
-        if (mn >= lim_mn) mn = 0;
-        d.kofs = 4 * (lane >> 4);
-        d.p = base + srow(rows, row_off, mn0 + mn) * ld + K_lo + d.kofs;
-        d.step = DMA_BK;
-        d.col = 0;
-        d.idx = 0;
-    } else {
-        d.kofs = 4 * (lane >> 4) + (c & 3);
-        const int mm = min(64 * (c >> 2) + 4 * (lane & 15), lim_mn - 4);
-        d.col = mn0 + mm;
-        d.p = base + (row_off + K_lo + d.kofs) * ld + d.col;
-        d.step = (long)DMA_BK * ld;
-        d.idx = rows ? rows[row_off + min(K_lo + d.kofs, K_hi - 1)] : 0;
+// acc (64 x 64 of one wave) += the k-tile in LDS
+template <int RA, int RB>
+ASCA_DEV void split_mma(f32x4 (&acc)[4][4], const char* As, const char* Bs, int wm, int wn, int lane) {
+    const char* ap = As + (lane >> 4) * sp_kg<RA>() + (wm + (lane & 15)) * 16;
+    const char* bp = Bs + (lane >> 4) * sp_kg<RB>() + (wn + (lane & 15)) * 16;
+    bf16x8 a[3][4];
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[s][i] = *reinterpret_cast<const bf16x8*>(ap + s * sp_plane<RA>() + i * 256);
+#pragma unroll
+    for (int y = 0; y < 4; ++y) {
+        bf16x8 b[3];
+#pragma unroll
+        for (int s = 0; s < 3; ++s) b[s] = *reinterpret_cast<const bf16x8*>(bp + s * sp_plane<RB>() + y * 256);
+        constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+        for (int s = 0; s < 6; ++s)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                acc[i][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[PA[s]][i], b[PB[s]], acc[i][y], 0, 0, 0);
     }
-    return d;
 }
 
-// Issue k-tile t of one chunk into LDS byte address `dst`, then advance.  In
-// a k-tile that reaches past K_hi (`tail`, the last one at most) a lane whose
-// k is past K_hi reads the zero block.
+// One operand element (row mn0 + r, k) for split_redo; 0 outside the product
 template <bool KC>
-ASCA_DEV void dma_issue(DmaSrc& d, long t, const float* base, long ld, const int* rows, long row_off, long K_lo,
-                        long K_hi, bool tail, unsigned dst) {
-    const long k = K_lo + t * DMA_BK + d.kofs;
-    const float* src = d.p;
-    if constexpr (!KC) {
-        if (rows) {  // uniform
-            src = base + (long)d.idx * ld + d.col;
-            d.idx = rows[row_off + min(k + DMA_BK, K_hi - 1)];  // next k-tile's storage row
-        }
-    }
-    if (tail && k >= K_hi) src = reinterpret_cast<const float*>(&g_dma_zero);  // tail: uniform
-    d.p += d.step;
-    dma16(src, dst);
+ASCA_DEV float split_elem(const float* base, long ld, const int* rows, long off, int mn0, int r, int lim_mn, long k,
+                          long K_hi) {
+    if (r >= lim_mn || k >= K_hi) return 0.0f;
+    return KC ? base[srow(rows, off, mn0 + r) * ld + k] : base[srow(rows, off, k) * ld + mn0 + r];
 }
 
-template <bool TA, bool TB, int WN>
-ASCA_DEV void dma_mainloop(f32x4 (&acc)[4][4], const float* A, const float* B, const GemmArgs& p, long a_off,
-                           long b_off, int m0, int n0, int lim_m, int lim_n, long K_lo, long K_hi, int w, int lane,
-                           int wm, int wn) {
-    constexpr bool A_KC = !TA, B_KC = TB;
-    constexpr int STAGE_B = dma_stage_bytes<WN>();
-    constexpr int APW = 4 / WN;  // A chunks per wave (8 chunks over 2 WN waves); B chunks: 2 per wave
+// The sums of the NX x NY 16 x 16 tiles from (x0, y0) of a wave's 64 x 64 again,
+// as f32 products straight from memory.
+template <bool TA, bool TB, int NX, int NY>
+ASCA_DEV void split_redo(f32x4 (&acc)[NX][NY], int x0, int y0, const float* A, const float* B, const GemmArgs& p,
+                         long a_off, long b_off, int m0, int n0, int lim_m, int lim_n, long K_lo, long K_hi,
+                         int lane) {
+    const int i = lane & 15;
+#pragma unroll
+    for (int x = 0; x < NX; ++x)
+#pragma unroll
+        for (int y = 0; y < NY; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (long k = K_lo; k < K_hi; k += 4) {
+        const long kk = k + (lane >> 4);
+        float a[NX], b[NY];
+#pragma unroll
+        for (int x = 0; x < NX; ++x)
+            a[x] = split_elem<!TA>(A, p.lda, p.a_rows, a_off, m0, TA ? 4 * i + x0 + x : 16 * (x0 + x) + i, lim_m, kk,
+                                   K_hi);
+#pragma unroll
+        for (int y = 0; y < NY; ++y)
+            b[y] = split_elem<TB>(B, p.ldb, p.b_rows, b_off, n0, TB ? 16 * (y0 + y) + i : 4 * i + y0 + y, lim_n, kk,
+                                  K_hi);
+#pragma unroll
+        for (int x = 0; x < NX; ++x)
+#pragma unroll
+            for (int y = 0; y < NY; ++y)
+                acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[x], b[y], acc[x][y], 0, 0, 0);
+    }
+}
+
+// The sums of the rows that were multiplied negated (odd rows of the tile:
+// row 16 x + 4 (lane / 16) + r, or 4 i + x of an mn-contiguous A), negated back.
+template <bool TA, int NX, int NY>
+ASCA_DEV void split_sign(f32x4 (&acc)[NX][NY], int x0) {
+#pragma unroll
+    for (int x = 0; x < NX; ++x)
+#pragma unroll
+        for (int y = 0; y < NY; ++y)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[x][y][r] = neg_if(acc[x][y][r], (TA ? x0 + x : r) & 1);
+}
+
+// Any infinity or NaN among a wave's sums?
+template <int NX, int NY>
+ASCA_DEV bool split_bad(const f32x4 (&acc)[NX][NY]) {
+    float z = 0.0f;
+#pragma unroll
+    for (int x = 0; x < NX; ++x)
+#pragma unroll
+        for (int y = 0; y < NY; ++y)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) z = fmaf(acc[x][y][r], 0.0f, z);
+    return __any(z != z);
+}
+
+// Main loop: a k-tile of 32 per step, loaded into registers two steps ahead,
+// split and stored to LDS one step ahead.  DB: two LDS stages and one barrier
+// per step (146 KB for 128 x 256, one block per CU); otherwise one stage and
+// two barriers (49 KB for 128 x 128), the CU's other block filling the waits.
+// Bound: power.  At 4096^3 the 128 x 256 tile runs 225 TFLOP/s (f32 products on
+// the same shape: 139), 1350 TFLOP/s of bf16 products, and 258 on operands of
+// zeros; a plain bf16 product of torch runs 1130 there.  16384x1536x512
+// 208 -> 140 us, its input gradient 210 -> 126, its weight gradient 218 -> 143.
+template <bool TA, bool TB, int GATHER, int WM, int WN, bool DB>
+ASCA_DEV void split_mainloop(f32x4 (&acc)[4][4], const float* A, const float* B, const GemmArgs& p, long a_off,
+                             long b_off, int m0, int n0, int lim_m, int lim_n, long K_lo, long K_hi, int tid,
+                             int wm, int wn) {
+    constexpr int NT = 64 * WM * WN, RA = 64 * WM, RB = 64 * WN, ST = sp_tile<RA>() + sp_tile<RB>();
     extern __shared__ float4 lds4[];
-    const float4* lds = lds4;
-    const unsigned lds_b = (unsigned)(unsigned long)((__attribute__((address_space(3))) float4*)lds4);
-    const int wu = __builtin_amdgcn_readfirstlane(w);
-    DmaSrc sa[APW];
-#pragma unroll
-    for (int j = 0; j < APW; ++j)
-        sa[j] = dma_src<A_KC>(APW * wu + j, lane, A, p.lda, p.a_rows, a_off, m0, lim_m, K_lo, K_hi);
-    DmaSrc sb0 = dma_src<B_KC>(2 * wu, lane, B, p.ldb, p.b_rows, b_off, n0, lim_n, K_lo, K_hi);
-    DmaSrc sb1 = dma_src<B_KC>(2 * wu + 1, lane, B, p.ldb, p.b_rows, b_off, n0, lim_n, K_lo, K_hi);
-    const unsigned ca = lds_b + (unsigned)(APW * wu) * 1024u, cb = lds_b + (unsigned)(8 + 2 * wu) * 1024u;
-    // tile t into stage S (compile-time)
-    const long t_tail = (K_hi - K_lo) / DMA_BK;  // first k-tile not wholly inside the K range
-    // TL (compile-time): tile t may reach past K_hi (only then are the lanes'
-    // k checked against it)
-    auto issue = [&](long t, auto S, auto TL) {
-        constexpr unsigned so = (unsigned)decltype(S)::value * STAGE_B;
-        const bool tail = decltype(TL)::value && t >= t_tail;
-#pragma unroll
-        for (int j = 0; j < APW; ++j)
-            dma_issue<A_KC>(sa[j], t, A, p.lda, p.a_rows, a_off, K_lo, K_hi, tail, ca + 1024u * j + so);
-        dma_issue<B_KC>(sb0, t, B, p.ldb, p.b_rows, b_off, K_lo, K_hi, tail, cb + so);
-        dma_issue<B_KC>(sb1, t, B, p.ldb, p.b_rows, b_off, K_lo, K_hi, tail, cb + 1024u + so);
+    char* lds = reinterpret_cast<char*>(lds4);
+    const int lane = tid & 63;
+    SplitTile<!TA, GATHER == 1, true, RA, NT> ta;
+    SplitTile<TB, GATHER == 2, false, RB, NT> tb;
+    ta.init(A, p.lda, p.a_rows, a_off, m0, lim_m, K_lo, K_hi, tid);
+    tb.init(B, p.ldb, p.b_rows, b_off, n0, lim_n, K_lo, K_hi, tid);
+    const long nk = (K_hi - K_lo + SP_BK - 1) / SP_BK;  // > 0
+    const bool whole = ta.whole(lim_m) && tb.whole(lim_n);
+    const long nw = whole ? (K_hi - K_lo) / SP_BK : 0;  // k-tiles that load without checks
+    auto load_as = [&](long kt, auto Whole) {
+        constexpr bool wh = decltype(Whole)::value;
+        const long k = kt * SP_BK, lim_k = K_hi - K_lo - k;
+        ta.template load<wh>(k, lim_k, lim_m);
+        tb.template load<wh>(k, lim_k, lim_n);
+        const long kn = K_lo + min(kt + 1, nk - 1) * SP_BK;  // the storage rows of the k-tile after it
+        if constexpr (GATHER == 1) ta.next_rows(p.a_rows, a_off, kn, K_hi);
+        if constexpr (GATHER == 2) tb.next_rows(p.b_rows, b_off, kn, K_hi);
     };
-    float fa[2][4][4], fb[2][4][4];
-    // fragments of stage S into buffer BUF (both compile-time): 16-byte reads
-    // at chunk + 16 lane
-    const float4* rb = lds + lane;
-    const int ax = A_KC ? (wm >> 4) : (wm >> 6) * 4, bx = 8 + (B_KC ? (wn >> 4) : (wn >> 6) * 4);
-    auto rd = [&](auto S, auto BUF) {
-        constexpr int st = decltype(S)::value * (STAGE_B / 16), buf = decltype(BUF)::value;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float4 v = rb[st + (ax + i) * 64];
-            if constexpr (A_KC) {
-                fa[buf][0][i] = v.x; fa[buf][1][i] = v.y; fa[buf][2][i] = v.z; fa[buf][3][i] = v.w;
-            } else {
-                fa[buf][i][0] = v.x; fa[buf][i][1] = v.y; fa[buf][i][2] = v.z; fa[buf][i][3] = v.w;
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float4 v = rb[st + (bx + i) * 64];
-            if constexpr (B_KC) {
-                fb[buf][0][i] = v.x; fb[buf][1][i] = v.y; fb[buf][2][i] = v.z; fb[buf][3][i] = v.w;
-            } else {
-                fb[buf][i][0] = v.x; fb[buf][i][1] = v.y; fb[buf][i][2] = v.z; fb[buf][i][3] = v.w;
-            }
-        }
+    auto load = [&](long kt) {
+        if (kt < nw)
+            load_as(kt, std::true_type{});
+        else if (kt < nk)
+            load_as(kt, std::false_type{});
     };
-    using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, 1>;
-    using I2 = std::integral_constant<int, 2>;
-    const long nk = (K_hi - K_lo + DMA_BK - 1) / DMA_BK;  // > 0
-    using Tail = std::true_type;
-    using NoTail = std::false_type;
-    issue(0, I0{}, Tail{});
-    if (nk > 1) issue(1, I1{}, Tail{});
-    dma_wait_all();
-    __syncthreads();
-    rd(I0{}, I0{});
-    // Step t at phase P = t % 6: tile t in buffer P % 2 and stage P % 3.
-    // The scheduling barriers keep the fragment reads for the next step ahead
-    // of the products and the next step's wait and barrier behind them (left
-    // alone, the compiler moved the reads down to the barrier, whose wait then
-    // fell on them).
-    auto step = [&](long t, auto P, auto TL) {
-        constexpr int ph = decltype(P)::value;
-        dma_wait_all();
-        __syncthreads();
-        if (t + 2 < nk) issue(t + 2, std::integral_constant<int, (ph + 2) % 3>{}, TL);
-        rd(std::integral_constant<int, (ph + 1) % 3>{}, std::integral_constant<int, (ph + 1) % 2>{});
-        __builtin_amdgcn_sched_barrier(0);
-        mfma_4xn<4>(acc, fa[ph % 2], fb[ph % 2]);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    using P3 = std::integral_constant<int, 3>;
-    using P4 = std::integral_constant<int, 4>;
-    using P5 = std::integral_constant<int, 5>;
+    load(0);
+    ta.store(lds, tid);
+    tb.store(lds + sp_tile<RA>(), tid);
+    load(1);
+    lds_barrier();
     long t = 0;
-    // steps whose issued tile t + 2 lies wholly inside the K range (t + 2 < t_tail)
-    for (; t + 6 < nk && t + 7 < t_tail; t += 6) {
-        step(t, I0{}, NoTail{});
-        step(t + 1, I1{}, NoTail{});
-        step(t + 2, I2{}, NoTail{});
-        step(t + 3, P3{}, NoTail{});
-        step(t + 4, P4{}, NoTail{});
-        step(t + 5, P5{}, NoTail{});
-    }
-    for (; t + 6 < nk; t += 6) {
-        step(t, I0{}, Tail{});
-        step(t + 1, I1{}, Tail{});
-        step(t + 2, I2{}, Tail{});
-        step(t + 3, P3{}, Tail{});
-        step(t + 4, P4{}, Tail{});
-        step(t + 5, P5{}, Tail{});
-    }
-    // the last 1..6 steps (the fragments read past the last tile are unused)
-    do {
-        step(t, I0{}, Tail{});
-        if (t + 1 >= nk) break;
-        step(t + 1, I1{}, Tail{});
-        if (t + 2 >= nk) break;
-        step(t + 2, I2{}, Tail{});
-        if (t + 3 >= nk) break;
-        step(t + 3, P3{}, Tail{});
-        if (t + 4 >= nk) break;
-        step(t + 4, P4{}, Tail{});
-        if (t + 5 >= nk) break;
-        step(t + 5, P5{}, Tail{});
-    } while (false);
-    dma_wait_all();
+    // Step t: k-tile t multiplied from its stage, t + 1 split and stored, t + 2
+    // loaded.  The steps whose loads need no checks run in a loop of their own:
+    // without branches the splits and the products of a step interleave.
+    auto step = [&](auto Whole) {
+        char* cur = lds + (DB && (t & 1) ? ST : 0);
+        char* nxt = lds + (DB && !(t & 1) ? ST : 0);
+        split_mma<RA, RB>(acc, cur, cur + sp_tile<RA>(), wm, wn, lane);
+        if constexpr (!DB) lds_barrier();
+        ta.store(nxt, tid);  // (past the last k-tile: not read)
+        tb.store(nxt + sp_tile<RA>(), tid);
+        if constexpr (decltype(Whole)::value)
+            load_as(t + 2, Whole);
+        else
+            load(t + 2);
+        if constexpr (DB && decltype(Whole)::value) {
+            // order of the step's instructions: fragment reads ahead of their
+            // products, splits and stores spread between the last 72 products
+            // (left alone the compiler puts all splits first, the matrix cores
+            // idle: 4096^3 641 -> 620 us)
+            __builtin_amdgcn_sched_group_barrier(0x100, 15, 0);
+            __builtin_amdgcn_sched_group_barrier(0x8, 12, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+            __builtin_amdgcn_sched_group_barrier(0x8, 12, 0);
+#pragma unroll
+            for (int q = 0; q < 9; ++q) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x2, 2, 0);
+                }
+                if (q == 1 || q == 4) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+                __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+            }
+        }
+        lds_barrier();
+    };
+    for (; t + 2 < nw; ++t) step(std::true_type{});
+    for (; t < nk; ++t) step(std::false_type{});
+    split_sign<TA>(acc, 0);
+    if (split_bad(acc))
+        split_redo<TA, TB>(acc, 0, 0, A, B, p, a_off, b_off, m0 + wm, n0 + wn, lim_m - wm, lim_n - wn, K_lo, K_hi, lane);
 }
 
-// Block tile (64 WM) x (16 TNW WN) on WM x WN waves; a wave owns 64 rows x
-// 16 TNW columns (TNW = 4, or 2 for the narrower tile that lets three blocks
-// share a CU).
-template <bool TA, bool TB, int EPI, bool VEC, int WM, int WN, int TNW = 4, bool DMA = false>
-__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(WM * WN >= 4 ? 2 : 1))) void gemm_k(GemmArgs p) {
-    constexpr int NT = 64 * WM * WN, BM = 64 * WM, BN = 16 * TNW * WN;
-    constexpr bool A_KC = !TA, B_KC = TB;
-    constexpr int A_F = tile_floats<A_KC, BM>();
-    constexpr int B_F = tile_floats<B_KC, BN>();
-    extern __shared__ float4 lds4[];
-    float* lds = reinterpret_cast<float*>(lds4);
-
-    // block -> tile, XCD-aware: hardware places block i on XCD i % 8, so give
-    // each XCD a contiguous run of logical tiles (neighbours share operand rows)
-    int L = blockIdx.x;
-    const int nb = gridDim.x;
-    if ((nb & 7) == 0) L = (L & 7) * (nb >> 3) + (L >> 3);
-    int g = 0, tm, tn = L % p.tiles_n;
-    int Mg = p.M;
-    long K_lo = 0, K_hi = p.K, goff_g = 0;
-    if (p.gmode == 1) {
-        int mt = L / p.tiles_n;
-        for (; g < p.ngroups; ++g) {
-            const int a = p.goff[g], b = p.goff[g + 1];
-            const int nt = (b - a + BM - 1) / BM;
-            if (mt < nt) break;
-            mt -= nt;
-        }
-        if (g >= p.ngroups) return;  // surplus block (grid is an upper bound)
-        tm = mt;
-        goff_g = p.goff[g];
-        Mg = p.goff[g + 1] - p.goff[g];
-    } else if (p.gmode == 2) {
-        const int r = L / p.tiles_n;
-        tm = r % p.tiles_m;
-        g = r / p.tiles_m;
-        goff_g = p.goff[g];
-        K_hi = p.goff[g + 1] - p.goff[g];
-    } else if (p.gmode == 3) {
-        const int r = L / p.tiles_n;
-        tm = r % p.tiles_m;
-        g = r / p.tiles_m;
-    } else {
-        tm = L / p.tiles_n;
-        K_lo = (long)blockIdx.y * p.k_per_split;
-        K_hi = min((long)p.K, K_lo + p.k_per_split);
-    }
-    const int m0 = tm * BM, n0 = tn * BN;
-    const float* A = p.A + g * p.a_gs;
-    const float* B = p.B + g * p.b_gs;
-    float* C = p.C + g * p.c_gs + (long)blockIdx.y * p.c_split_stride;
-    const float* bias = p.bias ? p.bias + g * p.bias_gs : nullptr;
-    const float* resid = p.resid ? p.resid + g * p.r_gs : nullptr;
-    const long a_off = ((p.gmode == 1 && !TA) || (p.gmode == 2 && TA)) ? goff_g : 0;
-    const long b_off = (p.gmode == 2 && !TB) ? goff_g : 0;
-
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int wm = (w / WN) * 64, wn = (w % WN) * 16 * TNW;
-    const int lim_m = Mg - m0, lim_n = p.N - n0;
-
-    f32x4 acc[4][TNW];
-#pragma unroll
-    for (int x = 0; x < 4; ++x)
-#pragma unroll
-        for (int y = 0; y < TNW; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    if constexpr (DMA) {
-        static_assert(WM == 2 && (WN == 4 || WN == 2) && TNW == 4 && VEC, "direct-to-LDS tile");
-        if (K_hi > K_lo)
-            dma_mainloop<TA, TB, WN>(acc, A, B, p, a_off, b_off, m0, n0, lim_m, lim_n, K_lo, K_hi, w, lane, wm, wn);
-    } else {
-    const long nk = (K_hi - K_lo + GM_BK - 1) / GM_BK;
-    float4 ra[8 * BM / NT], rb[8 * BN / NT];
-    // interior blocks (whole tiles in M and N) load without edge checks,
-    // except in a partial last k-tile
-    const bool interior = VEC && lim_m >= BM && lim_n >= BN;
-    long roa[8 * BM / NT], rob[8 * BN / NT];
-    if (A_KC) tile_rows<BM, NT>(roa, p.lda, p.a_rows, a_off, m0, lim_m, tid);
-    if (B_KC) tile_rows<BN, NT>(rob, p.ldb, p.b_rows, b_off, n0, lim_n, tid);
-    // gathered mn-contiguous operands: the row offsets of k-tile kt
-    auto krows = [&](long kt) {
-        const long k0 = K_lo + min(kt, nk - 1) * GM_BK;
-        if (!A_KC && p.a_rows) tile_krows<BM, NT>(roa, p.lda, p.a_rows, a_off, k0, K_hi - k0, tid);
-        if (!B_KC && p.b_rows) tile_krows<BN, NT>(rob, p.ldb, p.b_rows, b_off, k0, K_hi - k0, tid);
-    };
-    auto load = [&](long k0) {
-        if (interior && K_hi - k0 >= GM_BK) {
-            tile_load_full<A_KC, BM, NT>(ra, A, p.lda, p.a_rows, a_off, roa, m0, k0, tid);
-            tile_load_full<B_KC, BN, NT>(rb, B, p.ldb, p.b_rows, b_off, rob, n0, k0, tid);
+// The tile, group and K range of a block.
+template <bool TA, bool TB, int BM, int BN>
+struct BlockTile {
+    int m0, n0, lim_m, lim_n, Mg;
+    long K_lo, K_hi, goff_g, a_off, b_off;
+    const float *A, *B, *bias, *resid;
+    float* C;
+    // false: a surplus block (a grouped grid is an upper bound)
+    ASCA_DEV bool init(const GemmArgs& p) {
+        // block -> tile, XCD-aware: hardware places block i on XCD i % 8, so give
+        // each XCD a contiguous run of logical tiles (neighbours share operand rows)
+        int L = blockIdx.x;
+        const int nb = gridDim.x;
+        if ((nb & 7) == 0) L = (L & 7) * (nb >> 3) + (L >> 3);
+        int g = 0, tm, tn = L % p.tiles_n;
+        Mg = p.M;
+        K_lo = 0;
+        K_hi = p.K;
+        goff_g = 0;
+        if (p.gmode == 1) {
+            int mt = L / p.tiles_n;
+            for (; g < p.ngroups; ++g) {
+                const int a = p.goff[g], b = p.goff[g + 1];
+                const int nt = (b - a + BM - 1) / BM;
+                if (mt < nt) break;
+                mt -= nt;
+            }
+            if (g >= p.ngroups) return false;
+            tm = mt;
+            goff_g = p.goff[g];
+            Mg = p.goff[g + 1] - p.goff[g];
+        } else if (p.gmode == 2) {
+            const int r = L / p.tiles_n;
+            tm = r % p.tiles_m;
+            g = r / p.tiles_m;
+            goff_g = p.goff[g];
+            K_hi = p.goff[g + 1] - p.goff[g];
+        } else if (p.gmode == 3) {
+            const int r = L / p.tiles_n;
+            tm = r % p.tiles_m;
+            g = r / p.tiles_m;
         } else {
-            tile_load<A_KC, VEC, BM, NT>(ra, A, p.lda, p.a_rows, a_off, m0, lim_m, k0, K_hi - k0, tid);
-            tile_load<B_KC, VEC, BN, NT>(rb, B, p.ldb, p.b_rows, b_off, n0, lim_n, k0, K_hi - k0, tid);
+            tm = L / p.tiles_n;
+            K_lo = (long)blockIdx.y * p.k_per_split;
+            K_hi = min((long)p.K, K_lo + p.k_per_split);
         }
-    };
-    // Two halves per k-tile kt, split by one barrier.  Each half multiplies
-    // fragments that are already in registers while the other half's
-    // fragments are read:
-    //   A(kt): MFMAs of 16-k group 0 of kt | read group 1 of kt; store the
-    //          registers holding k-tile kt+1 to the other LDS buffer
-    //   B(kt): MFMAs of group 1 of kt | read group 0 of kt+1; issue the
-    //          global loads of k-tile kt+2 into the registers
-    // so a global load has a whole half plus most of the next to arrive.  The
-    // buffer written in A(kt) was last read in A(kt-1), before the barrier of
-    // kt-1.  Near the end the k-tile loaded is clamped to the last one (a
-    // repeated load that is never stored).
-    float fa0[4][4], fb0[4][TNW], fa1[4][4], fb1[4][TNW];
-    if (nk > 0) {
-        krows(0);
-        load(K_lo);
-        krows(1);
-        tile_store<A_KC, BM, NT>(ra, lds, tid);
-        tile_store<B_KC, BN, NT>(rb, lds + A_F, tid);
-        load(K_lo + (nk > 1 ? GM_BK : 0));
-        krows(2);
-        __syncthreads();
-        frag_read<A_KC, BM>(fa0, lds, wm, 0, lane);
-        frag_read_n<B_KC, BN, TNW>(fb0, lds + A_F, wn, 0, lane);
-        for (long kt = 0; kt < nk - 1; ++kt) {
-            float* const Cs = lds + (kt & 1) * (A_F + B_F);
-            float* const Ns = lds + ((kt + 1) & 1) * (A_F + B_F);
-            frag_read<A_KC, BM>(fa1, Cs, wm, 1, lane);
-            frag_read_n<B_KC, BN, TNW>(fb1, Cs + A_F, wn, 1, lane);
-            mfma_4xn<TNW>(acc, fa0, fb0);
-            tile_store<A_KC, BM, NT>(ra, Ns, tid);
-            tile_store<B_KC, BN, NT>(rb, Ns + A_F, tid);
-            __syncthreads();
-            frag_read<A_KC, BM>(fa0, Ns, wm, 0, lane);
-            frag_read_n<B_KC, BN, TNW>(fb0, Ns + A_F, wn, 0, lane);
-            load(K_lo + min(kt + 2, nk - 1) * GM_BK);
-            krows(kt + 3);
-            mfma_4xn<TNW>(acc, fa1, fb1);
-        }
-        float* const Ls = lds + ((nk - 1) & 1) * (A_F + B_F);
-        frag_read<A_KC, BM>(fa1, Ls, wm, 1, lane);
-        frag_read_n<B_KC, BN, TNW>(fb1, Ls + A_F, wn, 1, lane);
-        mfma_4xn<TNW>(acc, fa0, fb0);
-        mfma_4xn<TNW>(acc, fa1, fb1);
+        m0 = tm * BM;
+        n0 = tn * BN;
+        lim_m = Mg - m0;
+        lim_n = p.N - n0;
+        A = p.A + g * p.a_gs;
+        B = p.B + g * p.b_gs;
+        C = p.C + g * p.c_gs + (long)blockIdx.y * p.c_split_stride;
+        bias = p.bias ? p.bias + g * p.bias_gs : nullptr;
+        resid = p.resid ? p.resid + g * p.r_gs : nullptr;
+        a_off = ((p.gmode == 1 && !TA) || (p.gmode == 2 && TA)) ? goff_g : 0;
+        b_off = (p.gmode == 2 && !TB) ? goff_g : 0;
+        return true;
     }
-    }
+};
 
-    // epilogue: result register r of tile (x, y) sits at tile row 4 (lane / 16) + r,
+template <int N>
+ASCA_DEV void store_row(float* d, const float (&o)[N]) {
+    if constexpr (N == 4)
+        *reinterpret_cast<f32x4u*>(d) = f32x4u{o[0], o[1], o[2], o[3]};
+    else
+        *reinterpret_cast<f32x2u*>(d) = f32x2u{o[0], o[1]};
+}
+
+// C of the NX x NY 16 x 16 tiles from (x0, y0) of the wave's 64 x 64 at (m0, n0).
+template <bool TA, bool TB, int EPI, int NX, int NY, class T>
+ASCA_DEV void gemm_epilogue(const f32x4 (&acc)[NX][NY], int x0, int y0, int m0, int n0, const T& t, const GemmArgs& p,
+                            int lane) {
+    constexpr bool A_KC = !TA, B_KC = TB;
+    float* const C = t.C;
+    const float *const bias = t.bias, *const resid = t.resid;
+    const int Mg = t.Mg;
+    const long goff_g = t.goff_g;
+    // result register r of tile (x, y) sits at tile row 4 (lane / 16) + r,
     // tile column lane % 16.  Element y of a lane's row is column nc0 + NS y.
     // Every load the epilogue needs is unconditional (indices clamped into the
     // operand) and issued ahead of its use: the bias once per thread, the scatter
     // indices, residual, C and pre of four rows at a time.  A load under a
     // per-element condition is waited for on its own, one latency per element.
     constexpr int NS = B_KC ? 16 : 1;
-    const int nc0 = B_KC ? n0 + wn + (lane & 15) : n0 + wn + TNW * (lane & 15);
+    const int nc0 = B_KC ? n0 + 16 * y0 + (lane & 15) : n0 + 4 * (lane & 15) + y0;
     const int nmax = p.N - 1;
-    float bv[TNW];
+    float bv[NY];
     if (bias) {
 #pragma unroll
-        for (int y = 0; y < TNW; ++y) bv[y] = bias[min(nc0 + NS * y, nmax)];
+        for (int y = 0; y < NY; ++y) bv[y] = bias[min(nc0 + NS * y, nmax)];
     }
     const bool add_c = EPI == EPI_STORE && p.beta != 0.0f;
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
+    for (int x = 0; x < NX; ++x) {
         long srt[4], crow[4];
         bool rok[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int tr = 4 * (lane >> 4) + r;
-            const int m = m0 + wm + (A_KC ? 16 * x + tr : 4 * tr + x);
+            const int m = m0 + (A_KC ? 16 * (x0 + x) + tr : 4 * tr + x0 + x);
             rok[r] = m < Mg;
             srt[r] = (p.gmode == 1 ? goff_g : 0) + min(m, Mg - 1);
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) crow[r] = p.c_rows ? (long)p.c_rows[srt[r]] : srt[r];
-        float lr[4][TNW], lc[4][TNW], la[4][TNW];
+        float lr[4][NY], lc[4][NY], la[4][NY];
         if constexpr (EPI == EPI_STORE) {
             if (resid) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
 #pragma unroll
-                    for (int y = 0; y < TNW; ++y) lr[r][y] = resid[crow[r] * p.ld_resid + min(nc0 + NS * y, nmax)];
+                    for (int y = 0; y < NY; ++y) lr[r][y] = resid[crow[r] * p.ld_resid + min(nc0 + NS * y, nmax)];
             }
             if (add_c) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
 #pragma unroll
-                    for (int y = 0; y < TNW; ++y) lc[r][y] = C[crow[r] * p.ldc + min(nc0 + NS * y, nmax)];
+                    for (int y = 0; y < NY; ++y) lc[r][y] = C[crow[r] * p.ldc + min(nc0 + NS * y, nmax)];
             }
         } else if constexpr (EPI == EPI_SILU_BWD) {
 #pragma unroll
             for (int r = 0; r < 4; ++r)
 #pragma unroll
-                for (int y = 0; y < TNW; ++y) la[r][y] = p.aux[srt[r] * p.ld_aux + min(nc0 + NS * y, nmax)];
+                for (int y = 0; y < NY; ++y) la[r][y] = p.aux[srt[r] * p.ld_aux + min(nc0 + NS * y, nmax)];
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             if (!rok[r]) continue;
             float* Cr = C + crow[r] * p.ldc;
-            float o[TNW], hb[TNW];
+            float o[NY], hb[NY];
 #pragma unroll
-            for (int y = 0; y < TNW; ++y) {
+            for (int y = 0; y < NY; ++y) {
                 float a = p.alpha * acc[x][y][r];
                 if (bias) a += bv[y];
                 if constexpr (EPI == EPI_STORE) {
@@ -637,22 +669,16 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(WM
                 o[y] = a;
             }
             if constexpr (!B_KC) {
-                // columns nc0 .. nc0 + TNW - 1 of one row
+                // columns nc0 .. nc0 + NY - 1 of one row
                 if (nc0 >= p.N) continue;
-                const int cnt = min(p.N - nc0, TNW);
+                const int cnt = min(p.N - nc0, NY);
                 const long ao = srt[r] * p.ld_aux + nc0;
-                if (VEC && cnt == TNW && TNW == 4) {
-                    *reinterpret_cast<float4*>(Cr + nc0) = make_float4(o[0], o[1], o[TNW - 2], o[TNW - 1]);
-                    if constexpr (EPI == EPI_SILU)
-                        *reinterpret_cast<float4*>(p.aux_out + ao) =
-                            make_float4(hb[0], hb[1], hb[TNW - 2], hb[TNW - 1]);
-                } else if (VEC && cnt == TNW && TNW == 2) {
-                    *reinterpret_cast<float2*>(Cr + nc0) = make_float2(o[0], o[TNW - 1]);
-                    if constexpr (EPI == EPI_SILU)
-                        *reinterpret_cast<float2*>(p.aux_out + ao) = make_float2(hb[0], hb[TNW - 1]);
+                if (cnt == NY) {
+                    store_row<NY>(Cr + nc0, o);
+                    if constexpr (EPI == EPI_SILU) store_row<NY>(p.aux_out + ao, hb);
                 } else {
 #pragma unroll
-                    for (int y = 0; y < TNW; ++y)
+                    for (int y = 0; y < NY; ++y)
                         if (y < cnt) {
                             Cr[nc0 + y] = o[y];
                             if constexpr (EPI == EPI_SILU) p.aux_out[ao + y] = hb[y];
@@ -660,7 +686,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(WM
                 }
             } else {
 #pragma unroll
-                for (int y = 0; y < TNW; ++y) {
+                for (int y = 0; y < NY; ++y) {
                     const int n = nc0 + 16 * y;
                     if (n >= p.N) continue;
                     Cr[n] = o[y];
@@ -669,6 +695,206 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(WM
             }
         }
     }
+}
+
+// Block tile (64 WM) x (64 WN) on WM x WN waves; a wave owns 64 x 64.
+template <bool TA, bool TB, int EPI, int GATHER, int WM, int WN, bool DB>
+__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_k(GemmArgs p) {
+    BlockTile<TA, TB, 64 * WM, 64 * WN> t;
+    if (!t.init(p)) return;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int wm = (w / WN) * 64, wn = (w % WN) * 64;
+    f32x4 acc[4][4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (t.K_hi > t.K_lo)
+        split_mainloop<TA, TB, GATHER, WM, WN, DB>(acc, t.A, t.B, p, t.a_off, t.b_off, t.m0, t.n0, t.lim_m, t.lim_n,
+                                                   t.K_lo, t.K_hi, tid, wm, wn);
+    gemm_epilogue<TA, TB, EPI>(acc, 0, 0, t.m0 + wm, t.n0 + wn, t, p, lane);
+}
+
+// Products too small to fill the chip with the tiles above: one 64 x 64 tile
+// per block, the k-tiles dealt to its NW waves, whose sums are added through
+// LDS at the end (in wave order).  Nothing is staged: a wave loads its
+// fragments from memory (k-contiguous operands 8 k of one row per lane,
+// mn-contiguous ones 8 k of four columns) and splits them in registers, so
+// the loop has no barrier and a wave's next k-tile loads behind its products.
+// Loads are buffer loads (32-bit lane offsets, the k-tile's offset in a scalar
+// register: 64-bit addresses would take the registers the fragments need), so
+// an operand's rows must lie within 4 GB (small_fits).
+// NEG: odd rows negated.
+template <bool KC, bool GATHER, bool NEG>
+struct FragTile {
+    const float* base;           // KC: k = K_lo of row 0; MC: k = K_lo of the tile's first column
+    unsigned vo[KC ? 4 : 1];     // lane's byte offsets: KC: row 16 x + i at its k; MC: its k and column 4 i
+    long ld;
+    int kofs, col;
+    f32x4 x[8];  // KC: [2 x + half]; MC: [k]
+    ASCA_DEV void init(const float* b, long ld_, const int* rows, long off, int mn0, int lim_mn, long K_lo, int lane) {
+        ld = ld_;
+        kofs = 8 * (lane >> 4);
+        col = 4 * (lane & 15);
+        if constexpr (KC) {
+            base = b + (rows ? 0 : (off + mn0) * ld) + K_lo;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int r = min(16 * j + (lane & 15), lim_mn - 1);
+                vo[j] = (unsigned)(((rows ? rows[off + mn0 + r] : r) * ld + kofs) * 4);
+            }
+        } else {
+            base = b + mn0 + (GATHER ? 0 : (off + K_lo) * ld);
+            vo[0] = (unsigned)(((GATHER ? 0 : kofs * ld) + (col < lim_mn ? col : 0)) * 4);
+        }
+    }
+    ASCA_DEV static bool whole(int lim_mn) { return KC || lim_mn >= 64 || lim_mn % 4 == 0; }
+    static ASCA_DEV f32x4 ld4(Rsrc r, unsigned vo, unsigned so) {
+        const float4 v = buf_load4(r, vo, so);
+        return f32x4{v.x, v.y, v.z, v.w};
+    }
+    // k-tile at K_lo + k; WHOLE: no k past the range, whole(lim_mn)
+    template <bool WHOLE>
+    ASCA_DEV void load(const int* rows, long off, long K_lo, long k, long lim_k, int lim_mn) {
+        const int lk = (int)min(lim_k, (long)SP_BK);
+        if constexpr (KC) {
+            const Rsrc r = make_rsrc(base + k, ~0u);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    if constexpr (WHOLE) {
+                        x[2 * j + h] = ld4(r, vo[j], 16 * h);
+                    } else {
+                        const unsigned v = vo[j] - 4 * kofs;
+                        x[2 * j + h] = ld4_edge(kofs + 4 * h, lk, [&](int i) { return buf_load1(r, v + 4 * i, 0); });
+                    }
+                }
+        } else {
+            const Rsrc r = make_rsrc(base + (GATHER ? 0 : k * ld), ~0u);
+            const unsigned l4 = (unsigned)(4 * ld);
+            unsigned v[8], so[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int ke = WHOLE ? kofs + e : min(kofs + e, lk - 1);
+                v[e] = GATHER ? vo[0] + rows[off + K_lo + k + ke] * l4 : WHOLE ? vo[0] : vo[0] + (ke - kofs) * l4;
+                so[e] = GATHER || !WHOLE ? 0 : e * l4;
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                if constexpr (WHOLE) {
+                    x[e] = ld4(r, v[e], so[e]);
+                } else {
+                    const unsigned c0 = v[e] - 4 * (col < lim_mn ? col : 0);
+                    const f32x4 u = ld4_edge(col, lim_mn, [&](int i) { return buf_load1(r, c0 + 4 * i, 0); });
+                    x[e] = kofs + e < lk ? u : f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+            }
+        }
+    }
+    // the three bf16 fragments of 16-row tile j
+    ASCA_DEV void frag(int j, bf16x8 (&f)[3]) const {
+        typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+        u32x4 w[3];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float a = KC ? x[2 * j + e / 2][2 * (e & 1)] : x[2 * e][j];
+            float b = KC ? x[2 * j + e / 2][2 * (e & 1) + 1] : x[2 * e + 1][j];
+            if constexpr (NEG) {
+                a = neg_if(a, KC ? col & 4 : j & 1);  // col / 4 = lane % 16: the KC lane's row
+                b = neg_if(b, KC ? col & 4 : j & 1);
+            }
+            unsigned w0, w1, w2;
+            split2(a, b, w0, w1, w2);
+            w[0][e] = w0;
+            w[1][e] = w1;
+            w[2][e] = w2;
+        }
+#pragma unroll
+        for (int s = 0; s < 3; ++s) f[s] = __builtin_bit_cast(bf16x8, w[s]);
+    }
+};
+
+constexpr int SM_NW = 8;  // waves of a small-product block
+template <bool TA, bool TB, int EPI, int GATHER>
+__global__ __launch_bounds__(64 * SM_NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_small_k(GemmArgs p) {
+    BlockTile<TA, TB, 64, 64> t;
+    if (!t.init(p)) return;
+    extern __shared__ float4 lds4[];
+    f32x4* const part = reinterpret_cast<f32x4*>(lds4);  // [wave][tile][lane]
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    f32x4 acc[4][4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const long nk = (t.K_hi - t.K_lo + SP_BK - 1) / SP_BK;
+    if (w < nk) {
+        FragTile<!TA, GATHER == 1, true> fa;
+        FragTile<TB, GATHER == 2, false> fb;
+        fa.init(t.A, p.lda, p.a_rows, t.a_off, t.m0, t.lim_m, t.K_lo, lane);
+        fb.init(t.B, p.ldb, p.b_rows, t.b_off, t.n0, t.lim_n, t.K_lo, lane);
+        const bool whole = fa.whole(t.lim_m) && fb.whole(t.lim_n);
+        auto load_a = [&](long kt) {
+            const long k = kt * SP_BK, lim_k = t.K_hi - t.K_lo - k;
+            if (whole && lim_k >= SP_BK)
+                fa.template load<true>(p.a_rows, t.a_off, t.K_lo, k, lim_k, t.lim_m);
+            else
+                fa.template load<false>(p.a_rows, t.a_off, t.K_lo, k, lim_k, t.lim_m);
+        };
+        auto load_b = [&](long kt) {
+            const long k = kt * SP_BK, lim_k = t.K_hi - t.K_lo - k;
+            if (whole && lim_k >= SP_BK)
+                fb.template load<true>(p.b_rows, t.b_off, t.K_lo, k, lim_k, t.lim_n);
+            else
+                fb.template load<false>(p.b_rows, t.b_off, t.K_lo, k, lim_k, t.lim_n);
+        };
+        load_a(w);
+        load_b(w);
+#pragma unroll 1
+        for (long kt = w;;) {
+            bf16x8 a[4][3];
+#pragma unroll
+            for (int x = 0; x < 4; ++x) fa.frag(x, a[x]);
+            kt += SM_NW;
+            if (kt < nk) load_a(kt);
+            // one column tile at a time: its fragments are split beside the
+            // products of the one before (all at once, the registers spill)
+#pragma unroll
+            for (int y = 0; y < 4; ++y) {
+                bf16x8 b[3];
+                fb.frag(y, b);
+                constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+                for (int s = 0; s < 6; ++s)
+#pragma unroll
+                    for (int x = 0; x < 4; ++x)
+                        acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[x][PA[s]], b[PB[s]], acc[x][y], 0, 0, 0);
+                if (y < 3) __builtin_amdgcn_sched_barrier(0);
+            }
+            if (kt < nk) load_b(kt);
+            if (kt >= nk) break;
+        }
+    }
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) part[(w * 16 + 4 * x + y) * 64 + lane] = acc[x][y];
+    lds_barrier();
+    // wave w adds up and stores tiles (w / 2, 2 (w % 2)) and the one beside it
+    const int x0 = w >> 1, y0 = 2 * (w & 1);
+    f32x4 sum[1][2];
+#pragma unroll
+    for (int y = 0; y < 2; ++y) {
+        sum[0][y] = part[(4 * x0 + y0 + y) * 64 + lane];
+#pragma unroll
+        for (int v = 1; v < SM_NW; ++v) sum[0][y] += part[(v * 16 + 4 * x0 + y0 + y) * 64 + lane];
+    }
+    split_sign<TA>(sum, x0);
+    if (split_bad(sum))
+        split_redo<TA, TB>(sum, x0, y0, t.A, t.B, p, t.a_off, t.b_off, t.m0, t.n0, t.lim_m, t.lim_n, t.K_lo, t.K_hi, lane);
+    gemm_epilogue<TA, TB, EPI>(sum, x0, y0, t.m0, t.n0, t, p, lane);
 }
 
 // Persistent batched products (gmode 3, plain epilogue): a block walks work
@@ -894,23 +1120,65 @@ static int ws_check(const Ws& ws, size_t floats, const char* name) {
     return ASCA_OK;
 }
 
-template <bool TA, bool TB, int EPI, bool VEC, int WM = 2, int WN = 2, int TNW = 4, bool DMA = false>
+template <bool TA, bool TB, int EPI, int GATHER, int WM, int WN, bool DB>
 static int launch_gemm_t(const GemmArgs& a, dim3 grid, hipStream_t st) {
-    constexpr size_t lds =
-        DMA ? (size_t)DMA_STAGES * dma_stage_bytes<WN>()
-            : 2 * (size_t)(tile_floats<!TA, 64 * WM>() + tile_floats<TB, 16 * TNW * WN>()) * sizeof(float);
-    if (int arc = allow_lds(reinterpret_cast<const void*>(&gemm_k<TA, TB, EPI, VEC, WM, WN, TNW, DMA>), lds)) return arc;
-    hipLaunchKernelGGL((gemm_k<TA, TB, EPI, VEC, WM, WN, TNW, DMA>), grid, dim3(64 * WM * WN), lds, st, a);
+    constexpr size_t lds = (size_t)(DB ? 2 : 1) * (sp_tile<64 * WM>() + sp_tile<64 * WN>());
+    if (int arc = allow_lds(reinterpret_cast<const void*>(&gemm_k<TA, TB, EPI, GATHER, WM, WN, DB>), lds)) return arc;
+    hipLaunchKernelGGL((gemm_k<TA, TB, EPI, GATHER, WM, WN, DB>), grid, dim3(64 * WM * WN), lds, st, a);
     return ASCA_OK;
 }
 
-// Fraction of the block slots used over the rounds a launch of `tiles` blocks
-// takes, `per_cu` blocks resident per CU.
-static double round_fill(long tiles, int per_cu) {
-    const long slots = (long)per_cu * (cu_count() > 0 ? cu_count() : 256);
-    const long rounds = (tiles + slots - 1) / slots;
-    return rounds ? (double)tiles / (double)(rounds * slots) : 1.0;
+template <bool TA, bool TB, int EPI, int GATHER>
+static int launch_small_t(const GemmArgs& a, dim3 grid, hipStream_t st) {
+    constexpr size_t lds = (size_t)SM_NW * 64 * 64 * sizeof(float);
+    if (int arc = allow_lds(reinterpret_cast<const void*>(&gemm_small_k<TA, TB, EPI, GATHER>), lds)) return arc;
+    hipLaunchKernelGGL((gemm_small_k<TA, TB, EPI, GATHER>), grid, dim3(64 * SM_NW), lds, st, a);
+    return ASCA_OK;
 }
+
+// Which tile a product takes: the one whose time on the device this model puts
+// lowest.  Measured on MI355X, per k-tile of 32 (steps of them), a CU at a time:
+//   WIDE  (128 x 256, one block per CU)  2.5 us    (4096^3: 225 TFLOP/s against 195 with 128 x 128)
+//   T128  (128 x 128)                    1.75 us alone on its CU, 2.8 us for two blocks side by side
+//   SMALL (64 x 64, k-tiles over 8 waves) 3.5 us for eight k-tiles
+// and 3-5 us of first loads, sums and stores per round of blocks.  Products
+// that fill the chip with the large tiles take those (a 64 x 64 tile splits
+// each value for 64 products instead of 128 or 256); where those leave CUs idle
+// the small tile wins: 1000x1000x320 22 -> 9.5 us, 64x1536x512 30 -> 11 us,
+// 1000x320x1000 55 -> 19 us.
+enum Tile { T_SMALL, T_128, T_WIDE };
+static double tile_us(Tile t, long tiles, long steps) {
+    const long cus = cu_count() > 0 ? cu_count() : 256;
+    const double s = (double)steps;
+    if (t == T_SMALL) return (double)((tiles + cus - 1) / cus) * (3.5 * (double)((steps + 7) / 8) + 3.0);
+    if (t == T_WIDE) return (double)((tiles + cus - 1) / cus) * (2.5 * s + 5.0);
+    const long full = tiles / (2 * cus), rem = tiles % (2 * cus);
+    return (double)full * (2.8 * s + 4.0) + (rem == 0 ? 0.0 : rem <= cus ? 1.75 * s + 5.0 : 2.8 * s + 4.0);
+}
+// tiles of an M x N product (rows in `groups` buckets of about M / groups when grouped)
+static long tile_count(Tile t, long M, long N, int groups) {
+    const long bm = t == T_SMALL ? 64 : 128, bn = t == T_SMALL ? 64 : t == T_WIDE ? 256 : 128;
+    const long tn = (N + bn - 1) / bn;
+    if (groups <= 0) return (M + bm - 1) / bm * tn;
+    return (groups * ((M / groups + bm - 1) / bm) + (groups + 1) / 2) * tn;
+}
+static Tile best_tile(long M, long N, int groups, long mult, long steps, bool small_ok, double* us) {
+    Tile best = T_WIDE;
+    double t = tile_us(T_WIDE, mult * tile_count(T_WIDE, M, N, groups), steps);
+    for (Tile c : {T_128, T_SMALL}) {
+        if (c == T_SMALL && !small_ok) continue;
+        const double u = tile_us(c, mult * tile_count(c, M, N, groups), steps);
+        if (u < t) {
+            t = u;
+            best = c;
+        }
+    }
+    if (us) *us = t;
+    return best;
+}
+// The small tile addresses an operand tile with 32-bit byte offsets: 64 rows
+// (or 32 k-rows) of the leading dimension, or all `rows` of a gathered operand.
+static bool small_fits(long ld, long rows) { return ld <= (1L << 22) && rows <= (1L << 30) / ld; }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
@@ -943,58 +1211,23 @@ int gemm_launch(int ta, int tb, int epi, GemmArgs a, long m_total, hipStream_t s
                      (!a.aux_out || aligned16(a.aux_out)) && (a.a_gs % 4 == 0) && (a.b_gs % 4 == 0) &&
                      (a.c_gs % 4 == 0) && (a.c_split_stride % 4 == 0);
     // batched per-chunk products with at most 64 rows use 64 x 128 tiles
-    const int wm = (a.gmode == 3 && vec && a.M <= 64) ? 1 : 2;
-    const int wn = 2;  // a 64 x 64 tile needs 8 staged float4 per operand per lane and spills
-    // block count for a block-tile width bn
-    auto count = [&](int bn) -> long {
-        const long tn = (a.N + bn - 1) / bn, tm = (a.M + 64 * wm - 1) / (64 * wm);
-        const long splits = a.gmode == 0 && a.k_per_split > 0 ? (a.K + a.k_per_split - 1) / a.k_per_split : 1;
-        if (a.gmode == 1) return ((m_total + GM_BM - 1) / GM_BM + a.ngroups) * tn;
-        if (a.gmode == 2 || a.gmode == 3) return (long)a.ngroups * tm * tn;
-        return tm * tn * splits;
-    };
-    // 128 x 64 tiles when the 128 x 128 grid would leave a mostly idle last
-    // round.  Measured per-flop efficiency of the narrow tile against the wide
-    // one: ~0.8 with two blocks per CU (NN, NT), ~0.95 with three (A^T)
-    const size_t lds64 = 2 * (size_t)(ta ? GM_BK * 128 : 128 * GM_LDK) * sizeof(float) +
-                         2 * (size_t)(tb ? 64 * GM_LDK : GM_BK * 64) * sizeof(float);
-    // resident narrow blocks per CU: LDS, and registers (the A^T variants fit
-    // three waves per SIMD, the others two)
-    const int per_cu64 = (int)min((size_t)(ta ? 3 : 2), (size_t)(160 * 1024) / lds64);
-    const bool narrow =
-        vec && wm == 2 && a.gmode != 3 &&
-        round_fill(count(64), per_cu64) * (per_cu64 >= 3 ? 0.95 : 0.8) > round_fill(count(128), 2);
-    // Direct-to-LDS 128 x 256 tiles (one 8-wave block per CU) where every
-    // operand float4 is whole (k-contiguous operands need K in multiples of 4,
-    // mn-contiguous ones M or N) and the grid (tiles x K splits) fills whole
-    // rounds of the CUs.  Measured against the 128 x 128 register-staged tile:
-    // 5-9% faster on plain products with full rounds (16384 x {1536, 512} x 512
-    // NN and NT, 4096^3) and on the grouped-K expert weight gradients, and on
-    // the split-K weight gradients (512x1536x16384 TN, ten splits: 272 -> 243
-    // us; the configs[3] training step 21.55 -> 20.83 ms); slower with a partly
-    // empty last round and on the grouped-row products.
-    const bool kc_any = !ta || tb;
-    const bool dma_ops = vec && (!kc_any || a.K % 4 == 0) && (!ta || a.M % 4 == 0) && (tb || a.N % 4 == 0) &&
-                         a.N >= 4 && (!ta || a.M >= 4);
-    const bool dma_ok = dma_ops && (a.gmode == 0 || a.gmode == 2);
-    auto count_dma = [&]() -> long {
-        const long tn = (a.N + 255) / 256, tm = (a.M + 127) / 128;
-        const long sp = a.gmode == 0 && a.k_per_split > 0 ? (a.K + a.k_per_split - 1) / a.k_per_split : 1;
-        return a.gmode == 2 ? (long)a.ngroups * tm * tn : tm * tn * sp;
-    };
-    const bool dma = dma_ok && wm == 2 && round_fill(count_dma(), 1) >= 0.9;
-    // otherwise the same loads on a 128 x 128 tile (4 waves, two blocks per CU)
-    // for the grouped-row expert products and the other plain products
-    // (measured: MoE forward 466 -> 439 us, backward 903 -> 840 us, the
-    // 16384x256x512 head 52 -> 48 us, 512x1536x16384 TN split ten ways on
-    // this tile 272 -> 258 us)
-    const bool dma128 = !dma && dma_ops && wm == 2 && (a.gmode == 1 || a.gmode == 0);
-    const int bn = dma ? 256 : dma128 ? 128 : narrow ? 64 : 128;
+    const int wm = (a.gmode == 3 && vec && a.K > 0 && a.M <= 64) ? 1 : 2;
+    const bool batched = a.gmode == 3 && vec && a.K > 0;
+    const long splits = a.gmode == 0 && a.k_per_split > 0 ? (a.K + a.k_per_split - 1) / a.k_per_split : 1;
+    if (a.gmode != 0 || a.k_per_split <= 0) a.k_per_split = a.K;
+    // rows the gathered operands' indices can reach (grouped K: m_total rows in all)
+    const long grows = a.gmode == 0 && (a.a_rows || a.b_rows) ? LONG_MAX : m_total;
+    const bool small_ok = small_fits(max(a.lda, 1L), a.a_rows ? grows : 64) &&
+                          small_fits(max(a.ldb, 1L), a.b_rows ? grows : 64);
+    const long k_each = a.gmode == 2 ? m_total / max(a.ngroups, 1) : a.k_per_split;
+    const Tile tile = best_tile(a.gmode == 1 ? m_total : a.M, a.N, a.gmode == 1 ? a.ngroups : 0,
+                                a.gmode >= 2 ? a.ngroups : splits, (k_each + SP_BK - 1) / SP_BK, small_ok, nullptr);
+    const int bm = tile == T_SMALL ? 64 : GM_BM, bn = batched ? 128 : tile == T_SMALL ? 64 : tile == T_WIDE ? 256 : 128;
     a.tiles_n = (a.N + bn - 1) / bn;
-    a.tiles_m = (a.M + 64 * wm - 1) / (64 * wm);
+    a.tiles_m = batched ? (a.M + 64 * wm - 1) / (64 * wm) : (a.M + bm - 1) / bm;
     long blocks;
     if (a.gmode == 1)
-        blocks = ((m_total + GM_BM - 1) / GM_BM + a.ngroups) * a.tiles_n;
+        blocks = ((m_total + bm - 1) / bm + a.ngroups) * a.tiles_n;
     else if (a.gmode == 2 || a.gmode == 3)
         blocks = (long)a.ngroups * a.tiles_m * a.tiles_n;
     else
@@ -1003,26 +1236,23 @@ int gemm_launch(int ta, int tb, int epi, GemmArgs a, long m_total, hipStream_t s
     if (blocks > 0x7fffffffL) return fail(ASCA_ERR_INVALID, "%s: grid too large", name);
     int rc = pre_launch(name);
     if (rc) return rc;
-    const dim3 grid((unsigned)blocks, (unsigned)(a.gmode == 0 && a.k_per_split > 0 ? (a.K + a.k_per_split - 1) / a.k_per_split : 1));
-    if (a.gmode != 0 || a.k_per_split <= 0) a.k_per_split = a.K;
-#define ASCA_GEMM_CASE(TA_, TB_, EPI_)                                                                  \
-    if (ta == TA_ && tb == TB_ && epi == EPI_)                                                          \
-        rc = !vec ? launch_gemm_t<TA_, TB_, EPI_, false>(a, grid, st)                                   \
-             : dma    ? launch_gemm_t<TA_, TB_, EPI_, true, 2, 4, 4, true>(a, grid, st)                 \
-             : dma128 ? launch_gemm_t<TA_, TB_, EPI_, true, 2, 2, 4, true>(a, grid, st)                 \
-             : narrow ? launch_gemm_t<TA_, TB_, EPI_, true, 2, 2, 2>(a, grid, st)                       \
-                      : launch_gemm_t<TA_, TB_, EPI_, true>(a, grid, st);                                \
-    else
-#define ASCA_GEMM_SMALL(TA_, TB_)                                                                       \
-    if (ta == TA_ && tb == TB_)                                                                         \
-        rc = launch_gemm_t<TA_, TB_, EPI_STORE, true, 1, 2>(a, grid, st);                               \
+    const dim3 grid((unsigned)blocks, (unsigned)splits);
+    // operand whose K rows are gathered (mn-contiguous operands; k-contiguous ones gather rows in any variant)
+    const int gather = ta && a.a_rows ? 1 : !tb && a.b_rows ? 2 : 0;
+    if (gather && (!ta || tb || epi != EPI_STORE || (a.a_rows && a.b_rows)))
+        return fail(ASCA_ERR_UNSUPPORTED, "%s: one gathered operand, of A^T B", name);
+#define ASCA_GEMM_CASE(TA_, TB_, EPI_, G_)                                              \
+    if (ta == TA_ && tb == TB_ && epi == EPI_ && gather == G_)                          \
+        rc = tile == T_SMALL  ? launch_small_t<TA_, TB_, EPI_, G_>(a, grid, st)         \
+             : tile == T_WIDE ? launch_gemm_t<TA_, TB_, EPI_, G_, 2, 4, true>(a, grid, st) \
+                              : launch_gemm_t<TA_, TB_, EPI_, G_, 2, 2, false>(a, grid, st); \
     else
 #define ASCA_GEMM_BATCHED(TA_, TB_)                                                                     \
     if (ta == TA_ && tb == TB_)                                                                         \
         rc = wm == 1 ? launch_batched_t<TA_, TB_, 1, 2>(a, blocks, st)                                  \
                      : launch_batched_t<TA_, TB_, 2, 2>(a, blocks, st);                                 \
     else
-    if (a.gmode == 3 && vec && a.K > 0) {
+    if (batched) {
         ASCA_GEMM_BATCHED(0, 0)
         ASCA_GEMM_BATCHED(1, 0)
         ASCA_GEMM_BATCHED(0, 1)
@@ -1032,22 +1262,14 @@ int gemm_launch(int ta, int tb, int epi, GemmArgs a, long m_total, hipStream_t s
         return post_launch(name);
     }
 #undef ASCA_GEMM_BATCHED
-    if (wm == 1) {
-        ASCA_GEMM_SMALL(0, 0)
-        ASCA_GEMM_SMALL(1, 0)
-        ASCA_GEMM_SMALL(0, 1)
-        ASCA_GEMM_SMALL(1, 1)
-        rc = fail(ASCA_ERR_UNSUPPORTED, "%s: no kernel for this variant", name);
-        if (rc) return rc;
-        return post_launch(name);
-    }
-#undef ASCA_GEMM_SMALL
-    ASCA_GEMM_CASE(0, 0, EPI_STORE)
-    ASCA_GEMM_CASE(1, 0, EPI_STORE)
-    ASCA_GEMM_CASE(0, 1, EPI_STORE)
-    ASCA_GEMM_CASE(1, 1, EPI_STORE)
-    ASCA_GEMM_CASE(0, 0, EPI_SILU)
-    ASCA_GEMM_CASE(0, 1, EPI_SILU_BWD)
+    ASCA_GEMM_CASE(0, 0, EPI_STORE, 0)
+    ASCA_GEMM_CASE(1, 0, EPI_STORE, 0)
+    ASCA_GEMM_CASE(1, 0, EPI_STORE, 1)
+    ASCA_GEMM_CASE(1, 0, EPI_STORE, 2)
+    ASCA_GEMM_CASE(0, 1, EPI_STORE, 0)
+    ASCA_GEMM_CASE(1, 1, EPI_STORE, 0)
+    ASCA_GEMM_CASE(0, 0, EPI_SILU, 0)
+    ASCA_GEMM_CASE(0, 1, EPI_SILU_BWD, 0)
     rc = fail(ASCA_ERR_UNSUPPORTED, "%s: no kernel for this variant", name);
 #undef ASCA_GEMM_CASE
     if (rc) return rc;
@@ -1337,7 +1559,15 @@ int gemm_run(int trans_a, int trans_b, int M, int N, int K, float alpha, const f
     a.beta = beta;
     a.bias = bias;
     long kps = 0;
-    const int splits = K > 0 ? gemm_splits(M, N, K, &kps) : 1;
+    int splits = K > 0 ? gemm_splits(M, N, K, &kps) : 1;
+    if (splits > 1) {
+        // one pass over K where that is no slower than the partials and their sum
+        double one, cut;
+        const bool fits = small_fits(max(lda, 1L), 64) && small_fits(max(ldb, 1L), 64);
+        best_tile(M, N, 0, 1, (K + SP_BK - 1) / SP_BK, fits, &one);
+        best_tile(M, N, 0, splits, (kps + SP_BK - 1) / SP_BK, fits, &cut);
+        if (one <= cut + 5.0 + 1e-6 * splits * M * N) splits = 1;
+    }
     if (splits == 1) return gemm_launch(trans_a, trans_b, EPI_STORE, a, M, st, "gemm");
     const long MN = (long)M * N;
     int rc = ws_check(ws, (size_t)splits * MN, "gemm split-K");

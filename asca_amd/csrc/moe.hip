@@ -99,7 +99,7 @@ int asca::moe_bwd_weights(const float* xn, const float* hidden, const int32_t* p
     g2.goff = offsets;
     g2.ngroups = E;
     g2.gmode = 2;
-    int rc = gemm_launch(1, 0, EPI_STORE, g2, 0, st, "moe_bwd_dw2");
+    int rc = gemm_launch(1, 0, EPI_STORE, g2, T, st, "moe_bwd_dw2");
     if (rc) return rc;
     // db2 (+)= colsum(dout)
     if ((rc = colsum_launch(dout, T, d, d, nullptr, 0, db2, accumulate, ws, st))) return rc;
@@ -121,7 +121,7 @@ int asca::moe_bwd_weights(const float* xn, const float* hidden, const int32_t* p
     g1.goff = offsets;
     g1.ngroups = E;
     g1.gmode = 2;
-    return gemm_launch(1, 0, EPI_STORE, g1, 0, st, "moe_bwd_dw1");
+    return gemm_launch(1, 0, EPI_STORE, g1, T, st, "moe_bwd_dw1");
 }
 
 extern "C" {

@@ -49,6 +49,54 @@ def _ref_gemm(a, b, ta, tb, alpha, beta, c, bias):
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(64, 64, 31), (65, 67, 33), (1, 3, 257), (257, 129, 64), (384, 1030, 1027),
+                                   (4096, 512, 96), (4097, 511, 65), (2048, 2052, 128)])
+def test_gemm_split_products(g, ta, tb, M, N, K):
+    """The three-way bf16 split on every tile and at its edges: values over 24
+    binades against float64.  A result is at most 6 roundings (each below one
+    unit in the last place, 2^-23) per 32 terms and 16 more for partial sums
+    away from it, of at most sum |a||b|.  A sum of many results is as exact as
+    one (no rounding bias): 2^-23 of the rms times sqrt(rows) rows."""
+    rng = np.random.default_rng(M + N + K + ta + 2 * tb)
+    a = (rng.standard_normal((K, M) if ta else (M, K)) * 2.0 ** rng.integers(-12, 12, (K, M) if ta else (M, K)))
+    b = rng.standard_normal((N, K) if tb else (K, N))
+    a, b = a.astype(np.float32), b.astype(np.float32)
+    got = g.gemm(a, b, trans_a=bool(ta), trans_b=bool(tb)).astype(np.float64)
+    A, Bm = (a.T if ta else a).astype(np.float64), (b.T if tb else b).astype(np.float64)
+    ref = A @ Bm
+    bound = (6 * ((K + 31) // 32) + 16) * 2.0**-23 * (np.abs(A) @ np.abs(Bm))
+    assert np.all(np.abs(got - ref) <= bound), np.max(np.abs(got - ref) / bound)
+    rms = np.sqrt(np.mean(ref * ref))
+    if M * N >= 4096:
+        assert abs(np.mean(got - ref)) <= 2.0**-23 * rms * 8 / np.sqrt(min(M, N))
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 64, 40), (200, 300, 64), (4096, 512, 64)])
+def test_gemm_non_finite(g, M, N, K):
+    """Infinities, NaN and values beyond bf16's largest come out as f32 products
+    give them, and rows and columns without them are untouched."""
+    rng = np.random.default_rng(M + N)
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    b = rng.standard_normal((K, N)).astype(np.float32)
+    a[1, 3], a[5, 0], a[M - 1, K - 1] = np.inf, np.nan, -np.inf
+    a[7] = 0.0
+    a[7, 2] = np.float32(3.4e38)  # rounds to infinity in bf16
+    b[2, :] *= np.float32(0.01)
+    b[4, N - 2] = np.inf
+    b[3, 5] = 0.0  # inf * 0
+    with np.errstate(all="ignore"):
+        ref = a.astype(np.float64) @ b.astype(np.float64)
+    got = g.gemm(a, b).astype(np.float64)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+    inf = np.isinf(ref)
+    np.testing.assert_array_equal(got[inf], ref[inf])
+    ok = np.isfinite(ref)
+    with np.errstate(all="ignore"):
+        mag = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    assert np.all(np.abs(got[ok] - ref[ok]) <= (6 * ((K + 31) // 32) + 16) * 2.0**-23 * mag[ok])
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
 @pytest.mark.parametrize("M,N,K", [(128, 128, 32), (1, 1, 1), (300, 257, 77), (64, 1536, 512),
                                    (513, 16, 512), (130, 200, 4096), (7, 9, 0),
                                    (300, 260, 84), (129, 516, 36)])  # partial tiles and k-tails, N % 4 == 0
