@@ -28,6 +28,7 @@
 // multiple of C with identity steps: q = k = v = 0, alpha = 1, beta = 0) and the
 // per-chunk intermediates, so every batched product has one stride per chunk.
 #include "common.h"
+#include "delta.h"
 #include "gemm.h"
 #include "runtime.h"
 
@@ -1921,6 +1922,15 @@ static int chunk_fwd_tail(const ChunkDims& d, const ChunkWs& w, const uint16_t* 
 
 using namespace asca;
 
+// Shapes whose bf16 entry points run the blocked form's kernels (delta.h), which
+// advance 16 steps at a time whatever the chunk size: every width they have but
+// C = 64, dh = 128, which has kernels of its own here.  The decomposed form they
+// replace was bound by its launches and intermediates: B4 T1000 H8 dh64 C64
+// 1350 -> 301 us, T4096 B8 H8 dh64 C32 11.8 -> 1.24 ms.
+static bool chunk_blocked(int B, int T, int H, int dh, int C) {
+    return ut_width(dh) && !(C == FP_C && dh == FP_D) && (long)B * T * H > 0 && ut_fits(T, H, dh, (long)H * dh);
+}
+
 static int chunk_fwd_decomposed(const ChunkDims& d, const ChunkWs& w, const float* alpha, const float* beta,
                                 float* o, hipStream_t st);
 static int chunk_bwd_decomposed(const ChunkDims& d, const ChunkWs& w, float* dq, float* dk, float* dv,
@@ -1933,6 +1943,10 @@ int asca_chunk_ws_bytes(int B, int T, int H, int dh, int C, size_t* bytes) {
     int rc = chunk_check(B, T, H, dh, C);
     if (rc) return rc;
     *bytes = chunk_ws(chunk_dims(B, T, H, dh, C), nullptr).total * sizeof(float);
+    if (chunk_blocked(B, T, H, dh, C)) {
+        const size_t need = ut_ws_layout(B, T, H, dh, nullptr).bytes;
+        if (need > *bytes) *bytes = need;
+    }
     return ASCA_OK;
 }
 
@@ -1942,6 +1956,8 @@ int asca_chunk_fwd(const uint16_t* q, const uint16_t* k, const uint16_t* v, cons
     if (rc) return rc;
     if ((long)B * T * H == 0) return ASCA_OK;
     if (!q || !k || !v || !alpha || !beta || !o || !ws) return fail(ASCA_ERR_INVALID, "asca_chunk_fwd: null pointer");
+    if (chunk_blocked(B, T, H, dh, C))
+        return launch_ut_fwd(q, k, v, true, alpha, beta, o, ut_ws_layout(B, T, H, dh, ws), B, T, H, dh, as_stream(stream));
     const ChunkDims d = chunk_dims(B, T, H, dh, C);
     const ChunkWs w = chunk_ws(d, reinterpret_cast<float*>(ws));
     const hipStream_t st = as_stream(stream);
@@ -2008,6 +2024,10 @@ int asca_chunk_bwd(const uint16_t* q, const uint16_t* k, const uint16_t* v, cons
     if ((long)B * T * H == 0) return ASCA_OK;
     if (!q || !k || !v || !d_o || !ws || !dq || !dk || !dv || !dalpha || !dbeta)
         return fail(ASCA_ERR_INVALID, "asca_chunk_bwd: null pointer");
+    if (chunk_blocked(B, T, H, dh, C))
+        // raw gradients: the gates come from the forward's records
+        return launch_ut_bwd(false, q, k, v, true, nullptr, nullptr, d_o, ut_ws_layout(B, T, H, dh, ws), nullptr,
+                             nullptr, dq, dk, dv, (long)H * dh, dalpha, dbeta, H, B, T, H, dh, as_stream(stream));
     const ChunkDims d = chunk_dims(B, T, H, dh, C);
     const ChunkWs w = chunk_ws(d, reinterpret_cast<float*>(ws));
     const hipStream_t st = as_stream(stream);

@@ -1,6 +1,7 @@
 // Internals shared by the delta-rule translation units (delta.hip: the
-// recurrent kernels for every dh other than 64, on eight-lane column groups, and
-// the entry points; delta_ut64.hip: dh = 64 in the blocked form).
+// recurrent kernels on eight-lane column groups for the head widths that the
+// blocked form does not take, and the entry points; delta_ut64.hip,
+// delta_ut64_b.hip, delta_utn.hip: the blocked form).
 #pragma once
 #include "common.h"
 
@@ -20,7 +21,7 @@ namespace asca {
 struct DeltaWs {
     float* sk;
     float* ckpt;
-    float* rec;     // dh = 64 blocked form: per unit and 16-step block, K K^T, Q K^T, T, M, Gamma, gate vectors
+    float* rec;     // blocked form (else null): per unit and 16-step block, K K^T, Q K^T, T, M, Gamma, gate vectors
     int ck;
     int nslots;
     int cs;
@@ -67,21 +68,34 @@ ASCA_DEV void cross_step_sum(const float (&y)[CK], float* __restrict__ red_ab, i
     }
 }
 
-// dh = 64: the blocked (UT) form on the matrix cores (delta_ut64.hip), used for
-// every dh = 64 shape with one block per unit (ws.cs == 1).  Its workspace: the
-// u rows in `sk` (per unit and D64_BLK-step block, as the forward's wave tiles,
-// T rounded up to whole blocks), the state before every other block (every
-// D64_CK steps) and the final state in `ckpt`, per block a record of D64_REC
-// floats in `rec`, all written by the forward and read by the backward.  Any
-// pointer alignment.
+// The blocked (UT) form on the matrix cores (delta_ut64.hip), used for every
+// shape of the head widths 16, 32, 48, 64, 96 and 128.  Its workspace: the u
+// rows in `sk` (per unit and D64_BLK-step block, as the forward's wave tiles, T
+// rounded up to whole blocks), the state before every other block (every D64_CK
+// steps) and the final state in `ckpt`, per block a record of D64_REC floats in
+// `rec`, all written by the forward and read by the backward.  Any pointer
+// alignment.  Rows f32, or (bf) bf16 with raw gradients.
 constexpr int D64_BLK = 16;
 constexpr int D64_CK = 2 * D64_BLK;
 constexpr int D64_REC = 1344;
-int launch_ut_fwd64(const float* q, const float* k, const float* v, const float* alpha, const float* beta, float* o,
-                    const DeltaWs& ws, int B, int T, int H, hipStream_t st);
-int launch_ut_bwd64(bool fused, const float* q, const float* k, const float* v, const float* alpha,
-                    const float* beta, const float* d_o, const DeltaWs& ws, const float* qn, const float* kn,
-                    float* gq, float* gk, float* gv, long ldx, float* ga, float* gb, long ldg, int B, int T, int H,
-                    hipStream_t st);
+inline bool ut_width(int dh) { return dh == 16 || dh == 32 || dh == 48 || dh == 64 || dh == 96 || dh == 128; }
+// blocks a unit's value columns run on
+inline int ut_col_splits(int dh) { return dh > 64 ? dh / 32 : 1; }
+// every 32-bit offset of the kernels fits, with output rows of stride ld
+bool ut_fits(int T, int H, int dh, long ld);
+// the blocked form's workspace at `base` (`bytes` long)
+DeltaWs ut_ws_layout(int B, int T, int H, int dh, void* base);
+int launch_ut_fwd(const void* q, const void* k, const void* v, bool bf, const float* alpha, const float* beta,
+                  float* o, const DeltaWs& ws, int B, int T, int H, int dh, hipStream_t st);
+int launch_ut_bwd(bool fused, const void* q, const void* k, const void* v, bool bf, const float* alpha,
+                  const float* beta, const void* d_o, const DeltaWs& ws, const float* qn, const float* kn, float* gq,
+                  float* gk, float* gv, long ldx, float* ga, float* gb, long ldg, int B, int T, int H, int dh,
+                  hipStream_t st);
+// Adds the cs column splits' partial dq, dk (part_x: [2][cs][rows][H dh]) and
+// dalpha, dbeta (part_g: [cs][rows][2H]) and, fused, applies the L2-norm and
+// sigmoid backward (delta.hip).
+int launch_delta_combine(bool fused, int cs, const float* part_x, const float* part_g, const float* q, const float* k,
+                         const float* alpha, const float* beta, const float* qn, const float* kn, float* gq, float* gk,
+                         long ldx, float* ga, float* gb, long ldg, long rows, int H, int dh, hipStream_t st);
 
 }  // namespace asca

@@ -6,6 +6,8 @@
 //   S_t  = alpha_t S_{t-1} + k_t u_t^T,  o_t = S_t^T q_t.
 //
 // Design (MI355X-first, not a translation of rust/kernels/asca.cu):
+// These kernels take the head widths that the blocked form on the matrix cores
+// (ut64_kernels.h: 16, 32, 48, 64, 96 and 128) does not.
 //  * Column i of S only ever meets k, q, alpha, beta and its own v_i, sk_i, u_i,
 //    so the forward splits each (sequence, head) unit into dh/8 waves of 8 value
 //    columns that never talk to each other (two waves per SIMD at dh = 64).
@@ -54,21 +56,16 @@ ASCA_DEV float4* trash_f4(int i) { return g_trash4 + (i & 1023); }
 ASCA_DEV float readlane_f(float x, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l)); }
 
 // Masked vector helpers: invalid elements read 0 from a valid address.
-template <bool EXACT>
 ASCA_DEV float4 ld4m(const float* __restrict__ p, int col, int dh) {
-    if constexpr (EXACT) {
-        return *reinterpret_cast<const float4*>(p + col);
-    } else {
-        float4 r;
-        float* rr = reinterpret_cast<float*>(&r);
+    float4 r;
+    float* rr = reinterpret_cast<float*>(&r);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const bool ok = col + e < dh;
-            const float x = p[ok ? col + e : 0];
-            rr[e] = ok ? x : 0.0f;
-        }
-        return r;
+    for (int e = 0; e < 4; ++e) {
+        const bool ok = col + e < dh;
+        const float x = p[ok ? col + e : 0];
+        rr[e] = ok ? x : 0.0f;
     }
+    return r;
 }
 
 // ------------------------------------------------------------------ forward
@@ -104,7 +101,7 @@ struct FwdStage {
 
 // Global -> registers for chunk c (steps c*CK .. c*CK+CK-1, clamped to T-1);
 // wg: the wave's index among all waves of the unit (its value columns).
-template <int DH, int CS, bool EXACT>
+template <int DH, int CS>
 ASCA_DEV void fwd_stage_load(FwdStage<DH, CS>& st, int c, const float* __restrict__ q, const float* __restrict__ k,
                              const float* __restrict__ v, long ubase, long d, int T, int dh, int wg, int lane) {
     using L = FS<DH, CS>;
@@ -118,7 +115,7 @@ ASCA_DEV void fwd_stage_load(FwdStage<DH, CS>& st, int c, const float* __restric
         const int fl = f - tsr * (L::KQ_F / 4);
         const int j = fl / (DH / 4), c4 = fl % (DH / 4);
         const long t = min(t0 + j, T - 1);
-        st.kq[i] = ld4m<EXACT>((tsr ? q : k) + ubase + t * d, 4 * c4, dh);
+        st.kq[i] = ld4m((tsr ? q : k) + ubase + t * d, 4 * c4, dh);
     }
 #pragma unroll
     for (int i = 0; i < L::NV; ++i) {
@@ -126,7 +123,7 @@ ASCA_DEV void fwd_stage_load(FwdStage<DH, CS>& st, int c, const float* __restric
         const int f = f0 < CK * 2 ? f0 : 0;
         const int j = f / 2, half = f % 2;
         const long t = min(t0 + j, T - 1);
-        st.v[i] = ld4m<EXACT>(v + ubase + t * d, wg * 8 + half * 4, dh);
+        st.v[i] = ld4m(v + ubase + t * d, wg * 8 + half * 4, dh);
     }
 }
 
@@ -235,17 +232,11 @@ ASCA_DEV void fwd_steps(float (&s)[DH / 8], const float* __restrict__ buf, float
 
 // A lane's rows row0 .. row0+R-1 of column col into a checkpoint slot (S^T,
 // contiguous per column); masked elements go to the trash.
-template <int R, bool EXACT>
+template <int R>
 ASCA_DEV void store_ckpt(float* __restrict__ dst, const float (&s)[R], bool col_ok, int row0, int dh,
                          float* __restrict__ tr) {
-    if constexpr (EXACT && R % 4 == 0) {
 #pragma unroll
-        for (int j = 0; j < R; j += 4)
-            *reinterpret_cast<float4*>(dst + j) = make_float4(s[j], s[j + 1], s[j + 2], s[j + 3]);
-    } else {
-#pragma unroll
-        for (int j = 0; j < R; ++j) *((col_ok && row0 + j < dh) ? dst + j : tr + j) = s[j];
-    }
+    for (int j = 0; j < R; ++j) *((col_ok && row0 + j < dh) ? dst + j : tr + j) = s[j];
 }
 
 // One block per (sequence, head) unit, unit = h*B + b (the reference's s_pre
@@ -253,7 +244,7 @@ ASCA_DEV void store_ckpt(float* __restrict__ dst, const float (&s)[R], bool col_
 // unit, slot j = S^T before step j*CK (element (a, i) of S at [i*dh + a]), the
 // last slot S^T after step T-1.  Steps past T (the tail of the last chunk) run
 // with alpha = 1, beta = 0, which leaves the state unchanged.
-template <int DH, int CS, bool EXACT>
+template <int DH, int CS>
 __global__ __launch_bounds__((FS<DH, CS>::NT)) void delta_fwd_k(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     const float* __restrict__ alpha, const float* __restrict__ beta, float* __restrict__ o,
@@ -278,7 +269,7 @@ __global__ __launch_bounds__((FS<DH, CS>::NT)) void delta_fwd_k(
     float* skb = sk_out + ubase;
     const long gbase = (long)b * T * H + h;
     float* ckb = ckpt + (long)unit * nslots * dh2;
-    const bool col_ok = EXACT || col < dh;
+    const bool col_ok = col < dh;
     float* const tr = trash_f(threadIdx.x * 2);
     const int nchunk = (T + CK - 1) / CK;
 
@@ -292,7 +283,7 @@ __global__ __launch_bounds__((FS<DH, CS>::NT)) void delta_fwd_k(
     for (int j = 0; j < R; ++j) s[j] = 0.0f;
 
     FwdStage<DH, CS> stg;
-    fwd_stage_load<DH, CS, EXACT>(stg, 0, q, k, v, ubase, d, T, dh, wg, lane);
+    fwd_stage_load<DH, CS>(stg, 0, q, k, v, ubase, d, T, dh, wg, lane);
     // a gate of step t (lane-dependent: alpha or beta); past T, alpha = 1 and beta = 0
     const float gpad = gl < CK ? 1.0f : 0.0f;
     auto gate = [&](int t) {
@@ -308,8 +299,8 @@ __global__ __launch_bounds__((FS<DH, CS>::NT)) void delta_fwd_k(
         const float* buf = lds + (ci & 1) * L::BUF_F;
         const float gcur = gnext;
         gnext = gate(t0 + CK + gstep);
-        fwd_stage_load<DH, CS, EXACT>(stg, min(ci + 1, nchunk - 1), q, k, v, ubase, d, T, dh, wg, lane);
-        store_ckpt<R, EXACT>(ckb + (long)ci * dh2 + (long)col * dh + row0, s, col_ok, row0, dh, tr);
+        fwd_stage_load<DH, CS>(stg, min(ci + 1, nchunk - 1), q, k, v, ubase, d, T, dh, wg, lane);
+        store_ckpt<R>(ckb + (long)ci * dh2 + (long)col * dh + row0, s, col_ok, row0, dh, tr);
         // Lanes j < CK of gcur hold the chunk's alpha; when all of them lie in
         // [2^-8, 2^8] the chunk runs on the scaled state (fwd_steps).
         const bool bad = lane < CK && !(gcur >= 0x1p-8f && gcur <= 0x1p8f);
@@ -339,7 +330,7 @@ __global__ __launch_bounds__((FS<DH, CS>::NT)) void delta_fwd_k(
         fwd_stage_store<DH, CS>(stg, lds + ((ci + 1) & 1) * L::BUF_F, w, lane);
         lds_barrier();
     }
-    store_ckpt<R, EXACT>(ckb + (long)nchunk * dh2 + (long)col * dh + row0, s, col_ok, row0, dh, tr);
+    store_ckpt<R>(ckb + (long)nchunk * dh2 + (long)col * dh + row0, s, col_ok, row0, dh, tr);
 }
 
 // Full state history for download_states: S before every step then the final
@@ -441,7 +432,7 @@ struct BStage {
 };
 
 // wg: the wave's index among all waves of the unit (its value columns)
-template <int DH, int CS, bool EXACT, bool FUSED>
+template <int DH, int CS, bool FUSED>
 ASCA_DEV void bstage_load(BStage<DH, CS>& st, int g, const float* __restrict__ q, const float* __restrict__ k,
                           const float* __restrict__ v, const float* __restrict__ d_o,
                           const float* __restrict__ skv, const float* __restrict__ alpha,
@@ -459,7 +450,7 @@ ASCA_DEV void bstage_load(BStage<DH, CS>& st, int g, const float* __restrict__ q
         const int fl = f - tsr * S::QK4;
         const int j = fl / (DH / 4), c4 = fl % (DH / 4);
         const long t = min(t0 + j, T - 1);
-        st.rq[i] = ld4m<EXACT>((tsr ? k : q) + ubase + t * d, 4 * c4, dh);
+        st.rq[i] = ld4m((tsr ? k : q) + ubase + t * d, 4 * c4, dh);
     }
 #pragma unroll
     for (int i = 0; i < S::NW; ++i) {
@@ -470,7 +461,7 @@ ASCA_DEV void bstage_load(BStage<DH, CS>& st, int g, const float* __restrict__ q
         const int j = rem / 2, half = rem % 2;
         const long t = min(t0 + j, T - 1);
         const float* src = tsr == 0 ? d_o : (tsr == 1 ? v : skv);
-        st.rw[i] = ld4m<EXACT>(src + ubase + t * d, wg * 8 + half * 4, dh);
+        st.rw[i] = ld4m(src + ubase + t * d, wg * 8 + half * 4, dh);
     }
     {
         const int gl = lane & (2 * CK - 1);
@@ -482,19 +473,11 @@ ASCA_DEV void bstage_load(BStage<DH, CS>& st, int g, const float* __restrict__ q
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
         const int i = colb + n;
-        if constexpr (EXACT && M % 4 == 0) {
 #pragma unroll
-            for (int m = 0; m < M; m += 4) {
-                const float4 x = *reinterpret_cast<const float4*>(cks + (long)i * dh + rowb + m);
-                st.rck[n][m] = x.x; st.rck[n][m + 1] = x.y; st.rck[n][m + 2] = x.z; st.rck[n][m + 3] = x.w;
-            }
-        } else {
-#pragma unroll
-            for (int m = 0; m < M; ++m) {
-                const bool ok = i < dh && rowb + m < dh;
-                const float x = cks[ok ? (long)i * dh + rowb + m : 0];
-                st.rck[n][m] = ok ? x : 0.0f;
-            }
+        for (int m = 0; m < M; ++m) {
+            const bool ok = i < dh && rowb + m < dh;
+            const float x = cks[ok ? (long)i * dh + rowb + m : 0];
+            st.rck[n][m] = ok ? x : 0.0f;
         }
     }
 }
@@ -606,7 +589,7 @@ ASCA_DEV void bops_read(BOps<DH / 16>& o, const float* __restrict__ st_q, const 
 //     du~ = ds^T k = G_{j+1} du (one FMA per element), and every output term
 //     takes its scale from the step's gate-table row (g1 = G_{j+1}, r1 = 1/G_{j+1},
 //     ia = 1/alpha = G_j / G_{j+1}).
-template <int DH, bool EXACT, bool SC>
+template <int DH, bool SC>
 ASCA_DEV void bwd_step(const BOps<DH / 16>& in, const float (&sm)[DH / 16][2], const float (&sa)[DH / 16][2],
                        float (&ds)[DH / 16][2], float* __restrict__ rq, float* __restrict__ rk, float& pab_out,
                        float* __restrict__ rv, int rg, int cg,
@@ -717,7 +700,7 @@ ASCA_DEV void bwd_step(const BOps<DH / 16>& in, const float (&sm)[DH / 16][2], c
 // LDS buffer nbuf halfway, and reduce the per-step dalpha / dbeta partials.  With SC
 // the stash holds S / G_j and ds is carried as G_{j+1} dS inside the segment
 // (see bwd_step); ds enters and leaves unscaled.
-template <int DH, int CS, bool EXACT, bool SC>
+template <int DH, int CS, bool SC>
 ASCA_DEV void bwd_segment(const float (&s0)[DH / 16][2], float (&ds)[DH / 16][2], const BStage<DH, CS>& stg,
                           float* __restrict__ nbuf, float2* __restrict__ cks, const float* __restrict__ st_q,
                           const float* __restrict__ st_k, const float* __restrict__ st_w,
@@ -777,7 +760,7 @@ ASCA_DEV void bwd_segment(const float (&s0)[DH / 16][2], float (&ds)[DH / 16][2]
 #pragma unroll
     for (int jj = CK - 1; jj >= 0; --jj) {
         if (jj > 0) bops_read<DH>(op[(jj - 1) & 1], st_q, st_k, st_w, st_ab, jj - 1, w, rowb, cg);
-        bwd_step<DH, EXACT, SC>(op[jj & 1], stash[jj], stash[jj + 1], ds, red_q + (jj * W + w) * DH,
+        bwd_step<DH, SC>(op[jj & 1], stash[jj], stash[jj + 1], ds, red_q + (jj * W + w) * DH,
                                 red_k + (jj * W + w) * DH, pab[jj], red_v + jj * DH, rg, cg, rowb, colb, dh);
         if (jj == CK / 2) {
             // the staged operands of the next segment (loads issued at the
@@ -801,7 +784,7 @@ ASCA_DEV void bwd_segment(const float (&s0)[DH / 16][2], float (&ds)[DH / 16][2]
 // With CS = 2 the row sums dq, dk and dalpha, dbeta cover only the block's
 // columns: they go to the partial buffers (part_x [CS][B*T][H*dh], part_g
 // [CS][B*T][2H]) and delta_combine_k finishes them; dv is complete per column.
-template <int DH, int CS, bool EXACT, bool FUSED>
+template <int DH, int CS, bool FUSED>
 __global__ __launch_bounds__((BS<DH, CS>::NT)) void delta_bwd_k(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     const float* __restrict__ alpha, const float* __restrict__ beta, const float* __restrict__ d_o,
@@ -835,7 +818,7 @@ __global__ __launch_bounds__((BS<DH, CS>::NT)) void delta_bwd_k(
     for (int m = 0; m < M; ++m) ds[m][0] = ds[m][1] = 0.0f;
 
     BStage<DH, CS> stg;
-    bstage_load<DH, CS, EXACT, FUSED>(stg, nseg - 1, q, k, v, d_o, skv, alpha, beta, qnorm, knorm, ckb, ubase,
+    bstage_load<DH, CS, FUSED>(stg, nseg - 1, q, k, v, d_o, skv, alpha, beta, qnorm, knorm, ckb, ubase,
                                       gbase, d, dh2, T, H, dh, wg, lane, rowb, colb);
     {
         float* const b0 = lds + ((nseg - 1) & 1) * S::BUF_F + S::ST_OFF;
@@ -862,15 +845,15 @@ __global__ __launch_bounds__((BS<DH, CS>::NT)) void delta_bwd_k(
             s0[m][0] = x.x;
             s0[m][1] = x.y;
         }
-        bstage_load<DH, CS, EXACT, FUSED>(stg, g > 0 ? g - 1 : 0, q, k, v, d_o, skv, alpha, beta, qnorm, knorm, ckb,
+        bstage_load<DH, CS, FUSED>(stg, g > 0 ? g - 1 : 0, q, k, v, d_o, skv, alpha, beta, qnorm, knorm, ckb,
                                           ubase, gbase, d, dh2, T, H, dh, wg, lane, rowb, colb);
         lds_barrier();  // staging of this segment visible to all waves
 
         if (__builtin_amdgcn_readfirstlane(__float_as_int(st_ab[8 * CK])) == __float_as_int(1.0f))
-            bwd_segment<DH, CS, EXACT, true>(s0, ds, stg, nbuf, cks, st_q, st_k, st_w, st_ab, red_q, red_k,
+            bwd_segment<DH, CS, true>(s0, ds, stg, nbuf, cks, st_q, st_k, st_w, st_ab, red_q, red_k,
                                              red_ab, red_v, t0, T, w, lane, rg, cg, rowb, colb, dh);
         else
-            bwd_segment<DH, CS, EXACT, false>(s0, ds, stg, nbuf, cks, st_q, st_k, st_w, st_ab, red_q, red_k,
+            bwd_segment<DH, CS, false>(s0, ds, stg, nbuf, cks, st_q, st_k, st_w, st_ab, red_q, red_k,
                                               red_ab, red_v, t0, T, w, lane, rg, cg, rowb, colb, dh);
         lds_barrier();  // red_* of this segment complete
 
@@ -974,10 +957,10 @@ __global__ __launch_bounds__((BS<DH, CS>::NT)) void delta_bwd_k(
     }
 }
 
-// Finish a column-split backward: sum the CS = 2 partial row sums of dq, dk
-// and dalpha, dbeta and apply the fused norm / sigmoid backward as
-// delta_bwd_k does for CS = 1.  One wave per (row, head).
-template <bool FUSED>
+// Finish a column-split backward: sum the CS partial row sums of dq, dk and
+// dalpha, dbeta and apply the fused norm / sigmoid backward as delta_bwd_k does
+// for CS = 1.  One wave per (row, head).
+template <bool FUSED, int CS>
 __global__ __launch_bounds__(256) void delta_combine_k(
     const float* __restrict__ part_x, const float* __restrict__ part_g, const float* __restrict__ q,
     const float* __restrict__ k, const float* __restrict__ alpha, const float* __restrict__ beta,
@@ -994,21 +977,27 @@ __global__ __launch_bounds__(256) void delta_combine_k(
     // every load issued first (indices clamped into the head, lanes past dh
     // masked afterwards): a load under a per-lane condition is waited for on
     // its own
-    float x0[2], x1[2], x2[2], x3[2], qa[2], ka[2];
+    float xq[2][CS], xk[2][CS], qa[2], ka[2];
 #pragma unroll
     for (int ia = 0; ia < 2; ++ia) {
         const long a = o + min(lane + 64 * ia, dh - 1);
-        x0[ia] = part_x[a];
-        x1[ia] = part_x[n + a];
-        x2[ia] = part_x[2 * n + a];
-        x3[ia] = part_x[3 * n + a];
+#pragma unroll
+        for (int s = 0; s < CS; ++s) {
+            xq[ia][s] = part_x[s * n + a];
+            xk[ia][s] = part_x[(CS + s) * n + a];
+        }
         if constexpr (FUSED) {
             qa[ia] = q[a];
             ka[ia] = k[a];
         }
     }
     const long og = r * 2 * H + h, ng = rows * 2 * H;
-    const float g0 = part_g[og], g1 = part_g[ng + og], g2 = part_g[og + H], g3 = part_g[ng + og + H];
+    float gA[CS], gB[CS];
+#pragma unroll
+    for (int s = 0; s < CS; ++s) {
+        gA[s] = part_g[s * ng + og];
+        gB[s] = part_g[s * ng + og + H];
+    }
     float qn = 1.0f, kn = 1.0f, al = 0.0f, be = 0.0f;
     if constexpr (FUSED) {
         qn = qnorm[r * H + h];
@@ -1021,8 +1010,14 @@ __global__ __launch_bounds__(256) void delta_combine_k(
 #pragma unroll
     for (int ia = 0; ia < 2; ++ia) {
         const bool ok = lane + 64 * ia < dh;
-        dq[ia] = ok ? x0[ia] + x1[ia] : 0.0f;
-        dk[ia] = ok ? x2[ia] + x3[ia] : 0.0f;
+        float sq = xq[ia][0], sk = xk[ia][0];
+#pragma unroll
+        for (int s = 1; s < CS; ++s) {
+            sq += xq[ia][s];
+            sk += xk[ia][s];
+        }
+        dq[ia] = ok ? sq : 0.0f;
+        dk[ia] = ok ? sk : 0.0f;
         if constexpr (FUSED) {
             qa[ia] = ok ? qa[ia] : 0.0f;
             ka[ia] = ok ? ka[ia] : 0.0f;
@@ -1030,8 +1025,12 @@ __global__ __launch_bounds__(256) void delta_combine_k(
             dotk = fmaf(ka[ia], dk[ia], dotk);
         }
     }
-    const float dA = g0 + g1;
-    const float dB = g2 + g3;
+    float dA = gA[0], dB = gB[0];
+#pragma unroll
+    for (int s = 1; s < CS; ++s) {
+        dA += gA[s];
+        dB += gB[s];
+    }
     if constexpr (FUSED) {
         dotq = wave_sum(dotq);
         dotk = wave_sum(dotk);
@@ -1091,37 +1090,44 @@ static int ck_for(int dhc) {
 // blocks of 8 waves hold their ~215 without spilling.  A function of the shape
 // only, so the workspace size never depends on the device state.
 constexpr long SPLIT_UNITS = 128;
-// dh = 64 always runs a block per unit on the blocked kernels of delta_ut64.hip:
-// the unit's state lives in the accumulator tiles of one block's four chain
-// waves.  Even the per-step dh = 64 kernels they replaced were faster on one
-// block per unit than on two at any unit count (T = 1024, 8-128 units: forward
-// ~150 against ~157 us, backward ~345 against ~470 us).
-static int col_split(int B, int H, int dh, int dhc) {
-    if (dh == 64) return 1;
-    return (long)B * H <= SPLIT_UNITS || dhc == 128 ? 2 : 1;
-}
-
-static bool blocked64(int dh, int cs) { return dh == 64 && cs == 1; }
+static int col_split(int B, int H, int dhc) { return (long)B * H <= SPLIT_UNITS || dhc == 128 ? 2 : 1; }
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-static DeltaWs ws_layout(int B, int T, int H, int dh, void* base) {
+static DeltaWs layout(int B, int T, int H, int dh, int ck, int cs, size_t u_rows, size_t rec_floats, void* base) {
     DeltaWs w;
-    const int dhc = dh_class(dh);
-    w.cs = col_split(B, H, dh, dhc);
-    w.ck = blocked64(dh, w.cs) ? D64_CK : ck_for(dhc);
+    w.cs = cs;
+    w.ck = ck;
     w.nslots = (T + w.ck - 1) / w.ck + 1;   // the state before every chunk, then the final state
-    // the blocked form keeps the u rows per unit and 16-step block (ut64_kernels.h, U_TILE)
-    const size_t sk_rows = blocked64(dh, w.cs) ? (size_t)(T + D64_BLK - 1) / D64_BLK * D64_BLK : (size_t)T;
-    const size_t sk_bytes = align256((size_t)B * sk_rows * H * dh * sizeof(float));
+    const size_t sk_bytes = align256((size_t)B * u_rows * H * dh * sizeof(float));
     const size_t ck_bytes = align256((size_t)B * H * w.nslots * dh * dh * sizeof(float));
-    const size_t rec_bytes =
-        blocked64(dh, w.cs) ? align256((size_t)B * H * ((T + D64_BLK - 1) / D64_BLK) * D64_REC * sizeof(float)) : 0;
+    const size_t rec_bytes = align256((size_t)B * H * rec_floats * sizeof(float));
     char* c = reinterpret_cast<char*>(base);
     w.sk = reinterpret_cast<float*>(base);
     w.ckpt = base ? reinterpret_cast<float*>(c + sk_bytes) : nullptr;
     w.rec = base && rec_bytes ? reinterpret_cast<float*>(c + sk_bytes + ck_bytes) : nullptr;
     w.bytes = sk_bytes + ck_bytes + rec_bytes;
+    return w;
+}
+
+// the blocked form keeps the u rows per unit and 16-step block (ut64_kernels.h, U_TILE)
+DeltaWs ut_ws_layout(int B, int T, int H, int dh, void* base) {
+    const size_t blocks = (size_t)(T + D64_BLK - 1) / D64_BLK;
+    return layout(B, T, H, dh, D64_CK, 1, blocks * D64_BLK, blocks * D64_REC, base);
+}
+
+// Shapes on the blocked form: its widths, but for sequences whose rows pass its
+// 32-bit offsets (dh = 64 has no other kernels and refuses those).  A function
+// of the shape only: forward and backward must agree.
+static bool blocked(int T, int H, int dh) { return ut_width(dh) && (dh == 64 || ut_fits(T, H, dh, 3L * H * dh)); }
+
+static DeltaWs ws_layout(int B, int T, int H, int dh, void* base) {
+    const int dhc = dh_class(dh);
+    const DeltaWs g = layout(B, T, H, dh, ck_for(dhc), col_split(B, H, dhc), (size_t)T, 0, base);
+    if (!blocked(T, H, dh)) return g;
+    DeltaWs w = ut_ws_layout(B, T, H, dh, base);
+    // the size callers know for these widths, where the blocked form needs less
+    if (dh != 64) w.bytes = max(w.bytes, g.bytes);
     return w;
 }
 
@@ -1132,8 +1138,6 @@ static size_t part_floats(int cs, int B, int T, int H, int dh) {
     return (size_t)2 * cs * B * T * H * dh + (size_t)cs * B * T * 2 * H;
 }
 
-static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
-
 static int check_shape(int B, int T, int H, int dh) {
     if (B < 0 || T < 0 || H < 0) return fail(ASCA_ERR_INVALID, "negative shape B=%d T=%d H=%d", B, T, H);
     if (!dh_class(dh)) return fail(ASCA_ERR_UNSUPPORTED, "dh=%d outside 1..128", dh);
@@ -1141,16 +1145,16 @@ static int check_shape(int B, int T, int H, int dh) {
     return ASCA_OK;
 }
 
-template <int DH, bool EXACT>
+template <int DH>
 static int launch_fwd_t(const float* q, const float* k, const float* v, const float* alpha, const float* beta,
                         float* o, const DeltaWs& ws, int B, int T, int H, int dh, hipStream_t st) {
     int rc = pre_launch("delta_fwd");
     if (rc) return rc;
     if (DH == 128 || ws.cs > 1)
-        hipLaunchKernelGGL((delta_fwd_k<DH, 2, EXACT>), dim3(B * H * 2), dim3(FS<DH, 2>::NT), 0, st, q, k, v, alpha,
+        hipLaunchKernelGGL((delta_fwd_k<DH, 2>), dim3(B * H * 2), dim3(FS<DH, 2>::NT), 0, st, q, k, v, alpha,
                            beta, o, ws.sk, ws.ckpt, B, T, H, dh, ws.nslots);
     else if constexpr (DH < 128)  // dh = 128 always splits its columns
-        hipLaunchKernelGGL((delta_fwd_k<DH, 1, EXACT>), dim3(B * H), dim3(FS<DH, 1>::NT), 0, st, q, k, v, alpha,
+        hipLaunchKernelGGL((delta_fwd_k<DH, 1>), dim3(B * H), dim3(FS<DH, 1>::NT), 0, st, q, k, v, alpha,
                            beta, o, ws.sk, ws.ckpt, B, T, H, dh, ws.nslots);
     return post_launch("delta_fwd");
 }
@@ -1158,12 +1162,10 @@ static int launch_fwd_t(const float* q, const float* k, const float* v, const fl
 static int launch_fwd(const float* q, const float* k, const float* v, const float* alpha, const float* beta,
                       float* o, const DeltaWs& ws, int B, int T, int H, int dh, hipStream_t st) {
     const int dhc = dh_class(dh);
-    const bool exact = dh == dhc && aligned16(q) && aligned16(k);
-    if (blocked64(dh, ws.cs)) return launch_ut_fwd64(q, k, v, alpha, beta, o, ws, B, T, H, st);
+    if (blocked(T, H, dh)) return launch_ut_fwd(q, k, v, false, alpha, beta, o, ws, B, T, H, dh, st);
 #define ASCA_FWD(DHC)                                                                                    \
     if (dhc == DHC)                                                                                      \
-        return exact ? launch_fwd_t<DHC, true>(q, k, v, alpha, beta, o, ws, B, T, H, dh, st)             \
-                     : launch_fwd_t<DHC, false>(q, k, v, alpha, beta, o, ws, B, T, H, dh, st);
+        return launch_fwd_t<DHC>(q, k, v, alpha, beta, o, ws, B, T, H, dh, st);
     ASCA_FWD(16)
     ASCA_FWD(32)
     ASCA_FWD(64)
@@ -1182,13 +1184,35 @@ static int launch_states_t(const float* q, const float* k, const float* v, const
     return post_launch("delta_states");
 }
 
-template <int DH, int CS, bool EXACT, bool FUSED>
+int launch_delta_combine(bool fused, int cs, const float* part_x, const float* part_g, const float* q, const float* k,
+                         const float* alpha, const float* beta, const float* qn, const float* kn, float* gq, float* gk,
+                         long ldx, float* ga, float* gb, long ldg, long rows, int H, int dh, hipStream_t st) {
+    int rc = pre_launch("delta_combine");
+    if (rc) return rc;
+    const dim3 grid((unsigned)((rows * H + 3) / 4)), block(256);
+#define ASCA_COMBINE(F_, CS_)                                                                                   \
+    if (fused == F_ && cs == CS_)                                                                               \
+        hipLaunchKernelGGL((delta_combine_k<F_, CS_>), grid, block, 0, st, part_x, part_g, q, k, alpha, beta, qn, \
+                           kn, gq, gk, ldx, ga, gb, ldg, rows, H, dh);                                          \
+    else
+    ASCA_COMBINE(true, 2)
+    ASCA_COMBINE(true, 3)
+    ASCA_COMBINE(true, 4)
+    ASCA_COMBINE(false, 2)
+    ASCA_COMBINE(false, 3)
+    ASCA_COMBINE(false, 4)
+    return fail(ASCA_ERR_INVALID, "delta_combine: %d splits", cs);
+#undef ASCA_COMBINE
+    return post_launch("delta_combine");
+}
+
+template <int DH, int CS, bool FUSED>
 static int launch_bwd_cs(const float* q, const float* k, const float* v, const float* alpha, const float* beta,
                          const float* d_o, const DeltaWs& ws, const float* qn, const float* kn, float* gq, float* gk,
                          float* gv, long ldx, float* ga, float* gb, long ldg, int B, int T, int H, int dh,
                          hipStream_t st) {
     const size_t lds = BS<DH, CS>::LDS;
-    if (int arc = allow_lds(reinterpret_cast<const void*>(&delta_bwd_k<DH, CS, EXACT, FUSED>), lds)) return arc;
+    if (int arc = allow_lds(reinterpret_cast<const void*>(&delta_bwd_k<DH, CS, FUSED>), lds)) return arc;
     int rc = pre_launch("delta_bwd");
     if (rc) return rc;
     // the column halves' partials: scratch of this call on its stream
@@ -1196,7 +1220,7 @@ static int launch_bwd_cs(const float* q, const float* k, const float* v, const f
     if ((rc = sc.get(part_floats(CS, B, T, H, dh), st))) return rc;
     float* part_x = sc.ws.p;
     float* part_g = CS > 1 ? part_x + (size_t)2 * CS * B * T * H * dh : nullptr;
-    hipLaunchKernelGGL((delta_bwd_k<DH, CS, EXACT, FUSED>), dim3(B * H * CS), dim3(BS<DH, CS>::NT), lds, st, q, k,
+    hipLaunchKernelGGL((delta_bwd_k<DH, CS, FUSED>), dim3(B * H * CS), dim3(BS<DH, CS>::NT), lds, st, q, k,
                        v, alpha, beta, d_o, ws.sk, ws.ckpt, qn, kn, gq, gk, gv, ldx, ga, gb, ldg, part_x, part_g, B,
                        T, H, dh, ws.nslots);
     if ((rc = post_launch("delta_bwd"))) {
@@ -1204,28 +1228,22 @@ static int launch_bwd_cs(const float* q, const float* k, const float* v, const f
         return rc;
     }
     if (CS == 1) return sc.release(st);
-    if ((rc = pre_launch("delta_combine"))) {
-        (void)sc.release(st);
-        return rc;
-    }
-    const long rows = (long)B * T;
-    hipLaunchKernelGGL((delta_combine_k<FUSED>), dim3((unsigned)((rows * H + 3) / 4)), dim3(256), 0, st, part_x,
-                       part_g, q, k, alpha, beta, qn, kn, gq, gk, ldx, ga, gb, ldg, rows, H, dh);
-    rc = post_launch("delta_combine");
+    rc = launch_delta_combine(FUSED, CS, part_x, part_g, q, k, alpha, beta, qn, kn, gq, gk, ldx, ga, gb, ldg,
+                              (long)B * T, H, dh, st);
     const int rr = sc.release(st);
     return rc ? rc : rr;
 }
 
-template <int DH, bool EXACT, bool FUSED>
+template <int DH, bool FUSED>
 static int launch_bwd_t(const float* q, const float* k, const float* v, const float* alpha, const float* beta,
                         const float* d_o, const DeltaWs& ws, const float* qn, const float* kn, float* gq, float* gk,
                         float* gv, long ldx, float* ga, float* gb, long ldg, int B, int T, int H, int dh,
                         hipStream_t st) {
     if (DH == 128 || ws.cs > 1)
-        return launch_bwd_cs<DH, 2, EXACT, FUSED>(q, k, v, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx, ga, gb, ldg,
+        return launch_bwd_cs<DH, 2, FUSED>(q, k, v, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx, ga, gb, ldg,
                                                   B, T, H, dh, st);
     if constexpr (DH == 128) return fail(ASCA_ERR_UNSUPPORTED, "dh=128 without column split");
-    else return launch_bwd_cs<DH, 1, EXACT, FUSED>(q, k, v, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx, ga, gb, ldg, B,
+    else return launch_bwd_cs<DH, 1, FUSED>(q, k, v, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx, ga, gb, ldg, B,
                                               T, H, dh, st);
 }
 
@@ -1235,16 +1253,13 @@ static int launch_bwd(const float* q, const float* k, const float* v, const floa
                       float* gv, long ldx, float* ga, float* gb, long ldg, int B, int T, int H, int dh,
                       hipStream_t st) {
     const int dhc = dh_class(dh);
-    const bool exact = dh == dhc && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(d_o) &&
-                       aligned16(gv) && ((ldx * 4) % 16 == 0);
-    if (blocked64(dh, ws.cs))
-        return launch_ut_bwd64(FUSED, q, k, v, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx, ga, gb, ldg, B, T, H, st);
+    if (blocked(T, H, dh))
+        return launch_ut_bwd(FUSED, q, k, v, false, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx, ga, gb, ldg, B, T, H,
+                             dh, st);
 #define ASCA_BWD(DHC)                                                                                            \
     if (dhc == DHC)                                                                                              \
-        return exact ? launch_bwd_t<DHC, true, FUSED>(q, k, v, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx, ga, \
-                                                      gb, ldg, B, T, H, dh, st)                                  \
-                     : launch_bwd_t<DHC, false, FUSED>(q, k, v, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx,   \
-                                                       ga, gb, ldg, B, T, H, dh, st);
+        return launch_bwd_t<DHC, FUSED>(q, k, v, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx, ga, gb, ldg, B,   \
+                                        T, H, dh, st);
     ASCA_BWD(16)
     ASCA_BWD(32)
     ASCA_BWD(64)

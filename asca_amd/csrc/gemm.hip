@@ -1141,7 +1141,8 @@ static int launch_small_t(const GemmArgs& a, dim3 grid, hipStream_t st) {
 //   WIDE  (128 x 256, one block per CU)  2.5 us    (4096^3: 225 TFLOP/s against 195 with 128 x 128)
 //   T128  (128 x 128)                    1.75 us alone on its CU, 2.8 us for two blocks side by side
 //   SMALL (64 x 64, k-tiles over 8 waves) 3.5 us for eight k-tiles
-// and 3-5 us of first loads, sums and stores per round of blocks.  Products
+// and 4-7 us of first loads, sums and stores per round of blocks (the first
+// round's 3 us of a small tile overlap the launch).  Products
 // that fill the chip with the large tiles take those (a 64 x 64 tile splits
 // each value for 64 products instead of 128 or 256); where those leave CUs idle
 // the small tile wins: 1000x1000x320 22 -> 9.5 us, 64x1536x512 30 -> 11 us,
@@ -1150,7 +1151,7 @@ enum Tile { T_SMALL, T_128, T_WIDE };
 static double tile_us(Tile t, long tiles, long steps) {
     const long cus = cu_count() > 0 ? cu_count() : 256;
     const double s = (double)steps;
-    if (t == T_SMALL) return (double)((tiles + cus - 1) / cus) * (3.5 * (double)((steps + 7) / 8) + 3.0);
+    if (t == T_SMALL) return (double)((tiles + cus - 1) / cus) * (3.5 * (double)((steps + 7) / 8) + 7.0) - 4.0;
     if (t == T_WIDE) return (double)((tiles + cus - 1) / cus) * (2.5 * s + 5.0);
     const long full = tiles / (2 * cus), rem = tiles % (2 * cus);
     return (double)full * (2.8 * s + 4.0) + (rem == 0 ? 0.0 : rem <= cus ? 1.75 * s + 5.0 : 2.8 * s + 4.0);

@@ -133,12 +133,15 @@ ASCA_API void asca_rng_normal(uint64_t* state, float* out, size_t n, float scale
 /* --------------------------------------------------- delta rule (recurrent) */
 
 /* Bytes of the workspace a delta forward leaves for its backward: one dh-vector
- * per token-head (B*T*H*dh floats: S_{t-1}^T k_t; at dh = 64 the u_t rows, with
- * T rounded up to a multiple of 16) and state checkpoints every C steps plus the final state
- * (B*H*(ceil(T/C)+1)*dh*dh floats; C depends on dh, 32 at dh = 64); at dh = 64
- * also a record of 1344 floats per 16-step block and unit
+ * per token-head (B*T*H*dh floats: S_{t-1}^T k_t; at dh = 16, 32, 48, 64, 96 and
+ * 128, the widths of the blocked kernels, the u_t rows, with T rounded up to a
+ * multiple of 16) and state checkpoints every C steps plus the final state
+ * (B*H*(ceil(T/C)+1)*dh*dh floats; C depends on dh, 32 at those widths); at
+ * those widths also a record of 1344 floats per 16-step block and unit
  * (B*H*ceil(T/16)*1344 floats: the block's Gram products, triangular factors and
- * gate vectors).  It replaces the full state history DeltaDev.states of
+ * gate vectors), and never less there than the other kernels' layout (C = 8, or 2
+ * from dh = 65) takes, dh = 64 apart.  It replaces the full state history
+ * DeltaDev.states of
  * rust/src/cuda/mod.rs:1274-1275,1386-1397 ((T+1)*dh*dh floats per unit).
  * dh may be 1..128.  The forward writes the workspace and the backwards only
  * read it, so several backwards may use one forward's workspace at once. */
@@ -377,7 +380,9 @@ ASCA_API int asca_moe_bwd(const float* xn, const float* w1, const float* w2, con
  * S' = gamma_C S + (diag(Gamma[C-1,:]) K)^T U, with every product on the
  * matrix cores (f32 MFMA) and the state carried across chunks by one d x d
  * product per chunk.  At C = 64, dh = 128 each direction is one fused
- * per-chunk kernel around a persistent state scan; other shapes run batched
+ * per-chunk kernel around a persistent state scan; dh = 16, 32, 48, 64, 96 and
+ * (other C) 128 run the blocked kernels of asca_delta_fwd / asca_delta_bwd_raw on
+ * the bf16 rows, whose blocks are 16 steps whatever C; other shapes run batched
  * GEMMs over chunks.  Same results as asca_delta_fwd /
  * asca_delta_bwd_raw (DeltaBlock::scan_cpu / bptt_cpu, rust/src/delta.rs:244-334,
  * 475-587) up to f32 rounding.

@@ -61,6 +61,55 @@ def test_chunked_matches_recurrent(orc, g, B, T, H, dh, C):
     _check(orc, g, 40 + T, B, T, H, dh, C, "shape")
 
 
+@pytest.mark.parametrize("B,T,H,dh,C", [
+    (1, 1, 1, 64, 64), (2, 33, 3, 64, 16), (3, 50, 2, 16, 64), (2, 47, 2, 48, 32), (1, 130, 3, 32, 1),
+    (2, 65, 2, 96, 64), (2, 49, 3, 128, 48), (2, 75, 2, 24, 32), (1, 100, 2, 40, 64),  # 24, 40: batched products
+])
+def test_chunked_widths_extreme_gates(orc, g, B, T, H, dh, C):
+    # every head width of the blocked kernels on bf16 rows, whatever the chunk
+    # size, and two widths of the batched path, with gates of 0, 1e-6 and above 1
+    _check(orc, g, 70 + T, B, T, H, dh, C, "widths", gates=_extreme_gates)
+
+
+def test_chunked_unaligned(orc, g):
+    # bf16 rows two bytes past a 4-byte boundary and outputs four bytes past a
+    # 16-byte one give the bits of the aligned call
+    import ctypes as Ct
+
+    from asca_amd import _lib
+    from asca_amd.gpu import DevBuf, _vp, to_bf16
+
+    B, T, H, dh, C = 2, 37, 3, 64, 64
+    x = orc.DeltaInputs(5, B, T, H, dh)
+    rows, d = B * T, H * dh
+    wsb = Ct.c_size_t()
+    _lib.call("asca_chunk_ws_bytes", B, T, H, dh, C, Ct.byref(wsb))
+    got = []
+    for off in (0, 1):
+        bufs = []
+
+        def place(a):
+            bufs.append(DevBuf(a.nbytes + off * a.itemsize))
+            bufs[-1].upload(np.concatenate([np.zeros(off, a.dtype), a.ravel()]))
+            return _vp(bufs[-1].ptr + off * a.itemsize)
+
+        q, k, v, do = (place(to_bf16(a)) for a in (x.q, x.k, x.v, x.d_o))
+        al, be = place(x.alpha), place(x.beta)
+        bufs.append(DevBuf(wsb.value))
+        ws = _vp(bufs[-1])
+        sizes = [rows * d] * 4 + [rows * H] * 2
+        outs = [place(np.zeros(n, np.float32)) for n in sizes]
+        obufs = bufs[-6:]
+        _lib.call("asca_chunk_fwd", q, k, v, al, be, outs[0], ws, B, T, H, dh, C, None)
+        _lib.call("asca_chunk_bwd", q, k, v, do, ws, *outs[1:], B, T, H, dh, C, None)
+        _lib.call("asca_sync")
+        got.append([b.to_host((n + off,))[off:] for b, n in zip(obufs, sizes)])
+        for b in bufs:
+            b.free()
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)
+
+
 def test_chunked_config2_full_size(orc, g):
     # B=8, T=4096, H=16, dh=128, chunk 64, bf16 inputs, seed 0
     _check(orc, g, 0, 8, 4096, 16, 128, 64, "configs[2]")

@@ -331,3 +331,56 @@ def test_blocked_dh64_fused_unaligned(orc, g, shift):
     assert errs["o"] <= FWD_TOL and errs["d_qkv"] <= GRAD_TOL and errs["d_gate"] <= GRAD_TOL, errs
     for b in [*bufs, *small.values(), ws, o, dqkv, dgate]:
         b.free()
+
+
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("dh", [16, 32, 48, 96, 128])
+@pytest.mark.parametrize("B,T,H", [(1, 1, 1), (2, 15, 2), (1, 16, 3), (2, 33, 1), (3, 65, 2), (5, 50, 4)])
+def test_blocked_widths(orc, g, B, T, H, dh, off):
+    # The blocked kernels at every head width but 64 (tested above): lengths
+    # around their 16-step blocks, 32-step checkpoints and groups of blocks, odd
+    # unit counts, exact-zero and above-one gates; every array `off` floats past a
+    # 16-byte boundary; the raw and the fused gradients.  Bars as above.
+    import ctypes as C
+    from asca_amd import _lib
+    from asca_amd.gpu import DevBuf, _vp
+
+    x = orc.DeltaInputs(7 * dh + T, B, T, H, dh)
+    t = np.arange(B * T) % T
+    x.alpha[t % 7 == 3] = 0.0
+    x.alpha[t % 13 == 5] = 1.25
+    o_ref, dq, dk, dv, da, db = orc.delta_fwd_bwd(x.q, x.k, x.v, x.alpha, x.beta, x.d_o, B, T, H, dh)
+    d_qkv_ref, d_gate_ref = orc.delta_fuse(x.q, x.k, x.qn, x.kn, x.alpha, x.beta, dq, dk, dv, da, db, H, dh)
+    rows, d = B * T, H * dh
+    bufs = []
+
+    def placed(a):
+        bufs.append(DevBuf((a.size + off) * 4))
+        bufs[-1].upload(np.concatenate([np.zeros(off, np.float32), a.ravel()]))
+        return _vp(bufs[-1].ptr + 4 * off)
+
+    def out(n):
+        return placed(np.zeros(n, np.float32)), bufs[-1], n
+
+    def host(o, shape):
+        return o[1].to_host((o[2] + off,))[off:].reshape(shape)
+
+    q, k, v, al, be, qn, kn, do = (placed(getattr(x, n)) for n in
+                                   ("q", "k", "v", "alpha", "beta", "qn", "kn", "d_o"))
+    wsb = C.c_size_t()
+    _lib.call("asca_delta_ws_bytes", B, T, H, dh, C.byref(wsb))
+    bufs.append(DevBuf(wsb.value))
+    ws = _vp(bufs[-1])
+    o, raw = out(rows * d), [out(rows * d) for _ in range(3)] + [out(rows * H) for _ in range(2)]
+    dqkv, dgate = out(rows * 3 * d), out(rows * 2 * H)
+    _lib.call("asca_delta_fwd", q, k, v, al, be, o[0], ws, B, T, H, dh, None)
+    _lib.call("asca_delta_bwd_raw", q, k, v, al, be, do, ws, *[r[0] for r in raw], B, T, H, dh, None)
+    _lib.call("asca_delta_bwd_fused", q, k, v, al, be, qn, kn, do, ws, dqkv[0], dgate[0], B, T, H, dh, None)
+    _lib.call("asca_sync")
+    assert orc.rel_err(host(o, (rows, d)), o_ref) <= FWD_TOL
+    for r, ref in zip(raw, (dq, dk, dv, da, db)):
+        assert orc.rel_err(host(r, ref.shape), ref) <= GRAD_TOL
+    assert orc.rel_err(host(dqkv, (rows, 3 * d)), d_qkv_ref) <= GRAD_TOL
+    assert orc.rel_err(host(dgate, (rows, 2 * H)), d_gate_ref) <= GRAD_TOL
+    for b in bufs:
+        b.free()
