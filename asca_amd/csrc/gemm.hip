@@ -169,6 +169,12 @@ typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int SP_BK = 32;
 
+ASCA_DEV f32x2 buf_load2(Rsrc r, unsigned voff, unsigned soff) {
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+    const u32x2 x = __builtin_amdgcn_raw_buffer_load_b64(r, (int)voff, (int)soff, 0);
+    return f32x2{__uint_as_float(x[0]), __uint_as_float(x[1])};
+}
+
 // Elements c .. c + 3 of a run of n (> 0) valid floats, 0 past them: loads at
 // clamped places and no branch, since a conditional load is waited for on its
 // own.  at(i): element i.
@@ -380,7 +386,8 @@ ASCA_DEV float split_elem(const float* base, long ld, const int* rows, long off,
 
 // The sums of the NX x NY 16 x 16 tiles from (x0, y0) of a wave's 64 x 64 again,
 // as f32 products straight from memory.
-template <bool TA, bool TB, int NX, int NY>
+// (CB: columns of an mn-contiguous B interleaved over so many tiles)
+template <bool TA, bool TB, int CB, int NX, int NY>
 ASCA_DEV void split_redo(f32x4 (&acc)[NX][NY], int x0, int y0, const float* A, const float* B, const GemmArgs& p,
                          long a_off, long b_off, int m0, int n0, int lim_m, int lim_n, long K_lo, long K_hi,
                          int lane) {
@@ -399,7 +406,7 @@ ASCA_DEV void split_redo(f32x4 (&acc)[NX][NY], int x0, int y0, const float* A, c
                                    K_hi);
 #pragma unroll
         for (int y = 0; y < NY; ++y)
-            b[y] = split_elem<TB>(B, p.ldb, p.b_rows, b_off, n0, TB ? 16 * (y0 + y) + i : 4 * i + y0 + y, lim_n, kk,
+            b[y] = split_elem<TB>(B, p.ldb, p.b_rows, b_off, n0, TB ? 16 * (y0 + y) + i : CB * i + y0 + y, lim_n, kk,
                                   K_hi);
 #pragma unroll
         for (int x = 0; x < NX; ++x)
@@ -518,7 +525,7 @@ ASCA_DEV void split_mainloop(f32x4 (&acc)[4][4], const float* A, const float* B,
     for (; t < nk; ++t) step(std::false_type{});
     split_sign<TA>(acc, 0);
     if (split_bad(acc))
-        split_redo<TA, TB>(acc, 0, 0, A, B, p, a_off, b_off, m0 + wm, n0 + wn, lim_m - wm, lim_n - wn, K_lo, K_hi, lane);
+        split_redo<TA, TB, 4>(acc, 0, 0, A, B, p, a_off, b_off, m0 + wm, n0 + wn, lim_m - wm, lim_n - wn, K_lo, K_hi, lane);
 }
 
 // The tile, group and K range of a block.
@@ -541,13 +548,30 @@ struct BlockTile {
         K_hi = p.K;
         goff_g = 0;
         if (p.gmode == 1) {
+            // the group of row tile L / tiles_n: a wave's lanes count the tiles of 64
+            // groups at a time (one group after another, each bound read is waited for)
             int mt = L / p.tiles_n;
-            for (; g < p.ngroups; ++g) {
-                const int a = p.goff[g], b = p.goff[g + 1];
-                const int nt = (b - a + BM - 1) / BM;
-                if (mt < nt) break;
-                mt -= nt;
+            const int lane = threadIdx.x & 63;
+            for (; g < p.ngroups; g += 64) {
+                const int gl = min(g + lane, p.ngroups - 1);
+                const int nt = g + lane < p.ngroups ? (p.goff[gl + 1] - p.goff[gl] + BM - 1) / BM : 0;
+                int upto = nt;  // tiles of groups g .. g + lane
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int x = __shfl_up(upto, o);
+                    if (lane >= o) upto += x;
+                }
+                const unsigned long long past = __ballot(upto > mt);
+                if (past) {
+                    const int l = __builtin_ctzll(past);
+                    g += l;
+                    mt -= __builtin_amdgcn_readlane(upto - nt, l);
+                    break;
+                }
+                mt -= __builtin_amdgcn_readlane(upto, 63);
             }
+            g = __builtin_amdgcn_readfirstlane(g);
+            mt = __builtin_amdgcn_readfirstlane(mt);
             if (g >= p.ngroups) return false;
             tm = mt;
             goff_g = p.goff[g];
@@ -586,12 +610,14 @@ template <int N>
 ASCA_DEV void store_row(float* d, const float (&o)[N]) {
     if constexpr (N == 4)
         *reinterpret_cast<f32x4u*>(d) = f32x4u{o[0], o[1], o[2], o[3]};
-    else
+    else if constexpr (N == 2)
         *reinterpret_cast<f32x2u*>(d) = f32x2u{o[0], o[1]};
+    else
+        d[0] = o[0];
 }
 
 // C of the NX x NY 16 x 16 tiles from (x0, y0) of the wave's 64 x 64 at (m0, n0).
-template <bool TA, bool TB, int EPI, int NX, int NY, class T>
+template <bool TA, bool TB, int EPI, int CB, int NX, int NY, class T>
 ASCA_DEV void gemm_epilogue(const f32x4 (&acc)[NX][NY], int x0, int y0, int m0, int n0, const T& t, const GemmArgs& p,
                             int lane) {
     constexpr bool A_KC = !TA, B_KC = TB;
@@ -606,7 +632,7 @@ ASCA_DEV void gemm_epilogue(const f32x4 (&acc)[NX][NY], int x0, int y0, int m0, 
     // indices, residual, C and pre of four rows at a time.  A load under a
     // per-element condition is waited for on its own, one latency per element.
     constexpr int NS = B_KC ? 16 : 1;
-    const int nc0 = B_KC ? n0 + 16 * y0 + (lane & 15) : n0 + 4 * (lane & 15) + y0;
+    const int nc0 = B_KC ? n0 + 16 * y0 + (lane & 15) : n0 + CB * (lane & 15) + y0;
     const int nmax = p.N - 1;
     float bv[NY];
     if (bias) {
@@ -712,7 +738,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
     if (t.K_hi > t.K_lo)
         split_mainloop<TA, TB, GATHER, WM, WN, DB>(acc, t.A, t.B, p, t.a_off, t.b_off, t.m0, t.n0, t.lim_m, t.lim_n,
                                                    t.K_lo, t.K_hi, tid, wm, wn);
-    gemm_epilogue<TA, TB, EPI>(acc, 0, 0, t.m0 + wm, t.n0 + wn, t, p, lane);
+    gemm_epilogue<TA, TB, EPI, 4>(acc, 0, 0, t.m0 + wm, t.n0 + wn, t, p, lane);
 }
 
 // Products too small to fill the chip with the tiles above: one 64 x 64 tile
@@ -724,22 +750,23 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
 // Loads are buffer loads (32-bit lane offsets, the k-tile's offset in a scalar
 // register: 64-bit addresses would take the registers the fragments need), so
 // an operand's rows must lie within 4 GB (small_fits).
-// NEG: odd rows negated.
-template <bool KC, bool GATHER, bool NEG>
+// NTL 16-row tiles (mn-contiguous: row NTL i + j is row i of tile j).  NEG: odd
+// rows negated.
+template <bool KC, bool GATHER, bool NEG, int NTL>
 struct FragTile {
     const float* base;           // KC: k = K_lo of row 0; MC: k = K_lo of the tile's first column
-    unsigned vo[KC ? 4 : 1];     // lane's byte offsets: KC: row 16 x + i at its k; MC: its k and column 4 i
+    unsigned vo[KC ? NTL : 1];   // lane's byte offsets: KC: row 16 x + i at its k; MC: its k and column NTL i
     long ld;
     int kofs, col;
-    f32x4 x[8];  // KC: [2 x + half]; MC: [k]
+    f32x4 x[KC ? 2 * NTL : 8];   // KC: [2 x + half]; MC: [k], NTL columns
     ASCA_DEV void init(const float* b, long ld_, const int* rows, long off, int mn0, int lim_mn, long K_lo, int lane) {
         ld = ld_;
         kofs = 8 * (lane >> 4);
-        col = 4 * (lane & 15);
+        col = NTL * (lane & 15);
         if constexpr (KC) {
             base = b + (rows ? 0 : (off + mn0) * ld) + K_lo;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
+            for (int j = 0; j < NTL; ++j) {
                 const int r = min(16 * j + (lane & 15), lim_mn - 1);
                 vo[j] = (unsigned)(((rows ? rows[off + mn0 + r] : r) * ld + kofs) * 4);
             }
@@ -748,7 +775,7 @@ struct FragTile {
             vo[0] = (unsigned)(((GATHER ? 0 : kofs * ld) + (col < lim_mn ? col : 0)) * 4);
         }
     }
-    ASCA_DEV static bool whole(int lim_mn) { return KC || lim_mn >= 64 || lim_mn % 4 == 0; }
+    ASCA_DEV static bool whole(int lim_mn) { return KC || lim_mn >= 16 * NTL || lim_mn % NTL == 0; }
     static ASCA_DEV f32x4 ld4(Rsrc r, unsigned vo, unsigned so) {
         const float4 v = buf_load4(r, vo, so);
         return f32x4{v.x, v.y, v.z, v.w};
@@ -760,7 +787,7 @@ struct FragTile {
         if constexpr (KC) {
             const Rsrc r = make_rsrc(base + k, ~0u);
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < NTL; ++j)
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     if constexpr (WHOLE) {
@@ -783,11 +810,21 @@ struct FragTile {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 if constexpr (WHOLE) {
-                    x[e] = ld4(r, v[e], so[e]);
+                    if constexpr (NTL == 4) {
+                        x[e] = ld4(r, v[e], so[e]);
+                    } else if constexpr (NTL == 2) {
+                        const f32x2 u = buf_load2(r, v[e], so[e]);
+                        x[e][0] = u[0];
+                        x[e][1] = u[1];
+                    } else {
+                        x[e][0] = buf_load1(r, v[e], so[e]);
+                    }
                 } else {
                     const unsigned c0 = v[e] - 4 * (col < lim_mn ? col : 0);
-                    const f32x4 u = ld4_edge(col, lim_mn, [&](int i) { return buf_load1(r, c0 + 4 * i, 0); });
-                    x[e] = kofs + e < lk ? u : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int c = 0; c < NTL; ++c) x[e][c] = buf_load1(r, c0 + 4 * min(col + c, lim_mn - 1), 0);
+#pragma unroll
+                    for (int c = 0; c < NTL; ++c) x[e][c] = kofs + e < lk && col + c < lim_mn ? x[e][c] : 0.0f;
                 }
             }
         }
@@ -801,8 +838,8 @@ struct FragTile {
             float a = KC ? x[2 * j + e / 2][2 * (e & 1)] : x[2 * e][j];
             float b = KC ? x[2 * j + e / 2][2 * (e & 1) + 1] : x[2 * e + 1][j];
             if constexpr (NEG) {
-                a = neg_if(a, KC ? col & 4 : j & 1);  // col / 4 = lane % 16: the KC lane's row
-                b = neg_if(b, KC ? col & 4 : j & 1);
+                a = neg_if(a, KC ? col & NTL : j & 1);  // col / NTL = lane % 16: the KC lane's row
+                b = neg_if(b, KC ? col & NTL : j & 1);
             }
             unsigned w0, w1, w2;
             split2(a, b, w0, w1, w2);
@@ -815,24 +852,28 @@ struct FragTile {
     }
 };
 
+// NX x NY tiles of 16 x 16 per block: 4 x 4, or fewer columns or rows where
+// those leave CUs idle (decode: few rows, the weights streamed once).
 constexpr int SM_NW = 8;  // waves of a small-product block
-template <bool TA, bool TB, int EPI, int GATHER>
-__global__ __launch_bounds__(64 * SM_NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_small_k(GemmArgs p) {
-    BlockTile<TA, TB, 64, 64> t;
+template <bool TA, bool TB, int EPI, int GATHER, int NX, int NY>
+__global__ __launch_bounds__(64 * SM_NW) __attribute__((amdgpu_waves_per_eu(NX == 1 ? 4 : 2))) void gemm_small_k(
+    GemmArgs p) {
+    static_assert(!TA || NX == 4, "tile rows of A^T");
+    BlockTile<TA, TB, 16 * NX, 16 * NY> t;
     if (!t.init(p)) return;
     extern __shared__ float4 lds4[];
     f32x4* const part = reinterpret_cast<f32x4*>(lds4);  // [wave][tile][lane]
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    f32x4 acc[4][4];
+    f32x4 acc[NX][NY];
 #pragma unroll
-    for (int x = 0; x < 4; ++x)
+    for (int x = 0; x < NX; ++x)
 #pragma unroll
-        for (int y = 0; y < 4; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int y = 0; y < NY; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
     const long nk = (t.K_hi - t.K_lo + SP_BK - 1) / SP_BK;
     if (w < nk) {
-        FragTile<!TA, GATHER == 1, true> fa;
-        FragTile<TB, GATHER == 2, false> fb;
+        FragTile<!TA, GATHER == 1, true, NX> fa;
+        FragTile<TB, GATHER == 2, false, NY> fb;
         fa.init(t.A, p.lda, p.a_rows, t.a_off, t.m0, t.lim_m, t.K_lo, lane);
         fb.init(t.B, p.ldb, p.b_rows, t.b_off, t.n0, t.lim_n, t.K_lo, lane);
         const bool whole = fa.whole(t.lim_m) && fb.whole(t.lim_n);
@@ -854,47 +895,51 @@ __global__ __launch_bounds__(64 * SM_NW) __attribute__((amdgpu_waves_per_eu(2, 2
         load_b(w);
 #pragma unroll 1
         for (long kt = w;;) {
-            bf16x8 a[4][3];
+            bf16x8 a[NX][3];
 #pragma unroll
-            for (int x = 0; x < 4; ++x) fa.frag(x, a[x]);
+            for (int x = 0; x < NX; ++x) fa.frag(x, a[x]);
             kt += SM_NW;
             if (kt < nk) load_a(kt);
             // one column tile at a time: its fragments are split beside the
             // products of the one before (all at once, the registers spill)
 #pragma unroll
-            for (int y = 0; y < 4; ++y) {
+            for (int y = 0; y < NY; ++y) {
                 bf16x8 b[3];
                 fb.frag(y, b);
                 constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
                 for (int s = 0; s < 6; ++s)
 #pragma unroll
-                    for (int x = 0; x < 4; ++x)
+                    for (int x = 0; x < NX; ++x)
                         acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[x][PA[s]], b[PB[s]], acc[x][y], 0, 0, 0);
-                if (y < 3) __builtin_amdgcn_sched_barrier(0);
+                if (y < NY - 1) __builtin_amdgcn_sched_barrier(0);
             }
             if (kt < nk) load_b(kt);
             if (kt >= nk) break;
         }
     }
+    constexpr int TL = NX * NY, PW = TL > SM_NW ? TL / SM_NW : 1;  // tiles; tiles a wave adds up
+    static_assert(NY % PW == 0 && TL <= SM_NW * PW, "sums per wave");
 #pragma unroll
-    for (int x = 0; x < 4; ++x)
+    for (int x = 0; x < NX; ++x)
 #pragma unroll
-        for (int y = 0; y < 4; ++y) part[(w * 16 + 4 * x + y) * 64 + lane] = acc[x][y];
+        for (int y = 0; y < NY; ++y) part[(w * TL + NY * x + y) * 64 + lane] = acc[x][y];
     lds_barrier();
-    // wave w adds up and stores tiles (w / 2, 2 (w % 2)) and the one beside it
-    const int x0 = w >> 1, y0 = 2 * (w & 1);
-    f32x4 sum[1][2];
+    // wave w adds up and stores tiles PW w .. PW w + PW - 1
+    if (PW * w >= TL) return;
+    const int x0 = PW * w / NY, y0 = PW * w % NY;
+    f32x4 sum[1][PW];
 #pragma unroll
-    for (int y = 0; y < 2; ++y) {
-        sum[0][y] = part[(4 * x0 + y0 + y) * 64 + lane];
+    for (int y = 0; y < PW; ++y) {
+        sum[0][y] = part[(NY * x0 + y0 + y) * 64 + lane];
 #pragma unroll
-        for (int v = 1; v < SM_NW; ++v) sum[0][y] += part[(v * 16 + 4 * x0 + y0 + y) * 64 + lane];
+        for (int v = 1; v < SM_NW; ++v) sum[0][y] += part[(v * TL + NY * x0 + y0 + y) * 64 + lane];
     }
     split_sign<TA>(sum, x0);
     if (split_bad(sum))
-        split_redo<TA, TB>(sum, x0, y0, t.A, t.B, p, t.a_off, t.b_off, t.m0, t.n0, t.lim_m, t.lim_n, t.K_lo, t.K_hi, lane);
-    gemm_epilogue<TA, TB, EPI>(sum, x0, y0, t.m0, t.n0, t, p, lane);
+        split_redo<TA, TB, NY>(sum, x0, y0, t.A, t.B, p, t.a_off, t.b_off, t.m0, t.n0, t.lim_m, t.lim_n, t.K_lo, t.K_hi,
+                               lane);
+    gemm_epilogue<TA, TB, EPI, NY>(sum, x0, y0, t.m0, t.n0, t, p, lane);
 }
 
 // Persistent batched products (gmode 3, plain epilogue): a block walks work
@@ -1128,11 +1173,11 @@ static int launch_gemm_t(const GemmArgs& a, dim3 grid, hipStream_t st) {
     return ASCA_OK;
 }
 
-template <bool TA, bool TB, int EPI, int GATHER>
+template <bool TA, bool TB, int EPI, int GATHER, int NX, int NY>
 static int launch_small_t(const GemmArgs& a, dim3 grid, hipStream_t st) {
-    constexpr size_t lds = (size_t)SM_NW * 64 * 64 * sizeof(float);
-    if (int arc = allow_lds(reinterpret_cast<const void*>(&gemm_small_k<TA, TB, EPI, GATHER>), lds)) return arc;
-    hipLaunchKernelGGL((gemm_small_k<TA, TB, EPI, GATHER>), grid, dim3(64 * SM_NW), lds, st, a);
+    constexpr size_t lds = (size_t)SM_NW * 256 * NX * NY * sizeof(float);
+    if (int arc = allow_lds(reinterpret_cast<const void*>(&gemm_small_k<TA, TB, EPI, GATHER, NX, NY>), lds)) return arc;
+    hipLaunchKernelGGL((gemm_small_k<TA, TB, EPI, GATHER, NX, NY>), grid, dim3(64 * SM_NW), lds, st, a);
     return ASCA_OK;
 }
 
@@ -1176,6 +1221,32 @@ static Tile best_tile(long M, long N, int groups, long mult, long steps, bool sm
     }
     if (us) *us = t;
     return best;
+}
+// Shape of the small tile, in 16 x 16 tiles: one row tile where the rows (of a
+// group on average) do not pass 16 -- a 64-row tile would split and multiply
+// mostly padding -- and fewer columns per block while the blocks fill less than
+// half of the CUs.  One token for 64 sequences of the 8-layer d = 512 model (16 experts)
+// 834 -> 676 us: its projections 15.8 -> 9.9 us each, its expert products 25.6 ->
+// 15.0.  Sixteen waves per block instead of eight were slower (the 64 x 16 tile spills).
+static void small_shape(long M, long N, int groups, long mult, int& nx, int& ny) {
+    const long cus = cu_count() > 0 ? cu_count() : 256;
+    const long rows = groups > 0 ? M / groups : M;
+    if (rows <= 16) {
+        nx = 1;
+        return;
+    }
+    const long tm = mult * (groups > 0 ? groups : 1) * ((rows + 63) / 64);
+    if (2 * tm * ((N + 63) / 64) <= cus) ny = 2;
+    if (2 * tm * ((N + 31) / 32) <= cus) ny = 1;
+}
+template <bool TA, bool TB, int EPI, int GATHER>
+static int launch_small(const GemmArgs& a, int nx, int ny, dim3 grid, hipStream_t st) {
+    if constexpr (!TA) {
+        if (nx == 1) return launch_small_t<TA, TB, EPI, GATHER, 1, 4>(a, grid, st);
+        if (ny == 2) return launch_small_t<TA, TB, EPI, GATHER, 4, 2>(a, grid, st);
+        if (ny == 1) return launch_small_t<TA, TB, EPI, GATHER, 4, 1>(a, grid, st);
+    }
+    return launch_small_t<TA, TB, EPI, GATHER, 4, 4>(a, grid, st);
 }
 // The small tile addresses an operand tile with 32-bit byte offsets: 64 rows
 // (or 32 k-rows) of the leading dimension, or all `rows` of a gathered operand.
@@ -1223,7 +1294,12 @@ int gemm_launch(int ta, int tb, int epi, GemmArgs a, long m_total, hipStream_t s
     const long k_each = a.gmode == 2 ? m_total / max(a.ngroups, 1) : a.k_per_split;
     const Tile tile = best_tile(a.gmode == 1 ? m_total : a.M, a.N, a.gmode == 1 ? a.ngroups : 0,
                                 a.gmode >= 2 ? a.ngroups : splits, (k_each + SP_BK - 1) / SP_BK, small_ok, nullptr);
-    const int bm = tile == T_SMALL ? 64 : GM_BM, bn = batched ? 128 : tile == T_SMALL ? 64 : tile == T_WIDE ? 256 : 128;
+    // the small tile's rows and columns (16 nx x 16 ny)
+    int nx = 4, ny = 4;
+    if (tile == T_SMALL && !ta) small_shape(a.gmode == 1 ? m_total : a.M, a.N, a.gmode == 1 ? a.ngroups : 0,
+                                            a.gmode == 3 ? a.ngroups : splits, nx, ny);
+    const int bm = tile == T_SMALL ? 16 * nx : GM_BM;
+    const int bn = batched ? 128 : tile == T_SMALL ? 16 * ny : tile == T_WIDE ? 256 : 128;
     a.tiles_n = (a.N + bn - 1) / bn;
     a.tiles_m = batched ? (a.M + 64 * wm - 1) / (64 * wm) : (a.M + bm - 1) / bm;
     long blocks;
@@ -1244,7 +1320,7 @@ int gemm_launch(int ta, int tb, int epi, GemmArgs a, long m_total, hipStream_t s
         return fail(ASCA_ERR_UNSUPPORTED, "%s: one gathered operand, of A^T B", name);
 #define ASCA_GEMM_CASE(TA_, TB_, EPI_, G_)                                              \
     if (ta == TA_ && tb == TB_ && epi == EPI_ && gather == G_)                          \
-        rc = tile == T_SMALL  ? launch_small_t<TA_, TB_, EPI_, G_>(a, grid, st)         \
+        rc = tile == T_SMALL  ? launch_small<TA_, TB_, EPI_, G_>(a, nx, ny, grid, st)   \
              : tile == T_WIDE ? launch_gemm_t<TA_, TB_, EPI_, G_, 2, 4, true>(a, grid, st) \
                               : launch_gemm_t<TA_, TB_, EPI_, G_, 2, 2, false>(a, grid, st); \
     else
