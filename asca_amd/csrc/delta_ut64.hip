@@ -1,6 +1,6 @@
 // Gated delta rule in the blocked (UT) form: the launchers, and the f32 dh = 64
-// forward and fused backward on 16-byte-aligned rows (the configs[1] / training
-// hot path).  The kernels are in ut64_kernels.h; the other head widths and
+// forward and fused backward on 16-byte-aligned rows (the training hot
+// path).  The kernels are in ut64_kernels.h; the other head widths and
 // variants are launched from delta_ut64_b.hip and delta_utn.hip.
 #include "ut64_kernels.h"
 

@@ -38,6 +38,7 @@ struct GemmArgs {
     int tiles_m, tiles_n;
     long k_per_split;     // split-K: K range of blockIdx.y
     long c_split_stride;  // split-K: partial buffer stride per split
+    int cus, tail_max, tail_blocks;  // gemm_wide_k: tiles of its last round (set by gemm_launch)
 };
 
 GemmArgs gemm_args();

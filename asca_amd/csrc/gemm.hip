@@ -535,21 +535,40 @@ struct BlockTile {
     long K_lo, K_hi, goff_g, a_off, b_off;
     const float *A, *B, *bias, *resid;
     float* C;
-    // false: a surplus block (a grouped grid is an upper bound)
+    // Row tiles of all groups (gmode 1): 64 groups at a time, a wave's lanes count
+    // their tiles (one group after another, each bound read is waited for).
+    ASCA_DEV static int row_tiles(const GemmArgs& p) {
+        int n = 0;
+        const int lane = threadIdx.x & 63;
+        for (int g = lane; g < p.ngroups; g += 64) n += (p.goff[g + 1] - p.goff[g] + BM - 1) / BM;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) n += __shfl_xor(n, o);
+        return __builtin_amdgcn_readfirstlane(n);
+    }
+    ASCA_DEV static int total(const GemmArgs& p) {
+        return p.tiles_n * (p.gmode == 1 ? row_tiles(p) : p.gmode == 0 ? p.tiles_m : p.tiles_m * p.ngroups);
+    }
+    // Block b of n -> tile, XCD-aware: hardware places block i on XCD i % 8, so
+    // give each XCD a contiguous run of tiles (neighbours share operand rows).
+    ASCA_DEV static int of_block(int b, int n) {
+        const int x = b & 7;
+        return x * (n >> 3) + min(x, n & 7) + (b >> 3);
+    }
+    // The block's tile; false: a surplus block (a grouped grid is an upper bound).
     ASCA_DEV bool init(const GemmArgs& p) {
-        // block -> tile, XCD-aware: hardware places block i on XCD i % 8, so give
-        // each XCD a contiguous run of logical tiles (neighbours share operand rows)
-        int L = blockIdx.x;
-        const int nb = gridDim.x;
-        if ((nb & 7) == 0) L = (L & 7) * (nb >> 3) + (L >> 3);
+        const int n = p.gmode == 1 ? total(p) : (int)gridDim.x;
+        if ((int)blockIdx.x >= n) return false;
+        init(p, of_block(blockIdx.x, n));
+        return true;
+    }
+    // Tile L (below total()).
+    ASCA_DEV void init(const GemmArgs& p, int L) {
         int g = 0, tm, tn = L % p.tiles_n;
         Mg = p.M;
         K_lo = 0;
         K_hi = p.K;
         goff_g = 0;
         if (p.gmode == 1) {
-            // the group of row tile L / tiles_n: a wave's lanes count the tiles of 64
-            // groups at a time (one group after another, each bound read is waited for)
             int mt = L / p.tiles_n;
             const int lane = threadIdx.x & 63;
             for (; g < p.ngroups; g += 64) {
@@ -572,7 +591,6 @@ struct BlockTile {
             }
             g = __builtin_amdgcn_readfirstlane(g);
             mt = __builtin_amdgcn_readfirstlane(mt);
-            if (g >= p.ngroups) return false;
             tm = mt;
             goff_g = p.goff[g];
             Mg = p.goff[g + 1] - p.goff[g];
@@ -602,7 +620,6 @@ struct BlockTile {
         resid = p.resid ? p.resid + g * p.r_gs : nullptr;
         a_off = ((p.gmode == 1 && !TA) || (p.gmode == 2 && TA)) ? goff_g : 0;
         b_off = (p.gmode == 2 && !TB) ? goff_g : 0;
-        return true;
     }
 };
 
@@ -724,10 +741,8 @@ ASCA_DEV void gemm_epilogue(const f32x4 (&acc)[NX][NY], int x0, int y0, int m0, 
 }
 
 // Block tile (64 WM) x (64 WN) on WM x WN waves; a wave owns 64 x 64.
-template <bool TA, bool TB, int EPI, int GATHER, int WM, int WN, bool DB>
-__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_k(GemmArgs p) {
-    BlockTile<TA, TB, 64 * WM, 64 * WN> t;
-    if (!t.init(p)) return;
+template <bool TA, bool TB, int EPI, int GATHER, int WM, int WN, bool DB, class T>
+ASCA_DEV void gemm_tile(const T& t, const GemmArgs& p) {
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int wm = (w / WN) * 64, wn = (w % WN) * 64;
     f32x4 acc[4][4];
@@ -739,6 +754,13 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
         split_mainloop<TA, TB, GATHER, WM, WN, DB>(acc, t.A, t.B, p, t.a_off, t.b_off, t.m0, t.n0, t.lim_m, t.lim_n,
                                                    t.K_lo, t.K_hi, tid, wm, wn);
     gemm_epilogue<TA, TB, EPI, 4>(acc, 0, 0, t.m0 + wm, t.n0 + wn, t, p, lane);
+}
+
+template <bool TA, bool TB, int EPI, int GATHER>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_k(GemmArgs p) {
+    BlockTile<TA, TB, 128, 128> t;
+    if (!t.init(p)) return;
+    gemm_tile<TA, TB, EPI, GATHER, 2, 2, false>(t, p);
 }
 
 // Products too small to fill the chip with the tiles above: one 64 x 64 tile
@@ -855,12 +877,9 @@ struct FragTile {
 // NX x NY tiles of 16 x 16 per block: 4 x 4, or fewer columns or rows where
 // those leave CUs idle (decode: few rows, the weights streamed once).
 constexpr int SM_NW = 8;  // waves of a small-product block
-template <bool TA, bool TB, int EPI, int GATHER, int NX, int NY>
-__global__ __launch_bounds__(64 * SM_NW) __attribute__((amdgpu_waves_per_eu(NX == 1 ? 4 : 2))) void gemm_small_k(
-    GemmArgs p) {
+template <bool TA, bool TB, int EPI, int GATHER, int NX, int NY, class T>
+ASCA_DEV void small_tile(const T& t, const GemmArgs& p) {
     static_assert(!TA || NX == 4, "tile rows of A^T");
-    BlockTile<TA, TB, 16 * NX, 16 * NY> t;
-    if (!t.init(p)) return;
     extern __shared__ float4 lds4[];
     f32x4* const part = reinterpret_cast<f32x4*>(lds4);  // [wave][tile][lane]
     const int lane = threadIdx.x & 63;
@@ -940,6 +959,46 @@ __global__ __launch_bounds__(64 * SM_NW) __attribute__((amdgpu_waves_per_eu(NX =
         split_redo<TA, TB, NY>(sum, x0, y0, t.A, t.B, p, t.a_off, t.b_off, t.m0, t.n0, t.lim_m, t.lim_n, t.K_lo, t.K_hi,
                                lane);
     gemm_epilogue<TA, TB, EPI, NY>(sum, x0, y0, t.m0, t.n0, t, p, lane);
+}
+
+template <bool TA, bool TB, int EPI, int GATHER, int NX, int NY>
+__global__ __launch_bounds__(64 * SM_NW) __attribute__((amdgpu_waves_per_eu(NX == 1 ? 4 : 2))) void gemm_small_k(
+    GemmArgs p) {
+    BlockTile<TA, TB, 16 * NX, 16 * NY> t;
+    if (!t.init(p)) return;
+    small_tile<TA, TB, EPI, GATHER, NX, NY>(t, p);
+}
+
+// 128 x 256 tiles on 8 waves, one block per CU.  Where the tiles leave a last
+// round that is nearly empty (at most p.tail_max of them beyond whole rounds of
+// p.cus, a number that a grouped launch knows only on the device), the last
+// p.tail_blocks blocks take those as 64 x 64 tiles, which all CUs share:
+// 17408 x 1024 x 512 (544 tiles, 32 past two rounds) 125 -> 108 us, its twin of
+// 16 groups (the routed FFN) alike, 17000 x 512 x 512 74 -> 55 us, 10900 x 1532 x
+// 240 74 -> 63 us; whole rounds as before (16384 x 1536 x 512 144 us).
+template <bool TA, bool TB, int EPI, int GATHER>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_wide_k(GemmArgs p) {
+    BlockTile<TA, TB, 128, 256> t;
+    const int n = t.total(p), rem = n % p.cus;
+    const int cut = p.tail_blocks && rem <= p.tail_max ? n - rem : n;
+    const int first = gridDim.x - p.tail_blocks;  // blocks of whole tiles
+    if ((int)blockIdx.x < first) {
+        if ((int)blockIdx.x >= cut) return;
+        t.init(p, t.of_block(blockIdx.x, cut));
+        gemm_tile<TA, TB, EPI, GATHER, 2, 4, true>(t, p);
+        return;
+    }
+    for (int i = blockIdx.x - first; i < 8 * (n - cut); i += p.tail_blocks) {
+        t.init(p, cut + (i >> 3));
+        const int dm = 64 * ((i >> 2) & 1), dn = 64 * (i & 3);
+        t.m0 += dm;
+        t.n0 += dn;
+        t.lim_m -= dm;
+        t.lim_n -= dn;
+        if (t.lim_m <= 0 || t.lim_n <= 0) continue;  // uniform
+        small_tile<TA, TB, EPI, GATHER, 4, 4>(t, p);
+        lds_barrier();  // the sums are read before the next tile's are written
+    }
 }
 
 // Persistent batched products (gmode 3, plain epilogue): a block walks work
@@ -1165,11 +1224,19 @@ static int ws_check(const Ws& ws, size_t floats, const char* name) {
     return ASCA_OK;
 }
 
-template <bool TA, bool TB, int EPI, int GATHER, int WM, int WN, bool DB>
+template <bool TA, bool TB, int EPI, int GATHER>
 static int launch_gemm_t(const GemmArgs& a, dim3 grid, hipStream_t st) {
-    constexpr size_t lds = (size_t)(DB ? 2 : 1) * (sp_tile<64 * WM>() + sp_tile<64 * WN>());
-    if (int arc = allow_lds(reinterpret_cast<const void*>(&gemm_k<TA, TB, EPI, GATHER, WM, WN, DB>), lds)) return arc;
-    hipLaunchKernelGGL((gemm_k<TA, TB, EPI, GATHER, WM, WN, DB>), grid, dim3(64 * WM * WN), lds, st, a);
+    constexpr size_t lds = 2 * (size_t)sp_tile<128>();
+    if (int arc = allow_lds(reinterpret_cast<const void*>(&gemm_k<TA, TB, EPI, GATHER>), lds)) return arc;
+    hipLaunchKernelGGL((gemm_k<TA, TB, EPI, GATHER>), grid, dim3(256), lds, st, a);
+    return ASCA_OK;
+}
+template <bool TA, bool TB, int EPI, int GATHER>
+static int launch_wide_t(const GemmArgs& a, dim3 grid, hipStream_t st) {
+    constexpr size_t lds = 2 * (size_t)(sp_tile<128>() + sp_tile<256>());
+    static_assert(lds >= (size_t)SM_NW * 64 * 64 * sizeof(float), "the 64 x 64 tiles' sums fit");
+    if (int arc = allow_lds(reinterpret_cast<const void*>(&gemm_wide_k<TA, TB, EPI, GATHER>), lds)) return arc;
+    hipLaunchKernelGGL((gemm_wide_k<TA, TB, EPI, GATHER>), grid, dim3(512), lds, st, a);
     return ASCA_OK;
 }
 
@@ -1193,11 +1260,24 @@ static int launch_small_t(const GemmArgs& a, dim3 grid, hipStream_t st) {
 // the small tile wins: 1000x1000x320 22 -> 9.5 us, 64x1536x512 30 -> 11 us,
 // 1000x320x1000 55 -> 19 us.
 enum Tile { T_SMALL, T_128, T_WIDE };
-static double tile_us(Tile t, long tiles, long steps) {
+// The most tiles beyond whole rounds that WIDE does as 64 x 64 tiles: while those
+// take less time than another round (32 of 256 at K = 512: 14 us against 45; a
+// tile is eight of them, so 96 are three rounds of 14 us).
+static long tail_max(long steps) {
+    const long cus = cu_count() > 0 ? cu_count() : 256;
+    const double small = 3.5 * (double)((steps + 7) / 8) + 7.0;
+    return (long)((2.5 * (double)steps + 5.0) / small) * cus / 8;
+}
+static double tile_us(Tile t, long tiles, long steps, bool tail) {
     const long cus = cu_count() > 0 ? cu_count() : 256;
     const double s = (double)steps;
     if (t == T_SMALL) return (double)((tiles + cus - 1) / cus) * (3.5 * (double)((steps + 7) / 8) + 7.0) - 4.0;
-    if (t == T_WIDE) return (double)((tiles + cus - 1) / cus) * (2.5 * s + 5.0);
+    if (t == T_WIDE) {
+        const long rem = tiles % cus;
+        const double round = 2.5 * s + 5.0;
+        const double last = rem == 0 ? 0.0 : tail && rem <= tail_max(steps) ? tile_us(T_SMALL, 8 * rem, steps, false) + 4.0 : round;
+        return (double)(tiles / cus) * round + last;
+    }
     const long full = tiles / (2 * cus), rem = tiles % (2 * cus);
     return (double)full * (2.8 * s + 4.0) + (rem == 0 ? 0.0 : rem <= cus ? 1.75 * s + 5.0 : 2.8 * s + 4.0);
 }
@@ -1208,12 +1288,14 @@ static long tile_count(Tile t, long M, long N, int groups) {
     if (groups <= 0) return (M + bm - 1) / bm * tn;
     return (groups * ((M / groups + bm - 1) / bm) + (groups + 1) / 2) * tn;
 }
-static Tile best_tile(long M, long N, int groups, long mult, long steps, bool small_ok, double* us) {
+static Tile best_tile(long M, long N, int groups, long mult, long steps, bool small_ok, bool whole_k, double* us) {
     Tile best = T_WIDE;
-    double t = tile_us(T_WIDE, mult * tile_count(T_WIDE, M, N, groups), steps);
+    // (one K range: the splits' blocks are not tiles of one launch dimension)
+    const bool tail = small_ok && whole_k;
+    double t = tile_us(T_WIDE, mult * tile_count(T_WIDE, M, N, groups), steps, tail);
     for (Tile c : {T_128, T_SMALL}) {
         if (c == T_SMALL && !small_ok) continue;
-        const double u = tile_us(c, mult * tile_count(c, M, N, groups), steps);
+        const double u = tile_us(c, mult * tile_count(c, M, N, groups), steps, false);
         if (u < t) {
             t = u;
             best = c;
@@ -1293,7 +1375,7 @@ int gemm_launch(int ta, int tb, int epi, GemmArgs a, long m_total, hipStream_t s
                           small_fits(max(a.ldb, 1L), a.b_rows ? grows : 64);
     const long k_each = a.gmode == 2 ? m_total / max(a.ngroups, 1) : a.k_per_split;
     const Tile tile = best_tile(a.gmode == 1 ? m_total : a.M, a.N, a.gmode == 1 ? a.ngroups : 0,
-                                a.gmode >= 2 ? a.ngroups : splits, (k_each + SP_BK - 1) / SP_BK, small_ok, nullptr);
+                                a.gmode >= 2 ? a.ngroups : splits, (k_each + SP_BK - 1) / SP_BK, small_ok, splits == 1, nullptr);
     // the small tile's rows and columns (16 nx x 16 ny)
     int nx = 4, ny = 4;
     if (tile == T_SMALL && !ta) small_shape(a.gmode == 1 ? m_total : a.M, a.N, a.gmode == 1 ? a.ngroups : 0,
@@ -1313,6 +1395,13 @@ int gemm_launch(int ta, int tb, int epi, GemmArgs a, long m_total, hipStream_t s
     if (blocks > 0x7fffffffL) return fail(ASCA_ERR_INVALID, "%s: grid too large", name);
     int rc = pre_launch(name);
     if (rc) return rc;
+    if (tile == T_WIDE && !batched) {
+        a.cus = cu_count() > 0 ? cu_count() : 256;
+        a.tail_max = splits == 1 && small_ok ? (int)tail_max((k_each + SP_BK - 1) / SP_BK) : 0;
+        const long rem = blocks % a.cus;
+        a.tail_blocks = a.tail_max == 0 ? 0 : a.gmode == 1 ? a.cus : rem <= a.tail_max ? (int)min((long)a.cus, 8 * rem) : 0;
+        blocks += a.tail_blocks;
+    }
     const dim3 grid((unsigned)blocks, (unsigned)splits);
     // operand whose K rows are gathered (mn-contiguous operands; k-contiguous ones gather rows in any variant)
     const int gather = ta && a.a_rows ? 1 : !tb && a.b_rows ? 2 : 0;
@@ -1321,8 +1410,8 @@ int gemm_launch(int ta, int tb, int epi, GemmArgs a, long m_total, hipStream_t s
 #define ASCA_GEMM_CASE(TA_, TB_, EPI_, G_)                                              \
     if (ta == TA_ && tb == TB_ && epi == EPI_ && gather == G_)                          \
         rc = tile == T_SMALL  ? launch_small<TA_, TB_, EPI_, G_>(a, nx, ny, grid, st)   \
-             : tile == T_WIDE ? launch_gemm_t<TA_, TB_, EPI_, G_, 2, 4, true>(a, grid, st) \
-                              : launch_gemm_t<TA_, TB_, EPI_, G_, 2, 2, false>(a, grid, st); \
+             : tile == T_WIDE ? launch_wide_t<TA_, TB_, EPI_, G_>(a, grid, st)          \
+                              : launch_gemm_t<TA_, TB_, EPI_, G_>(a, grid, st);         \
     else
 #define ASCA_GEMM_BATCHED(TA_, TB_)                                                                     \
     if (ta == TA_ && tb == TB_)                                                                         \
@@ -1641,8 +1730,8 @@ int gemm_run(int trans_a, int trans_b, int M, int N, int K, float alpha, const f
         // one pass over K where that is no slower than the partials and their sum
         double one, cut;
         const bool fits = small_fits(max(lda, 1L), 64) && small_fits(max(ldb, 1L), 64);
-        best_tile(M, N, 0, 1, (K + SP_BK - 1) / SP_BK, fits, &one);
-        best_tile(M, N, 0, splits, (kps + SP_BK - 1) / SP_BK, fits, &cut);
+        best_tile(M, N, 0, 1, (K + SP_BK - 1) / SP_BK, fits, true, &one);
+        best_tile(M, N, 0, splits, (kps + SP_BK - 1) / SP_BK, fits, false, &cut);
         if (one <= cut + 5.0 + 1e-6 * splits * M * N) splits = 1;
     }
     if (splits == 1) return gemm_launch(trans_a, trans_b, EPI_STORE, a, M, st, "gemm");
