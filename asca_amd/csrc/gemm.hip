@@ -1527,28 +1527,31 @@ int colsum_launch(const float* X, long rows, int N, long ldx, const int* goff, i
 // the 16-wide MFMA output tile matches them, where a 128-wide block tile of
 // the general kernel would multiply mostly padding.
 //
-// Forward Y (T x n) = X (T x K) W (K x n) + b: one wave per 16 rows.  Lane
+// Forward Y (T x n) = X (T x K) W (K x n) + b: one block per 16 rows, a quarter
+// of K to each of its four waves (a wave's loads and its chain of products are
+// the time of a decode step's few rows; the sums meet in LDS: 64 rows of K = 512
+// 8.7 -> 3.7 us, 16384 rows 12.0 -> 9.7).  Lane
 // (i = l % 16, q = l / 16) supplies A = X[row i][16 j + 4 q + e] from one
 // 16-byte load per 16-k group j (e = 0..3 are four MFMA k-steps: the k index
 // is permuted inside each group of 16, which the sum does not see) and keeps
-// the matching B = W[16 j + 4 q + e][i] for the whole K in registers.
-template <int KT>  // K = 16 KT
+// the matching B = W[16 j + 4 q + e][i] for its whole K in registers.
+template <int KT>  // K = 64 KT
 __global__ __launch_bounds__(256) void skinny_fwd_k(const float* __restrict__ X, long ldx, const float* __restrict__ W,
                                                     const float* __restrict__ b, float* __restrict__ Y, long T, int n) {
+    __shared__ f32x4 part[4][64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const long r0 = ((long)blockIdx.x * 4 + w) * 16;
-    if (r0 >= T) return;  // whole wave
+    const long r0 = (long)blockIdx.x * 16;
     const int i = lane & 15, q = lane >> 4;
-    const int ic = min(i, n - 1);
+    const int ic = min(i, n - 1), k0 = 16 * KT * w + 4 * q;
     float wb[4 * KT];
 #pragma unroll
     for (int j = 0; j < KT; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float v = W[(long)(16 * j + 4 * q + e) * n + ic];
+            const float v = W[(long)(k0 + 16 * j + e) * n + ic];
             wb[4 * j + e] = i < n ? v : 0.0f;
         }
-    const float* xr = X + min(r0 + i, T - 1) * ldx + 4 * q;
+    const float* xr = X + min(r0 + i, T - 1) * ldx + k0;
     float4 xv[KT];
 #pragma unroll
     for (int j = 0; j < KT; ++j) xv[j] = *reinterpret_cast<const float4*>(xr + 16 * j);
@@ -1563,6 +1566,10 @@ __global__ __launch_bounds__(256) void skinny_fwd_k(const float* __restrict__ X,
         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[j].z, wb[4 * j + 2], acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[j].w, wb[4 * j + 3], acc, 0, 0, 0);
     }
+    part[w][lane] = acc;
+    __syncthreads();
+    if (w) return;
+    acc = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
     const float bi = b ? b[ic] : 0.0f;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -1572,53 +1579,69 @@ __global__ __launch_bounds__(256) void skinny_fwd_k(const float* __restrict__ X,
 }
 
 // Weight gradient G (K x n) = X^T D and bias gradient db = column sums of D,
-// over T rows.  Wave (tile it, chunk s) reduces rows s*SK_T .. +SK_T into a
-// 16 x 16 partial of G (i = 16 it + lane % 16): per MFMA k-step the four lane
-// groups q take rows t = 4 m + q, lane (i, q) supplies X[t][16 it + i] and
-// D[t][i].  Waves of tile 0 also sum their D values for db.  Partials go to
-// part[s][K + 1][16] (row K: db) and skinny_reduce_k adds them in a fixed order.
-constexpr int SK_T = 256;  // rows per wave
+// over T rows.  Block (64 columns of X, chunk s) reduces rows s*SK_T .. +SK_T
+// into a 64 x 16 partial of G, its four waves a quarter of the rows each: per
+// MFMA k-step the four lane groups q take rows t = 4 m + q, lane (i, q) supplies
+// X[t][64 it + 4 i .. + 3] (16 bytes; the four columns go to four output tiles)
+// and D[t][i].  The kernel is the reading of X, so a wave has all its loads in
+// flight and rows are read 256 bytes at a time.  Blocks of it = 0 also sum D for
+// db.  Partials go to part[s][K + 1][16] (row K: db) and skinny_reduce_k adds
+// them in a fixed order.  16384 x 512: 75 us with a wave per 16 columns (64 bytes
+// of a row, each 128-byte line read by two XCDs), 28 us beside the backward's
+// products.
+constexpr int SK_T = 256;  // rows per block
 __global__ __launch_bounds__(256) void skinny_wgrad_k(const float* __restrict__ X, long ldx,
                                                       const float* __restrict__ D, long T, int K, int n,
                                                       float* __restrict__ part) {
+    __shared__ float4 red[4][16 * 16];  // [wave][column of X, output column / 4]
+    __shared__ float red_db[4][16];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int it = blockIdx.x;
-    const long s = (long)blockIdx.y * 4 + w;
-    const long nch = (T + SK_T - 1) / SK_T;
-    if (s >= nch) return;  // whole wave
+    const int it = blockIdx.x % (K / 64);
+    const long s = blockIdx.x / (K / 64);
     const int i = lane & 15, q = lane >> 4;
     const int ic = min(i, n - 1);
-    const long t0 = s * SK_T;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    const long t0 = s * SK_T + w * (SK_T / 4) + q;
+    f32x4 acc[4] = {};
     float dsum = 0.0f;
-    constexpr int NM = SK_T / 4;
-    constexpr int G = 16;  // k-steps whose loads are issued together
-#pragma unroll 1
-    for (int m0 = 0; m0 < NM; m0 += G) {
-        float av[G], bv[G];
+    constexpr int NM = SK_T / 16;
+    float4 av[NM];
+    float bv[NM];
 #pragma unroll
-        for (int u = 0; u < G; ++u) {
-            const long t = t0 + 4 * (m0 + u) + q;
-            const long tc = min(t, T - 1);
-            const float xa = X[tc * ldx + 16 * it + i];
-            const float db = D[tc * n + ic];
-            av[u] = t < T ? xa : 0.0f;
-            bv[u] = (t < T && i < n) ? db : 0.0f;
-        }
-        __builtin_amdgcn_sched_barrier(0);  // the group's loads go out together
-#pragma unroll
-        for (int u = 0; u < G; ++u) {
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u], bv[u], acc, 0, 0, 0);
-            dsum += bv[u];
-        }
+    for (int m = 0; m < NM; ++m) {
+        const long t = min(t0 + 4 * m, T - 1);
+        av[m] = *reinterpret_cast<const float4*>(X + t * ldx + 64 * it + 4 * i);
+        bv[m] = D[t * n + ic];
     }
-    float* ps = part + s * (long)(K + 1) * 16;
+    __builtin_amdgcn_sched_barrier(0);  // the loads go out together
 #pragma unroll
-    for (int r = 0; r < 4; ++r) ps[(16 * it + 4 * q + r) * 16 + i] = acc[r];
+    for (int m = 0; m < NM; ++m) {
+        const bool in = t0 + 4 * m < T;
+        const float b = in && i < n ? bv[m] : 0.0f;
+        acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? av[m].x : 0.0f, b, acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? av[m].y : 0.0f, b, acc[1], 0, 0, 0);
+        acc[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? av[m].z : 0.0f, b, acc[2], 0, 0, 0);
+        acc[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? av[m].w : 0.0f, b, acc[3], 0, 0, 0);
+        dsum += b;
+    }
+    float* const mine = reinterpret_cast<float*>(red[w]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) mine[(16 * q + 4 * r + u) * 16 + i] = acc[u][r];
     if (it == 0) {
         dsum += __shfl_xor(dsum, 16);
         dsum += __shfl_xor(dsum, 32);
-        if (q == 0) ps[K * 16 + i] = dsum;
+        if (q == 0) red_db[w][i] = dsum;
+    }
+    __syncthreads();
+    float* const ps = part + s * (long)(K + 1) * 16;
+    const float4 a = red[0][threadIdx.x], b = red[1][threadIdx.x], c = red[2][threadIdx.x], d = red[3][threadIdx.x];
+    reinterpret_cast<float4*>(ps + 64 * it * 16)[threadIdx.x] =
+        make_float4((a.x + b.x) + (c.x + d.x), (a.y + b.y) + (c.y + d.y), (a.z + b.z) + (c.z + d.z),
+                    (a.w + b.w) + (c.w + d.w));
+    if (it == 0 && threadIdx.x < 16) {
+        const int j = threadIdx.x;
+        ps[K * 16 + j] = (red_db[0][j] + red_db[1][j]) + (red_db[2][j] + red_db[3][j]);
     }
 }
 
@@ -1632,7 +1655,14 @@ __global__ __launch_bounds__(256) void skinny_reduce_k(const float* __restrict__
     if (row > K) return;  // whole wave
     const int c = lane & 15, g = lane >> 4;
     float acc = 0.0f;
-    for (long s = g; s < nch; s += 4) acc += part[(s * (K + 1) + row) * 16 + c];
+    for (long s = g; s < nch; s += 4 * CS_U) {
+        float x[CS_U];
+#pragma unroll
+        for (int u = 0; u < CS_U; ++u) x[u] = part[(min(s + 4 * u, nch - 1) * (K + 1) + row) * 16 + c];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < CS_U; ++u) acc += s + 4 * u < nch ? x[u] : 0.0f;
+    }
     acc += __shfl_xor(acc, 16);
     acc += __shfl_xor(acc, 32);
     if (g == 0 && c < n) {
@@ -1667,13 +1697,13 @@ int skinny_fwd_launch(const float* X, long ldx, const float* W, const float* b, 
     }
     int rc = pre_launch("skinny_fwd");
     if (rc) return rc;
-    const dim3 grid((unsigned)((T + 63) / 64));
+    const dim3 grid((unsigned)((T + 15) / 16));
     if (K == 512)
-        hipLaunchKernelGGL(skinny_fwd_k<32>, grid, dim3(256), 0, st, X, ldx, W, b, Y, T, n);
-    else if (K == 256)
-        hipLaunchKernelGGL(skinny_fwd_k<16>, grid, dim3(256), 0, st, X, ldx, W, b, Y, T, n);
-    else
         hipLaunchKernelGGL(skinny_fwd_k<8>, grid, dim3(256), 0, st, X, ldx, W, b, Y, T, n);
+    else if (K == 256)
+        hipLaunchKernelGGL(skinny_fwd_k<4>, grid, dim3(256), 0, st, X, ldx, W, b, Y, T, n);
+    else
+        hipLaunchKernelGGL(skinny_fwd_k<2>, grid, dim3(256), 0, st, X, ldx, W, b, Y, T, n);
     return post_launch("skinny_fwd");
 }
 
@@ -1687,7 +1717,7 @@ size_t skinny_wgrad_ws_floats(long T, int K, int n) {
 int skinny_wgrad_launch(const float* X, long ldx, const float* D, float* G, float* db, long T, int K, int n,
                         Ws ws, hipStream_t st) {
     if (n <= 0 || K <= 0) return ASCA_OK;
-    if (T <= 0 || !skinny_ok(X, ldx, K, n) || K % 16) {
+    if (T <= 0 || !skinny_ok(X, ldx, K, n)) {
         int rc = gemm_run(1, 0, K, n, (int)T, 1.0f, X, ldx, D, n, 0.0f, G, n, nullptr, ws, st);
         if (rc || !db) return rc;
         return colsum_launch(D, T, n, n, nullptr, 0, db, 0, ws, st);
@@ -1697,8 +1727,8 @@ int skinny_wgrad_launch(const float* X, long ldx, const float* D, float* G, floa
     if (rc) return rc;
     float* const part = ws.p;
     if ((rc = pre_launch("skinny_wgrad"))) return rc;
-    hipLaunchKernelGGL(skinny_wgrad_k, dim3((unsigned)(K / 16), (unsigned)((nch + 3) / 4)), dim3(256), 0, st, X, ldx,
-                       D, T, K, n, part);
+    hipLaunchKernelGGL(skinny_wgrad_k, dim3((unsigned)(K / 64 * nch)), dim3(256), 0, st, X, ldx, D, T, K, n,
+                       part);
     if ((rc = post_launch("skinny_wgrad"))) return rc;
     if ((rc = pre_launch("skinny_reduce"))) return rc;
     hipLaunchKernelGGL(skinny_reduce_k, dim3((unsigned)((K + 1 + 3) / 4)), dim3(256), 0, st, part, nch, K, n, G, db);

@@ -34,6 +34,7 @@ def _models(cfg, seed):
     ((256, 512, 8, 8, 16, 1024), 1, 1024),  # configs[3] at full depth and length, one of its 16 sequences
     ((200, 48, 3, 2, 5, 40), 3, 17),        # ragged: odd widths, dh 16, T not a multiple of 8
     ((256, 128, 4, 1, 4, 64), 3, 100),      # gate projection on the 16-column kernels with K = 128, 300 rows
+    ((256, 256, 8, 1, 4, 64), 1, 277),      # K = 256, 16 gate columns, last row block of 5 and row chunk of 21
     ((256, 256, 16, 1, 4, 64), 2, 20),      # 2H = 32 gate columns: the general GEMM
 ])
 def test_train_step_grads_match_oracle(cfg, batch, seq):
