@@ -119,13 +119,23 @@ __global__ __launch_bounds__(RT_NT) void route_count_k(const uint32_t* __restric
 
 // Pass 2 (one block, thread e = bucket): bucket offsets and, per block, where
 // its tokens of each bucket start; blkcnt is rewritten in place as the starts.
+constexpr int RT_U = 16;
 __global__ __launch_bounds__(RT_MAXB) void route_scan_k(int nblk, int E, int32_t* __restrict__ blkcnt,
                                                         int32_t* __restrict__ offsets) {
     __shared__ int wtot[RT_MAXB / 64];
     const int e = threadIdx.x, lane = e & 63, w = e >> 6;
+    // RT_U counts in flight (one after another each load was waited for, twice:
+    // 64 blocks of 16384 tokens 17.7 -> 6.7 us)
     int total = 0;
     if (e < E)
-        for (int b = 0; b < nblk; ++b) total += blkcnt[b * E + e];
+        for (int b = 0; b < nblk; b += RT_U) {
+            int c[RT_U];
+#pragma unroll
+            for (int u = 0; u < RT_U; ++u) c[u] = blkcnt[min(b + u, nblk - 1) * E + e];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < RT_U; ++u) total += b + u < nblk ? c[u] : 0;
+        }
     int incl = total;  // inclusive scan inside the wave
 #pragma unroll
     for (int s = 1; s < 64; s <<= 1) {
@@ -140,10 +150,17 @@ __global__ __launch_bounds__(RT_MAXB) void route_scan_k(int nblk, int E, int32_t
         offsets[e] = base;
         if (e == E - 1) offsets[E] = incl;
         int run = base;
-        for (int b = 0; b < nblk; ++b) {
-            const int c = blkcnt[b * E + e];
-            blkcnt[b * E + e] = run;
-            run += c;
+        for (int b = 0; b < nblk; b += RT_U) {
+            int c[RT_U];
+#pragma unroll
+            for (int u = 0; u < RT_U; ++u) c[u] = blkcnt[min(b + u, nblk - 1) * E + e];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < RT_U; ++u)
+                if (b + u < nblk) {
+                    blkcnt[(b + u) * E + e] = run;
+                    run += c[u];
+                }
         }
     }
 }
