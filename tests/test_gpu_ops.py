@@ -325,6 +325,25 @@ def test_rmsnorm_fwd_bwd(orc, g, rows, cols):
     assert orc.rel_err(g.rmsnorm_bwd(x, dy, 1e-6), orc.rmsnorm_bwd(x, dy)) <= GRAD_TOL
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 4), (7, 252), (64, 512), (5, 516), (9, 1024), (6, 1028)])
+def test_rmsnorm_rows_in_registers(orc, g, rows, cols):
+    """Rows held in registers (at most 512 and 1024 columns, multiples of 4) and the
+    first length past them, at scales whose squares differ by 40 binades."""
+    rng = np.random.default_rng(rows + cols)
+    x = (rng.standard_normal((rows, cols)) * 2.0 ** rng.integers(-10, 10, (rows, 1))).astype(np.float32)
+    dy = rng.standard_normal((rows, cols)).astype(np.float32)
+    y, inv = g.rmsnorm(x, 1e-6)
+    x64, d64 = x.astype(np.float64), dy.astype(np.float64)
+    i64 = 1.0 / np.sqrt((x64 * x64).mean(axis=1, keepdims=True) + 1e-6)
+    # a sum of squares of 16 partial sums and 6 lane steps, and 4 roundings after it
+    np.testing.assert_allclose(inv, i64[:, 0], rtol=16 * 2.0**-24)
+    np.testing.assert_allclose(y, x64 * i64, rtol=17 * 2.0**-24)
+    mean = (d64 * x64).mean(axis=1, keepdims=True) * i64
+    ref = i64 * (d64 - x64 * i64 * mean)
+    mag = i64 * (np.abs(d64) + np.abs(x64) * i64 * (np.abs(d64 * x64)).mean(axis=1, keepdims=True) * i64)
+    assert np.all(np.abs(g.rmsnorm_bwd(x, dy, 1e-6) - ref) <= 64 * 2.0**-24 * mag)
+
+
 @pytest.mark.parametrize("n,E", [(16384, 16), (1, 1), (1000, 64), (0, 16), (70001, 7), (256, 16)])
 def test_hash_route_bit_exact(orc, g, n, E):
     rng = np.random.default_rng(n + E)
