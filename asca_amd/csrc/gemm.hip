@@ -1737,8 +1737,8 @@ int skinny_wgrad_launch(const float* X, long ldx, const float* D, float* G, floa
 
 // Split-K decision of a plain product: split K when the output has too few
 // tiles to fill the chip, into as many K ranges as keep the grid within one
-// round of two blocks per CU (rounding up gave 512x1536x16384 eleven splits,
-// 528 blocks: a second round of 16; ten splits take it 315 -> 277 us).
+// round of two blocks per CU (rounding up would give 512x1536x16384 eleven
+// splits, 528 blocks: a second round of 16).
 // Returns the split count and the K range per split.
 static int gemm_splits(int M, int N, int K, long* kps_out) {
     const long tiles = (long)((M + GM_BM - 1) / GM_BM) * ((N + GM_BN - 1) / GM_BN);

@@ -865,9 +865,11 @@ int asca_model_create(int vocab, int d_model, int n_heads, int n_layers, int n_e
         P.b2 = add("moe.b2", 1, d);
         M->lay.push_back(P);
     }
-    // AdamW chunk table
+    // AdamW chunk table: 4096 elements are one unrolled pass of a block, and a small
+    // tensor still gives many blocks (256 x 512: 59 us in 8 chunks of 16384, 38 us in
+    // 32; a layer's 17.9M elements 140 -> 130 us, both beside the backward)
     std::vector<AdamChunk> ch;
-    const long CH = 16384;
+    const long CH = 4096;
     for (size_t j = 0; j < M->t.size(); ++j)
         for (long s = 0; s < (long)M->t[j].n; s += CH)
             ch.push_back({(int)j, 0, (long)M->t[j].off + s, std::min(CH, (long)M->t[j].n - s)});
