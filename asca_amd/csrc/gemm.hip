@@ -150,8 +150,16 @@ ASCA_DEV void frag_read(float (&f)[4][4], const float* t, int w0, int h, int lan
 // negated and negated back at the end, which makes every second row's error
 // positive.
 //
-// A value that is not finite, or rounds to infinity in bf16, leaves a
-// non-finite sum wherever it enters: a wave that finds one among its sums
+// The bf16 MFMA takes subnormal inputs as zero, and x1 and x2 lie up to 2^9 and
+// 2^17 below x: unscaled, operands below 2^-110 lost them (a product of rows at
+// 2^-120 had an error of 3.5e-5, at 2^-128 9e-3).  So both operands are split as
+// 2^24 x, where the smallest subnormal float is a normal bf16, and the sums are
+// scaled back by 2^-48: the same bits where nothing under- or overflows.  The
+// odd rows' sign is part of the factor.  The multiplications cost 1 to 2%
+// (16384x512x1536 forward and backward 418 -> 426 us, training step 14.00 -> 14.15 ms).
+//
+// A value that is not finite, or is 2^104 or more, or a sum of 2^80 or more
+// leaves a non-finite sum wherever it enters: a wave that finds one among its sums
 // computes its tile again with f32 products (split_redo), so infinities and
 // NaN come out as the f32 products give them.
 //
@@ -208,8 +216,9 @@ ASCA_DEV void split2(float a, float b, unsigned& w0, unsigned& w1, unsigned& w2)
     w2 = pk_bf16(a, b);
 }
 
-// x, negated where `odd` is not zero (a power of two)
-ASCA_DEV float neg_if(float x, int odd) { return odd ? -x : x; }
+constexpr float SP_SCALE = 0x1p24f, SP_UNSCALE = 0x1p-48f;
+// the factor of an operand's values: SP_SCALE, negative where `odd` is not zero
+ASCA_DEV float sp_factor(int odd) { return odd ? -SP_SCALE : SP_SCALE; }
 
 // A thread's share of one operand tile (R rows x 32 k on NT threads).
 //   KC (k-contiguous, stored [mn][k]): items of 8 consecutive k of one row,
@@ -220,7 +229,7 @@ ASCA_DEV float neg_if(float x, int odd) { return odd ? -x : x; }
 //     consecutive columns in one lane.
 // Rows past the operand's extent repeat a valid one (KC) or read as 0 (MC);
 // k past the range read as 0.
-// NEG: odd rows are stored negated.
+// Stored as SP_SCALE x; NEG: odd rows negated.
 template <bool KC, bool GATHER, bool NEG, int R, int NT>
 struct SplitTile {
     static constexpr int NI = KC ? R * 4 / NT : 1, W = R * 8 / NT, NF = R * 32 / NT;
@@ -324,7 +333,7 @@ struct SplitTile {
                 static_assert(NT % 8 == 0, "a thread's rows share their parity");
                 float y[8];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) y[e] = NEG ? neg_if(x[8 * j + e], tid & 4) : x[8 * j + e];
+                for (int e = 0; e < 8; ++e) y[e] = sp_factor(NEG ? tid & 4 : 0) * x[8 * j + e];
                 uint4 w0, w1, w2;
                 split2(y[0], y[1], w0.x, w1.x, w2.x);
                 split2(y[2], y[3], w0.y, w1.y, w2.y);
@@ -339,7 +348,7 @@ struct SplitTile {
 #pragma unroll
             for (int c = 0; c < W; ++c) {
                 const int o = (W == 4 ? c : (col & 2) + c) * 256;
-                constexpr float sg[2] = {1.0f, NEG ? -1.0f : 1.0f};
+                constexpr float sg[2] = {SP_SCALE, NEG ? -SP_SCALE : SP_SCALE};
                 const float f = sg[c & 1];
                 uint2 w0, w1, w2;
                 split2(f * x[c], f * x[W + c], w0.x, w1.x, w2.x);
@@ -416,8 +425,9 @@ ASCA_DEV void split_redo(f32x4 (&acc)[NX][NY], int x0, int y0, const float* A, c
     }
 }
 
-// The sums of the rows that were multiplied negated (odd rows of the tile:
-// row 16 x + 4 (lane / 16) + r, or 4 i + x of an mn-contiguous A), negated back.
+// The sums scaled back, those of the rows that were multiplied negated (odd rows
+// of the tile: row 16 x + 4 (lane / 16) + r, or 4 i + x of an mn-contiguous A)
+// negated back.
 template <bool TA, int NX, int NY>
 ASCA_DEV void split_sign(f32x4 (&acc)[NX][NY], int x0) {
 #pragma unroll
@@ -425,7 +435,7 @@ ASCA_DEV void split_sign(f32x4 (&acc)[NX][NY], int x0) {
 #pragma unroll
         for (int y = 0; y < NY; ++y)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[x][y][r] = neg_if(acc[x][y][r], (TA ? x0 + x : r) & 1);
+            for (int r = 0; r < 4; ++r) acc[x][y][r] *= (TA ? x0 + x : r) & 1 ? -SP_UNSCALE : SP_UNSCALE;
 }
 
 // Any infinity or NaN among a wave's sums?
@@ -852,17 +862,16 @@ struct FragTile {
         }
     }
     // the three bf16 fragments of 16-row tile j
-    ASCA_DEV void frag(int j, bf16x8 (&f)[3]) const {
+    ASCA_DEV void frag(int j, bf16x8 (&out)[3]) const {
         typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
         u32x4 w[3];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             float a = KC ? x[2 * j + e / 2][2 * (e & 1)] : x[2 * e][j];
             float b = KC ? x[2 * j + e / 2][2 * (e & 1) + 1] : x[2 * e + 1][j];
-            if constexpr (NEG) {
-                a = neg_if(a, KC ? col & NTL : j & 1);  // col / NTL = lane % 16: the KC lane's row
-                b = neg_if(b, KC ? col & NTL : j & 1);
-            }
+            const float f = sp_factor(!NEG ? 0 : KC ? col & NTL : j & 1);  // col / NTL = lane % 16: the KC lane's row
+            a *= f;
+            b *= f;
             unsigned w0, w1, w2;
             split2(a, b, w0, w1, w2);
             w[0][e] = w0;
@@ -870,7 +879,7 @@ struct FragTile {
             w[2][e] = w2;
         }
 #pragma unroll
-        for (int s = 0; s < 3; ++s) f[s] = __builtin_bit_cast(bf16x8, w[s]);
+        for (int s = 0; s < 3; ++s) out[s] = __builtin_bit_cast(bf16x8, w[s]);
     }
 };
 

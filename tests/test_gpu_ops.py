@@ -99,6 +99,21 @@ def test_gemm_non_finite(g, M, N, K):
     assert np.all(np.abs(got[ok] - ref[ok]) <= (6 * ((K + 31) // 32) + 16) * 2.0**-23 * mag[ok])
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1)])
+@pytest.mark.parametrize("sa,sb", [(-112, 60), (-125, 60), (60, -125), (-140, 110), (50, 40)])
+@pytest.mark.parametrize("M,N,K", [(16, 64, 64), (200, 300, 72), (4096, 256, 64), (4096, 4096, 32)])
+def test_gemm_range(g, M, N, K, sa, sb, ta, tb):
+    """Operands at the ends of the float range (subnormal among them) keep all of
+    their bits: the bound of test_gemm_rounding, and a result's own rounding."""
+    rng = np.random.default_rng(M + N + K)
+    a = np.ldexp(rng.standard_normal((M, K)).astype(np.float32), sa).astype(np.float32)
+    b = np.ldexp(rng.standard_normal((K, N)).astype(np.float32), sb).astype(np.float32)
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    mag = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    got = g.gemm(np.ascontiguousarray(a.T) if ta else a, np.ascontiguousarray(b.T) if tb else b, bool(ta), bool(tb))
+    assert np.all(np.abs(got.astype(np.float64) - ref) <= (6 * ((K + 31) // 32) + 16) * 2.0**-23 * mag + 2.0**-149)
+
+
 @pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
 @pytest.mark.parametrize("M,N,K", [(128, 128, 32), (1, 1, 1), (300, 257, 77), (64, 1536, 512),
                                    (513, 16, 512), (130, 200, 4096), (7, 9, 0),
