@@ -37,6 +37,8 @@
 // delta_ut64_b.hip and delta_utn.hip (the other variants and head widths,
 // compiled with the default one).
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 #include "delta.h"
 #include "runtime.h"
@@ -62,6 +64,9 @@ struct Dim {
     static constexpr int NR = NR_, NV = NV_, NH = NH_;
     static constexpr int KS = NR / NH, VS = NR / NV;
     static_assert(NR % NV == 0, "tile split");
+    // whether a non-finite value is kept to the steps that the recurrence takes it
+    // to (any_bad below); the dh = 64 kernels spread it over its block of 16 steps
+    static constexpr bool CAUSAL = NR != 4;
     static constexpr int DH = 16 * NR, DH2 = DH * DH;
     static constexpr int NWT = NV + NH, NT = 64 * NWT;   // waves, threads of a block
     // row pitches in LDS (4 mod 32 at 64 columns: the 16-byte reads of 16 rows
@@ -93,8 +98,22 @@ ASCA_DEV float acc_sum(const f32x4 (&a)[N], int i) {
     else if constexpr (N == 3) return (a[0][i] + a[1][i]) + a[2][i];
     else return (a[0][i] + a[1][i]) + (a[2][i] + a[3][i]);
 }
+// Non-finite values.  The triangular products of a block (T R, M U, M^T dO, T^T dU,
+// (Gamma o dM) K, ...) multiply masked zeros with every row of the block, and zero
+// times an infinity or NaN is NaN: one at step t would reach outputs and gradients
+// of the block's other steps that do not depend on it.  So where such a product's
+// sum is not finite (rare: one check per block), it is formed again with only the
+// terms that belong to it, at the end of the step (a branch inside one holds up what
+// the scheduler would move past it).  The checks cost B4 T128 H4 dh32 31.6 -> 32.5
+// us, B8 T1000 H8 dh128 528 -> 531 us.
+ASCA_DEV bool any_bad(float x) { return __builtin_expect(__any(!__builtin_isfinite(x)), 0); }
 ASCA_DEV float readlane_f(float x, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l)); }
 ASCA_DEV float el(const float4& v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
+
+// Orders the wave's own LDS writes before its reads of other lanes' values.  The
+// LDS executes one wave's instructions in issue order, so only the compiler has
+// to keep them in program order: a compiler barrier, no wait.
+ASCA_DEV void wave_sync() { asm volatile("" ::: "memory"); }
 
 // Rows of q, k, v, dO are f32 or (BF) bf16, widened exactly.  Four consecutive
 // elements as loaded, and widened:
@@ -148,6 +167,7 @@ constexpr int P_M = 256;    // M = tril(Gamma o Q K^T), row-major [16][16]
 constexpr int P_GAM = 512;  // gamma_t
 constexpr int P_BET = 528;  // beta_t (0 past the sequence end)
 constexpr int P_GC = 544;   // Gamma[15][m] = prod_{m<s<=15} alpha_s
+constexpr int P_AL = 560;   // alpha_t (1 past the sequence end)
 constexpr int P_SZ = 576;
 
 // Buffer resources over the unit's part of every array the forward reads or
@@ -221,6 +241,7 @@ ASCA_DEV void prep_compute(const PrepIn<D>& pi, int p, int T, float* __restrict_
         ps[P_GAM + n] = gam;
         ps[P_BET + n] = b;
         ps[P_GC + n] = pr;
+        if constexpr (D::CAUSAL) ps[P_AL + n] = a;
     }
     buf_store1(rrec, 4u * (R_V + lane), g == 0 ? gam : g == 1 ? b * gam : g == 2 ? pr : b, srec);
     const float4 bt = *reinterpret_cast<const float4*>(ps + P_BET + 4 * g);
@@ -257,22 +278,47 @@ ASCA_DEV void prep_compute(const PrepIn<D>& pi, int p, int T, float* __restrict_
         for (int j = 0; j < m; ++j) x[j] -= x[m] * el(rw[(m + 1) & 1][j >> 2], j & 3);
         __builtin_amdgcn_sched_barrier(0);   // keep the solve's steps in order (bounds the live registers)
     }
-    if (g == 0) {
+    // T row-major for the forward, then in the accumulator layout for the record
+    auto put_t = [&] {
+        if (g == 0) {
 #pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4)
-            *reinterpret_cast<float4*>(ps + P_T + n * 16 + 4 * q4) =
-                make_float4(x[4 * q4], x[4 * q4 + 1], x[4 * q4 + 2], x[4 * q4 + 3]);
-    }
+            for (int q4 = 0; q4 < 4; ++q4)
+                *reinterpret_cast<float4*>(ps + P_T + n * 16 + 4 * q4) =
+                    make_float4(x[4 * q4], x[4 * q4 + 1], x[4 * q4 + 2], x[4 * q4 + 3]);
+        }
+    };
+    auto record_t = [&] {
+        const float* tp = ps + P_T + 64 * g + n;
+        buf_store4(rrec, 16u * ((R_T >> 2) + lane), make_float4(tp[0], tp[16], tp[32], tp[48]), srec);
+    };
+    put_t();
     buf_store4(rrec, 16u * ((R_A >> 2) + lane), make_float4(A[0], A[1], A[2], A[3]), srec);
     buf_store4(rrec, 16u * ((R_BQ >> 2) + lane), make_float4(Bq[0], Bq[1], Bq[2], Bq[3]), srec);
-    const float* tp = ps + P_T + 64 * g + n;
-    buf_store4(rrec, 16u * ((R_T >> 2) + lane), make_float4(tp[0], tp[16], tp[32], tp[48]), srec);
+    record_t();
     const float* mp = ps + P_M + 64 * g + n;
     buf_store4(rrec, 16u * ((R_M >> 2) + lane), make_float4(mp[0], mp[16], mp[32], mp[48]), srec);
     buf_store4(rrec, 16u * ((R_G >> 2) + lane),
                make_float4(n <= 4 * g ? G[0] : 0.f, n <= 4 * g + 1 ? G[1] : 0.f, n <= 4 * g + 2 ? G[2] : 0.f,
                            n <= 4 * g + 3 ? G[3] : 0.f),
                srec);
+    if constexpr (D::CAUSAL) {
+        if (any_bad((Lv[0] + Lv[1]) + (Lv[2] + Lv[3]))) {  // row n of T from the rows of L up to n
+#pragma unroll
+            for (int j = 0; j < C; ++j) x[j] = n == j ? 1.f : 0.f;
+#pragma unroll
+            for (int m = C - 1; m >= 1; --m) {
+#pragma unroll
+                for (int j = 0; j < m; ++j) {
+                    const float y = x[j] - x[m] * scr[m * 16 + j];
+                    x[j] = m <= n ? y : x[j];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            put_t();
+            wave_sync();
+            record_t();
+        }
+    }
 }
 
 // Staging of a group's k, q, v rows in LDS: NH blocks x 16 rows, two buffers
@@ -345,13 +391,83 @@ ASCA_DEV void ck_store(const FRes& R, int slot, const f32x4 (&S)[D::NR], float* 
     }
 }
 
+// A block's o and u rows leave as 16-byte stores: the 16 x 16 tiles go through the
+// wave's LDS scratch `ot` (lane: row lane / 4, columns 4 (lane % 4) .. +3).
+template <class D, bool FULL, bool AL>
+ASCA_DEV void store_ou(const f32x4& O, const f32x4& U, float* __restrict__ ot, int c, float* __restrict__ o,
+                       const FRes& res, long ubase, long d, int T, int vt, int lane) {
+    const int n = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        ot[(4 * g + i) * OTP + n] = O[i];
+        ot[C * OTP + (4 * g + i) * OTP + n] = U[i];
+    }
+    const int rr = lane >> 2, cc = 4 * (lane & 3);
+    const float4 o4 = *reinterpret_cast<const float4*>(ot + rr * OTP + cc);
+    const float4 u4 = *reinterpret_cast<const float4*>(ot + C * OTP + rr * OTP + cc);
+    if constexpr (AL) {
+        // rows past the sequence end fall outside the resource: dropped
+        buf_store4(res.o, 4u * (unsigned)(rr * d + 16 * vt + cc), o4, 4u * (unsigned)(c * C * d));
+    } else {
+        const long t = (long)c * C + rr;
+        if (FULL || t < T) {
+            float* po = o + ubase + t * d + 16 * vt + cc;
+            po[0] = o4.x; po[1] = o4.y; po[2] = o4.z; po[3] = o4.w;
+        }
+    }
+    // u tile: 1 KB contiguous per wave and block (layout at U_TILE)
+    buf_store4(res.u, 4u * (unsigned)(vt * 256 + rr * 16 + cc), u4, 4u * (unsigned)(c * D::U_BLK));
+}
+
+// The `nt` steps of a block one after another (see any_bad): S advanced in place,
+// the o and u rows in the accumulator layout.  Per step the lane's keys of S^T k and
+// S^T q, added over the four lanes of column n.
+template <class D>
+ASCA_DEV void chain_by_steps(f32x4 (&S)[D::NR], f32x4& O, f32x4& U, const float* __restrict__ kb,
+                             const float* __restrict__ qb, const float* __restrict__ vb,
+                             const float* __restrict__ ps, int nt, int w, int lane) {
+    const int n = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) O[i] = U[i] = 0.0f;
+#pragma unroll 1
+    for (int t = 0; t < nt; ++t) {
+        const float a = ps[P_AL + t], b = ps[P_BET + t];
+        float4 kr[D::NR];
+        float sk = 0.0f, o = 0.0f;
+#pragma unroll
+        for (int r = 0; r < D::NR; ++r) {
+            kr[r] = *reinterpret_cast<const float4*>(kb + t * D::RK + 16 * r + 4 * g);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sk = fmaf(el(kr[r], i), S[r][i], sk);
+        }
+        sk = add_xor32(add_xor16(sk));
+        const float u = b * (vb[t * D::RV + 16 * w + n] - a * sk);
+#pragma unroll
+        for (int r = 0; r < D::NR; ++r) {
+            const float4 qr = *reinterpret_cast<const float4*>(qb + t * D::RK + 16 * r + 4 * g);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                S[r][i] = fmaf(el(kr[r], i), u, a * S[r][i]);
+                o = fmaf(el(qr, i), S[r][i], o);
+            }
+        }
+        o = add_xor32(add_xor16(o));
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (t == 4 * g + i) {
+                O[i] = o;
+                U[i] = u;
+            }
+    }
+}
+
 // One block of 16 steps for the wave's dh x 16 slab of S (value tile vt, the
 // block's w-th): outputs o, the u rows
 // (for the backward), the checkpoint (state before the block, even blocks) and the block
 // update.  `kb` points at the block's first staged k row
 // (q and v rows follow at qb, vb).
 template <class D, bool FULL, bool AL>
-ASCA_DEV void chain_step(f32x4 (&S)[D::NR], const float* __restrict__ kb, const float* __restrict__ qb,
+ASCA_DEV float chain_step(f32x4 (&S)[D::NR], const float* __restrict__ kb, const float* __restrict__ qb,
                          const float* __restrict__ vb, const float* __restrict__ ps,
                          float* __restrict__ ot, int c, float* __restrict__ o, const FRes& res, bool ckw, long ubase,
                          long d, int T, int w, int vt, int lane) {
@@ -410,30 +526,7 @@ ASCA_DEV void chain_step(f32x4 (&S)[D::NR], const float* __restrict__ kb, const 
 #pragma unroll
     for (int i = 0; i < 4; ++i) O = mfma4(el(mr, i), U[i], O);
     if (ckw) ck_store<D>(res, c >> 1, S, ot + 2 * C * OTP, vt, lane);
-    // o and u rows leave as 16-byte stores: the 16 x 16 tiles go through the
-    // wave's LDS scratch (lane: row lane / 4, columns 4 (lane % 4) .. +3)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        ot[(4 * g + i) * OTP + n] = O[i];
-        ot[C * OTP + (4 * g + i) * OTP + n] = U[i];
-    }
-    {
-        const int rr = lane >> 2, cc = 4 * (lane & 3);
-        const float4 o4 = *reinterpret_cast<const float4*>(ot + rr * OTP + cc);
-        const float4 u4 = *reinterpret_cast<const float4*>(ot + C * OTP + rr * OTP + cc);
-        if constexpr (AL) {
-            // rows past the sequence end fall outside the resource: dropped
-            buf_store4(res.o, 4u * (unsigned)(rr * d + 16 * vt + cc), o4, 4u * (unsigned)(c * C * d));
-        } else {
-            const long t = (long)c * C + rr;
-            if (FULL || t < T) {
-                float* po = o + ubase + t * d + 16 * vt + cc;
-                po[0] = o4.x; po[1] = o4.y; po[2] = o4.z; po[3] = o4.w;
-            }
-        }
-        // u tile: 1 KB contiguous per wave and block (layout at U_TILE)
-        buf_store4(res.u, 4u * (unsigned)(vt * 256 + rr * 16 + cc), u4, 4u * (unsigned)(c * D::U_BLK));
-    }
+    store_ou<D, FULL, AL>(O, U, ot, c, o, res, ubase, d, T, vt, lane);
     float Ut[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) Ut[i] = el(gc, i) * U[i];
@@ -443,6 +536,7 @@ ASCA_DEV void chain_step(f32x4 (&S)[D::NR], const float* __restrict__ kb, const 
 #pragma unroll
         for (int i = 0; i < 4; ++i) S[r] = mfma4(kt[r][i], Ut[i], S[r]);
     }
+    return O[0];  // (a U that is not finite is in every row of M U)
 }
 
 // A helper wave's gate loads: lane l holds alpha, beta of step 16 c + (l % 16).
@@ -549,17 +643,43 @@ __global__ __launch_bounds__(D::NT) void ut_fwd_k(const void* __restrict__ q, co
     const int NCF = T / C;
     for (int c0 = 0; c0 < NC; c0 += NH) {
         const float* buf = lds + D::F_STG + ((c0 / NH) & 1) * D::S_BUF;
+        f32x4 S0[D::CAUSAL ? D::NR : 1];  // the state before the group
+        if constexpr (D::CAUSAL)
+#pragma unroll
+            for (int r = 0; r < D::NR; ++r) S0[r] = S[r];
+        float bad = 0.0f;  // NaN once a block of the group has sums that are not finite
         if (c0 + NH <= NCF) {
 #pragma unroll
-            for (int j = 0; j < NH; ++j)
-                chain_step<D, true, AL>(S, buf + j * C * D::RK, buf + D::S_Q + j * C * D::RK,
-                                        buf + D::S_V + j * C * D::RV, lds + ((c0 + j) % D::NSLOT) * P_SZ, ot, c0 + j,
-                                        o, R, ((NH % 2 ? c0 + j : j) & 1) == 0, ubase, d, T, w, vt, lane);
+            for (int j = 0; j < NH; ++j) {
+                const float o0 = chain_step<D, true, AL>(
+                    S, buf + j * C * D::RK, buf + D::S_Q + j * C * D::RK, buf + D::S_V + j * C * D::RV,
+                    lds + ((c0 + j) % D::NSLOT) * P_SZ, ot, c0 + j, o, R, ((NH % 2 ? c0 + j : j) & 1) == 0, ubase, d,
+                    T, w, vt, lane);
+                if constexpr (D::CAUSAL) bad = fmaf(o0, 0.0f, bad);
+            }
         } else {
-            for (int j = 0; j < NH && c0 + j < NC; ++j)
-                chain_step<D, false, AL>(S, buf + j * C * D::RK, buf + D::S_Q + j * C * D::RK,
-                                         buf + D::S_V + j * C * D::RV, lds + ((c0 + j) % D::NSLOT) * P_SZ, ot,
-                                         c0 + j, o, R, ((c0 + j) & 1) == 0, ubase, d, T, w, vt, lane);
+            for (int j = 0; j < NH && c0 + j < NC; ++j) {
+                const float o0 = chain_step<D, false, AL>(
+                    S, buf + j * C * D::RK, buf + D::S_Q + j * C * D::RK, buf + D::S_V + j * C * D::RV,
+                    lds + ((c0 + j) % D::NSLOT) * P_SZ, ot, c0 + j, o, R, ((c0 + j) & 1) == 0, ubase, d, T, w, vt, lane);
+                if constexpr (D::CAUSAL) bad = fmaf(o0, 0.0f, bad);
+            }
+        }
+        if constexpr (D::CAUSAL) {
+            if (any_bad(bad)) {
+#pragma unroll
+                for (int r = 0; r < D::NR; ++r) S[r] = S0[r];
+#pragma unroll 1
+                for (int j = 0; j < NH && c0 + j < NC; ++j) {
+                    const int c = c0 + j;
+                    if ((c & 1) == 0) ck_store<D>(R, c >> 1, S, ot + 2 * C * OTP, vt, lane);
+                    f32x4 O, U;
+                    chain_by_steps<D>(S, O, U, buf + j * C * D::RK, buf + D::S_Q + j * C * D::RK,
+                                      buf + D::S_V + j * C * D::RV, lds + (c % D::NSLOT) * P_SZ, min(C, T - c * C), w,
+                                      lane);
+                    store_ou<D, false, AL>(O, U, ot, c, o, R, ubase, d, T, vt, lane);
+                }
+            }
         }
         lds_barrier();
     }
@@ -631,11 +751,6 @@ struct BL {
     static constexpr size_t B_LDS = (size_t)B_END * 4;
     static_assert(B_LDS <= 160 * 1024 && B_HO % 4 == 0 && B_EP % 4 == 0 && B_SCR % 4 == 0, "backward LDS");
 };
-
-// Orders the wave's own LDS writes before its reads of other lanes' values.  The
-// LDS executes one wave's instructions in issue order, so only the compiler has
-// to keep them in program order: a compiler barrier, no wait.
-ASCA_DEV void wave_sync() { asm volatile("" ::: "memory"); }
 
 // 16x16 tile in the accumulator layout (lane (g, n) holds X[4g + j][n]) ->
 // lane (g, n) receives X[n][4g .. 4g + 3].
@@ -769,8 +884,10 @@ ASCA_DEV void bchain_load(BChainIn<BF>& ci, int c, const BArgs& A, const BRes& R
     ci.bn = buf_load1(R.rec, 4u * (RV_BET + n), sb);
 }
 
-template <class D, bool BF, bool AL>
-ASCA_DEV void bchain_step(f32x4 (&X)[D::NR], const BChainIn<BF>& ci, const float* __restrict__ sb,
+// Returns Y[0], not finite where a dU or dO is not (they are in every row of T^T dU).
+// MASKED: dU[m] and Y[m] from the steps t >= m alone (see any_bad).
+template <class D, bool BF, bool AL, bool MASKED = false>
+ASCA_DEV float bchain_step(f32x4 (&X)[D::NR], const BChainIn<BF>& ci, const float* __restrict__ sb,
                           float* __restrict__ ho, float* __restrict__ scr, int c, const BArgs& A, int w, int vt,
                           int lane) {
     using L = BL<D>;
@@ -800,11 +917,38 @@ ASCA_DEV void bchain_step(f32x4 (&X)[D::NR], const BChainIn<BF>& ci, const float
     f32x4 dU;
 #pragma unroll
     for (int j = 0; j < 4; ++j) dU[j] = el(gc, j) * acc_sum(kx, j);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) dU = mfma4(el(ci.mr, j), dO[j], dU);
     f32x4 Y = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (!MASKED) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) Y = mfma4(el(ci.tr, j), dU[j], Y);
+        for (int j = 0; j < 4; ++j) dU = mfma4(el(ci.mr, j), dO[j], dU);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) Y = mfma4(el(ci.tr, j), dU[j], Y);
+    } else {
+        // M[t][m], T[t][m] at 4 (16 (t / 4) + m) + t % 4 of their record tiles
+        const float* rec = A.rec + (unsigned)(c * R_SZ);
+#pragma unroll 1
+        for (int t = 0; t < C; ++t) {
+            const float x = sb[L::SB_DO + t * D::RV + 16 * w + n];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float y = fmaf(rec[R_M + 4 * (16 * (t >> 2) + 4 * g + j) + (t & 3)], x, dU[j]);
+                dU[j] = t >= 4 * g + j ? y : dU[j];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) scr[(4 * g + j) * OTP + n] = dU[j];
+        wave_sync();
+#pragma unroll 1
+        for (int t = 0; t < C; ++t) {
+            const float x = scr[t * OTP + n];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float y = fmaf(rec[R_T + 4 * (16 * (t >> 2) + 4 * g + j) + (t & 3)], x, Y[j]);
+                Y[j] = t >= 4 * g + j ? y : Y[j];
+            }
+        }
+        wave_sync();
+    }
     // hand X (the gradient after this block) and Y over to the helpers
 #pragma unroll
     for (int r = 0; r < NR; ++r)
@@ -845,6 +989,25 @@ ASCA_DEV void bchain_step(f32x4 (&X)[D::NR], const BChainIn<BF>& ci, const float
             X[r] = mfma4(kv, Yb[j], X[r]);
         }
     }
+    return Y[0];
+}
+
+// The step of block c again, with the masked products.
+template <class D, bool BF, bool AL>
+ASCA_DEV void bchain_again(f32x4 (&X)[D::NR], const float* __restrict__ sb, float* __restrict__ ho,
+                           float* __restrict__ scr, int c, const BArgs& A, const BRes& R, int w, int vt, int lane) {
+    using L = BL<D>;
+    const int n = lane & 15, g = lane >> 4;
+    BChainIn<BF> ci;
+    bchain_load<BF, AL>(ci, c, A, R, vt, lane);
+    // X before its update, from the tiles handed over
+#pragma unroll
+    for (int r = 0; r < D::NR; ++r)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            X[r][j] = ho[L::HO_DS + ((r * D::NV + w) * 64 + 16 * (n >> 2) + 4 * g + j) * 4 + (n & 3)];
+    wave_sync();
+    bchain_step<D, BF, AL, true>(X, ci, sb, ho, scr, c, A, w, vt, lane);
 }
 
 template <class D>
@@ -905,8 +1068,10 @@ struct BCarry {
 // 16kt + 4g + r, so the per-step gate factors are the lane's own, the row sums
 // over keys are in-register sums plus two lane swaps, and dq, dk leave without a
 // transpose.
-template <class D>
-ASCA_DEV void bhelp_products(BCarry<D>& cy, const BHelpIn<D>& hi, const float* __restrict__ sb,
+// Returns a value that is not finite where a dq or dk of the lane is not.
+// MASKED: dq and dk from the terms of their own steps alone (see any_bad).
+template <class D, bool MASKED = false>
+ASCA_DEV float bhelp_products(BCarry<D>& cy, const BHelpIn<D>& hi, const float* __restrict__ sb,
                              const float* __restrict__ sbp, const float* __restrict__ ho, float* __restrict__ ep,
                              float* __restrict__ scr, int c, const BArgs& A, int hw, int lane) {
     using L = BL<D>;
@@ -1004,11 +1169,27 @@ ASCA_DEV void bhelp_products(BCarry<D>& cy, const BHelpIn<D>& hi, const float* _
             dq[j] = gam * F[s][j];
             dk[j] = gcn * Dx[s][j] - bt * gam * Zt[s][j];
         }
+        if constexpr (!MASKED) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            dq = mfma4(kb[j], el(gdmt, j), dq);
-            dk = mfma4(qb[j], GdM[j], dk);
-            dk = mfma4(kb[j], dA[j] + el(dat, j), dk);
+            for (int j = 0; j < 4; ++j) {
+                dq = mfma4(kb[j], el(gdmt, j), dq);
+                dk = mfma4(qb[j], GdM[j], dk);
+                dk = mfma4(kb[j], dA[j] + el(dat, j), dk);
+            }
+        } else {  // (Gamma o dM and dA are in scr)
+#pragma unroll 1
+            for (int m = 0; m < C; ++m) {
+                const float4 km = *reinterpret_cast<const float4*>(sb + L::SB_K + m * RK + k0 + 4 * g);
+                const float4 qm = *reinterpret_cast<const float4*>(sb + L::SB_Q + m * RK + k0 + 4 * g);
+                const float gnm = scr[n * OTP + m], gmn = scr[m * OTP + n];
+                const float a = scr[(C + max(m, n)) * OTP + min(m, n)];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (m <= n) dq[j] = fmaf(el(km, j), gnm, dq[j]);
+                    if (m >= n) dk[j] = fmaf(el(qm, j), gmn, dk[j]);
+                    if (m != n) dk[j] = fmaf(el(km, j), a, dk[j]);
+                }
+            }
         }
         // row sums over the helper's keys: in-register, then over the four lanes of
         // row n (lane bits 4 and 5)
@@ -1026,6 +1207,7 @@ ASCA_DEV void bhelp_products(BCarry<D>& cy, const BHelpIn<D>& hi, const float* _
         cy.qr[s] = qr;
         cy.kr[s] = kr;
     }
+    const float qkb = rs[EP_RQ] + rs[EP_RK];
 #pragma unroll
     for (int e = 0; e < 5; ++e) rs[e] = add_xor32(add_xor16(rs[e]));
     float* gs = A.gsc + (unsigned)(c * GS_SZ);
@@ -1049,6 +1231,7 @@ ASCA_DEV void bhelp_products(BCarry<D>& cy, const BHelpIn<D>& hi, const float* _
     }
     cy.rq = __builtin_amdgcn_rcpf(hi.qn);
     cy.rk = __builtin_amdgcn_rcpf(hi.kn);
+    return qkb;
 }
 
 template <class D, bool FUSED, bool AL>
@@ -1131,7 +1314,7 @@ ASCA_DEV void bgate_load(BGateIn<NH>& gi, int c, const BArgs& A, int lane) {
 // interleave and the LDS transposes share their wave syncs.  scr holds NB
 // areas of WSCR floats.  Blocks past the sequence end (clamped loads) store
 // nothing: their rows lie outside the resources' range.
-template <bool FUSED, int NH, int NB>
+template <bool FUSED, bool CAUSAL, int NH, int NB>
 ASCA_DEV void bgate_batch(const BGateIn<NH> (&gin)[NB], const int (&cs)[NB], float* __restrict__ scr,
                           const BArgs& A, Rsrc rga, Rsrc rgb, int lane) {
     const int n = lane & 15, g = lane >> 4;
@@ -1207,6 +1390,25 @@ ASCA_DEV void bgate_batch(const BGateIn<NH> (&gin)[NB], const int (&cs)[NB], flo
         t2 = add_xor32(add_xor16(t2));
         const float gprev = dpp_or<0x111>(1.0f, gin[i].gam);   // gamma_{n-1}
         dal[i] = gprev * t1[i] + t2;
+        if constexpr (CAUSAL) {
+            if (any_bad(dal[i])) {  // dalpha of step n from the rows t >= n and columns before n
+                float s1 = 0.0f, s2 = 0.0f;
+#pragma unroll 1
+                for (int t = 0; t < C; ++t) {
+                    const float G = st[C * OTP + t * OTP + n];
+                    float r = 0.0f;
+#pragma unroll 1
+                    for (int m = 0; m < C - 1; ++m) {
+                        const float x = fmaf(st[t * OTP + m], st[C * OTP + max(n - 1, 0) * OTP + m], r);
+                        r = m < n ? x : r;
+                    }
+                    const float x1 = fmaf(G, st[SVO + t], s1), x2 = fmaf(G, r, s2);
+                    s1 = t >= n ? x1 : s1;
+                    s2 = t >= n ? x2 : s2;
+                }
+                dal[i] = fmaf(gprev, s1, s2);
+            }
+        }
         // dbeta of step n: Y.V - gamma Z'.K + sum_l dL Gamma A (row n's sum from lane (n/4, .))
         const float rbn = st[SVO + 64 + n];
         dbe[i] = gin[i].yv - gin[i].gam * szk[i] + rbn;
@@ -1312,7 +1514,7 @@ ASCA_DEV void bgate_tail(const BArgs& A, float* __restrict__ lds, int w, int lan
             cs[i] = c0 + D::NWT * i;                // past NC: rows beyond T, stores dropped
             bgate_load<FUSED>(gin[i], min(cs[i], A.NC - 1), A, lane);
         }
-        bgate_batch<FUSED, D::NH, NB>(gin, cs, scr, A, rga, rgb, lane);
+        bgate_batch<FUSED, D::CAUSAL, D::NH, NB>(gin, cs, scr, A, rga, rgb, lane);
     }
 }
 
@@ -1376,11 +1578,20 @@ __global__ __launch_bounds__(D::NT) void ut_bwd_k(BArgs A) {
             const int cp = NC - s;
             if (s >= 2)
                 bhelp_epilogue<D, FUSED, AL>(cy, lds + L::B_EP + ((cp + 1) & 1) * L::EP_SZ, cp + 1, A, hw, lane);
-            bhelp_products<D>(cy, hb, lds + L::B_STG + (cp % NSB) * L::SB_BUF,
-                              lds + L::B_STG + ((cp + NSB - 1) % NSB) * L::SB_BUF,
-                              lds + L::B_HO + (cp & 1) * L::HO_SZ, lds + L::B_EP + (cp & 1) * L::EP_SZ, scr, cp, A,
-                              hw, lane);
+            auto products = [&](const BHelpIn<D>& in, auto Masked) {
+                return bhelp_products<D, decltype(Masked)::value>(
+                    cy, in, lds + L::B_STG + (cp % NSB) * L::SB_BUF, lds + L::B_STG + ((cp + NSB - 1) % NSB) * L::SB_BUF,
+                    lds + L::B_HO + (cp & 1) * L::HO_SZ, lds + L::B_EP + (cp & 1) * L::EP_SZ, scr, cp, A, hw, lane);
+            };
+            const float qk = products(hb, std::false_type{});
             bhelp_load<D, FUSED>(hb, max(cp - 2, 0), A, R, hw, lane);
+            if constexpr (D::CAUSAL) {
+                if (any_bad(qk)) {
+                    BHelpIn<D> h2;
+                    bhelp_load<D, FUSED>(h2, cp, A, R, hw, lane);
+                    products(h2, std::true_type{});
+                }
+            }
             lds_barrier();
         };
         for (int s = 1; s <= NC; s += 2) {
@@ -1409,25 +1620,30 @@ __global__ __launch_bounds__(D::NT) void ut_bwd_k(BArgs A) {
     lds_barrier();
     for (int s = 0; s < NC; ++s) {
         const int c = NC - 1 - s;
+        float y0;
         // the chain's inputs are loaded two steps ahead into buffer s & 1
         // (static indices: no register copies; X is updated on every path)
         if ((s & 1) == 0) {
             // block c - 1 < NC - 1 is whole (only the last block can be partial)
             if (c >= 1)
                 bstage_store<true>(sg[0], c - 1, lds + L::B_STG + ((c - 1) % NSB) * L::SB_BUF, A.T, w, lane);
-            bchain_step<D, BF, AL>(X, cb[0], lds + L::B_STG + (c % NSB) * L::SB_BUF, lds + L::B_HO + (c & 1) * L::HO_SZ,
-                                   scr, c, A, w, vt, lane);
+            y0 = bchain_step<D, BF, AL>(X, cb[0], lds + L::B_STG + (c % NSB) * L::SB_BUF,
+                                        lds + L::B_HO + (c & 1) * L::HO_SZ, scr, c, A, w, vt, lane);
             bchain_load<BF, AL>(cb[0], max(c - 2, 0), A, R, vt, lane);
             bstage_load<D, BF, AL, NV>(sg[0], max(c - 1 - SETS, 0), A, R, w, lane);
         } else {
             // block c - 1 < NC - 1 is whole (only the last block can be partial)
             if (c >= 1)
                 bstage_store<true>(sg[SETS - 1], c - 1, lds + L::B_STG + ((c - 1) % NSB) * L::SB_BUF, A.T, w, lane);
-            bchain_step<D, BF, AL>(X, cb[1], lds + L::B_STG + (c % NSB) * L::SB_BUF, lds + L::B_HO + (c & 1) * L::HO_SZ,
-                                   scr, c, A, w, vt, lane);
+            y0 = bchain_step<D, BF, AL>(X, cb[1], lds + L::B_STG + (c % NSB) * L::SB_BUF,
+                                        lds + L::B_HO + (c & 1) * L::HO_SZ, scr, c, A, w, vt, lane);
             bchain_load<BF, AL>(cb[1], max(c - 2, 0), A, R, vt, lane);
             bstage_load<D, BF, AL, NV>(sg[SETS - 1], max(c - 1 - SETS, 0), A, R, w, lane);
         }
+        if constexpr (D::CAUSAL)
+            if (any_bad(y0))
+                bchain_again<D, BF, AL>(X, lds + L::B_STG + (c % NSB) * L::SB_BUF, lds + L::B_HO + (c & 1) * L::HO_SZ, scr,
+                                        c, A, R, w, vt, lane);
         lds_barrier();
     }
     // the helpers' last two steps (products of block 0, then its epilogue)

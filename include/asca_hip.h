@@ -156,6 +156,10 @@ ASCA_API int asca_delta_ws_bytes(int B, int T, int H, int dh, size_t* bytes);
  *   q, k, v : (B*T, H*dh), q and k already L2-normalised per head
  *   alpha, beta : (B*T, H)
  *   o : (B*T, H*dh) output
+ * An infinity or NaN in an input of step t reaches the outputs (and, in the
+ * backwards, the gradients) that the step-by-step recurrence takes it to, at
+ * every dh but 64, where it can also reach those of the up to 15 other steps of
+ * its block of 16 (as it can in the chunked form, of its chunk).
  *   ws : asca_delta_ws_bytes(B,T,H,dh) bytes, kept for asca_delta_bwd_* (which
  *        read it and never write it) */
 ASCA_API int asca_delta_fwd(const float* q, const float* k, const float* v,

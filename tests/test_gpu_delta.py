@@ -384,3 +384,30 @@ def test_blocked_widths(orc, g, B, T, H, dh, off):
     assert orc.rel_err(host(dgate, (rows, 2 * H)), d_gate_ref) <= GRAD_TOL
     for b in bufs:
         b.free()
+
+
+@pytest.mark.parametrize("dh", [8, 16, 32, 48, 96, 128])
+@pytest.mark.parametrize("name,val", [("v", np.inf), ("v", np.nan), ("k", np.nan), ("q", np.nan), ("q", np.inf),
+                                      ("d_o", np.inf), ("d_o", np.nan), ("alpha", np.nan), ("beta", np.nan)])
+@pytest.mark.parametrize("T,t", [(50, 21), (50, 37), (50, 48), (64, 15), (40, 32)])
+def test_non_finite_step_reaches_what_the_recurrence_reaches(orc, g, dh, name, val, T, t):
+    # One infinity or NaN at step t of one sequence and head (inside a block of 16
+    # steps, at its ends, in the ragged last one): it is found where the step-by-step
+    # recurrence takes it (outputs from t on, gradients of the steps before where the
+    # adjoint passes t), and every other output is as good as without it.
+    B, H = 2, 2
+    x = orc.DeltaInputs(dh + t, B, T, H, dh)
+    a = getattr(x, name)
+    a[T + t, 1 if name in ("alpha", "beta") else dh + dh // 2] = val
+    with np.errstate(all="ignore"):
+        o, dq, dk, dv, da, db = orc.delta_fwd_bwd(x.q, x.k, x.v, x.alpha, x.beta, x.d_o, B, T, H, dh)
+        d_qkv, d_gate = orc.delta_fuse(x.q, x.k, x.qn, x.kn, x.alpha, x.beta, dq, dk, dv, da, db, H, dh)
+    o_got, dev = g.delta_scan(x.q, x.k, x.v, x.alpha, x.beta, B, T, H, dh)
+    raw = g.delta_bwd_raw(dev, x.d_o)
+    fused = g.delta_bwd_dev(dev, x.d_o, x.qn, x.kn)
+    for n, got, ref, tol in [("o", o_got, o, FWD_TOL)] + [
+            (n, gt, r, GRAD_TOL) for n, gt, r in zip(("dq", "dk", "dv", "dalpha", "dbeta", "d_qkv", "d_gate"),
+                                                     (*raw, *fused), (dq, dk, dv, da, db, d_qkv, d_gate))]:
+        fin = np.isfinite(ref)
+        np.testing.assert_array_equal(np.isfinite(got), fin, err_msg=n)
+        assert np.max(np.abs(got[fin] - ref[fin])) <= tol * np.max(np.abs(ref[fin])), n
