@@ -67,6 +67,9 @@ struct Dim {
     // whether a non-finite value is kept to the steps that the recurrence takes it
     // to (any_bad below); the dh = 64 kernels spread it over its block of 16 steps
     static constexpr bool CAUSAL = NR != 4;
+    // whether sums of a few terms are added up apart from the large value that they
+    // join, in short chains (mfma_sum; T held without its unit diagonal)
+    static constexpr bool FINE = NR != 4;
     static constexpr int DH = 16 * NR, DH2 = DH * DH;
     static constexpr int NWT = NV + NH, NT = 64 * NWT;   // waves, threads of a block
     // row pitches in LDS (4 mod 32 at 64 columns: the 16-byte reads of 16 rows
@@ -107,6 +110,57 @@ ASCA_DEV float acc_sum(const f32x4 (&a)[N], int i) {
 // the scheduler would move past it).  The checks cost B4 T128 H4 dh32 31.6 -> 32.5
 // us, B8 T1000 H8 dh128 528 -> 531 us.
 ASCA_DEV bool any_bad(float x) { return __builtin_expect(__any(!__builtin_isfinite(x)), 0); }
+// FINE sums.  A product over 16 k (a[i], b[i]: its four MFMAs) from zero in NC chains,
+// so that its terms are rounded against their own sum: where it joins a larger value,
+// once against that instead of sixteen times.  Sums of 16 terms that join one (T R,
+// M^T dO, T^T dU, the Gamma o dM and dA parts of dq and dk), the Gram products and
+// dO U^T, Y U^T are formed so.  Error against float64 (forward and fused backward,
+// 2-norm over all outputs, 1e-7) of the per-step kernels, of one chain for every sum,
+// of these: dh16 1.19 1.43 1.18, dh32 1.22 1.44 1.20, dh48 1.24 1.46 1.23, dh96 1.21
+// 1.49 1.21, dh128 1.23 1.53 1.23 (o alone at dh128: 1.11 1.44 1.17).  Time against
+// one chain, forward + backward: B8 T512 H8 dh16 42.5 + 59.8 -> 41.6 + 61.9 us, B4 T128
+// H4 dh32 11.2 + 21.4 -> 11.4 + 21.9, B16 T512 H8 dh48 44.1 + 98.5 -> 43.6 + 99.5, B8
+// T512 H8 dh96 65.4 + 144 -> 66.9 + 150, B8 T1000 H8 dh128 152 + 370 -> 157 + 374.
+template <int NC = 2>
+ASCA_DEV f32x4 mfma_sum(const float (&a)[4], const float (&b)[4]) {
+    const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (NC == 4)
+        return (mfma4(a[0], b[0], z) + mfma4(a[1], b[1], z)) + (mfma4(a[2], b[2], z) + mfma4(a[3], b[3], z));
+    else
+        return mfma4(a[1], b[1], mfma4(a[0], b[0], z)) + mfma4(a[3], b[3], mfma4(a[2], b[2], z));
+}
+ASCA_DEV f32x4 mfma_sum(const float4& a, const float (&b)[4]) {
+    const float x[4] = {a.x, a.y, a.z, a.w};
+    return mfma_sum(x, b);
+}
+template <int NC = 2>
+ASCA_DEV f32x4 mfma_sum(const float4& a, const float4& b) {
+    const float x[4] = {a.x, a.y, a.z, a.w}, y[4] = {b.x, b.y, b.z, b.w};
+    return mfma_sum<NC>(x, y);
+}
+// A product and (E) its rounding error: h + e.
+template <bool E>
+struct Prod {
+    float h, e;
+    ASCA_DEV float value() const { return E ? h + e : h; }
+};
+template <bool E>
+ASCA_DEV Prod<E> operator*(Prod<E> a, Prod<E> b) {
+    const float p = a.h * b.h;
+    if constexpr (!E) return {p, 0.0f};
+    return {p, fmaf(a.h, b.h, -p) + fmaf(a.h, b.e, a.e * b.h)};
+}
+// even (or low) and odd (high) 16-lane rows' (32-lane halves') values, in both
+ASCA_DEV void row_pair16(float x, float& lo, float& hi) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    lo = __uint_as_float(r[0]);
+    hi = __uint_as_float(r[1]);
+}
+ASCA_DEV void row_pair32(float x, float& lo, float& hi) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    lo = __uint_as_float(r[0]);
+    hi = __uint_as_float(r[1]);
+}
 ASCA_DEV float readlane_f(float x, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l)); }
 ASCA_DEV float el(const float4& v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
 
@@ -162,7 +216,7 @@ ASCA_DEV const void* at_el(const void* p, long off) {
 }
 
 // One block's state-independent matrices in LDS (floats).
-constexpr int P_T = 0;      // T = (I + L)^-1, row-major [16][16]
+constexpr int P_T = 0;      // T = (I + L)^-1 (FINE: T - I), row-major [16][16]
 constexpr int P_M = 256;    // M = tril(Gamma o Q K^T), row-major [16][16]
 constexpr int P_GAM = 512;  // gamma_t
 constexpr int P_BET = 528;  // beta_t (0 past the sequence end)
@@ -210,32 +264,60 @@ ASCA_DEV void prep_compute(const PrepIn<D>& pi, int p, int T, float* __restrict_
     const float a = live ? pi.a : 1.0f;
     const float b = live ? pi.b : 0.0f;
     // Gram products: A[t][m] = k_t . k_m, Bq[t][m] = q_t . k_m (lane: t = 4g + i, m = n)
-    // (the key tiles dealt to NA accumulators, as in the chain; one at dh = 64)
-    constexpr int NA = D::NR == 4 ? 1 : D::NR < 4 ? D::NR : 4;
-    f32x4 As[NA], Bs[NA], A, Bq;
+    f32x4 A = {0.f, 0.f, 0.f, 0.f}, Bq = A;
 #pragma unroll
-    for (int a = 0; a < NA; ++a) As[a] = Bs[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r < D::NR; ++r) {
+        if constexpr (D::FINE) {
+            constexpr int NC = D::NR < 4 ? 4 : 2;  // (four chains spill at dh = 128)
+            A += mfma_sum<NC>(pi.kr[r], pi.kr[r]);
+            Bq += mfma_sum<NC>(pi.qr[r], pi.kr[r]);
+        } else {
 #pragma unroll
-    for (int r = 0; r < D::NR; ++r)
+            for (int i = 0; i < 4; ++i) {
+                A = mfma4(el(pi.kr[r], i), el(pi.kr[r], i), A);
+                Bq = mfma4(el(pi.qr[r], i), el(pi.kr[r], i), Bq);
+            }
+        }
+    }
+    // gam: lane n's gamma_n; G[i] = Gamma[4g + i][n] for 4g + i >= n; pr = Gamma[15][n]
+    float gam, G[4] = {1.f, 1.f, 1.f, 1.f}, pr = 1.0f;
+    if constexpr (D::FINE) {
+        // with their rounding errors at the column splits, where a helper has the time
+        // (dh128 forward 155 -> 157 us; at dh16 it is what the chain waits for, 42 -> 47)
+        using P = Prod<(D::VS > 1)>;
+        P x = {a, 0.0f};
+        x = P{dpp_or<0x111>(1.0f, x.h), dpp_or<0x111>(0.0f, x.e)} * x;
+        x = P{dpp_or<0x112>(1.0f, x.h), dpp_or<0x112>(0.0f, x.e)} * x;
+        x = P{dpp_or<0x114>(1.0f, x.h), dpp_or<0x114>(0.0f, x.e)} * x;
+        x = P{dpp_or<0x118>(1.0f, x.h), dpp_or<0x118>(0.0f, x.e)} * x;
+        gam = x.value();
+        // products over the lane group's own steps 4g .. 4g + i past n, then those of
+        // the groups before it and of all four
+        P l[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            As[r % NA] = mfma4(el(pi.kr[r], i), el(pi.kr[r], i), As[r % NA]);
-            Bs[r % NA] = mfma4(el(pi.qr[r], i), el(pi.kr[r], i), Bs[r % NA]);
+            const float as = __shfl(a, 4 * g + i);
+            const P y = {4 * g + i > n ? as : 1.0f, 0.0f};
+            l[i] = i ? l[i - 1] * y : y;
         }
+        P even, odd, low, high;
+        row_pair16(l[3].h, even.h, odd.h);
+        row_pair16(l[3].e, even.e, odd.e);
+        const P two = even * odd;
+        row_pair32(two.h, low.h, high.h);
+        row_pair32(two.e, low.e, high.e);
+        pr = (low * high).value();
+        const P one = {1.0f, 0.0f}, three = low * even, pre = g == 0 ? one : g == 1 ? even : g == 2 ? low : three;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        A[i] = acc_sum(As, i);
-        Bq[i] = acc_sum(Bs, i);
-    }
-    const float gam = prefix_prod<16>(a);  // lane n: gamma_n
-    // G[i] = Gamma[4g + i][n] for 4g + i >= n; pr ends as Gamma[15][n]
-    float G[4] = {1.f, 1.f, 1.f, 1.f};
-    float pr = 1.0f;
+        for (int i = 0; i < 4; ++i) G[i] = (pre * l[i]).value();
+    } else {
+        gam = prefix_prod<16>(a);
 #pragma unroll
-    for (int s = 0; s < C; ++s) {
-        const float as = readlane_f(a, s);
-        pr = s > n ? pr * as : pr;
-        if ((s >> 2) == g) G[s & 3] = pr;
+        for (int s = 0; s < C; ++s) {
+            const float as = readlane_f(a, s);
+            pr = s > n ? pr * as : pr;
+            if ((s >> 2) == g) G[s & 3] = pr;
+        }
     }
     if (g == 0) {
         ps[P_GAM + n] = gam;
@@ -285,6 +367,11 @@ ASCA_DEV void prep_compute(const PrepIn<D>& pi, int p, int T, float* __restrict_
             for (int q4 = 0; q4 < 4; ++q4)
                 *reinterpret_cast<float4*>(ps + P_T + n * 16 + 4 * q4) =
                     make_float4(x[4 * q4], x[4 * q4 + 1], x[4 * q4 + 2], x[4 * q4 + 3]);
+        }
+        if constexpr (D::FINE) {
+            wave_sync();
+            ps[P_T + 17 * n] = 0.0f;
+            wave_sync();
         }
     };
     auto record_t = [&] {
@@ -518,8 +605,14 @@ ASCA_DEV float chain_step(f32x4 (&S)[D::NR], const float* __restrict__ kb, const
         qs[i] = acc_sum(qa, i);
     }
     f32x4 U = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (D::FINE) {
+        U = mfma_sum(tr, R);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) U = mfma4(el(tr, i), R[i], U);
+        for (int i = 0; i < 4; ++i) U[i] += R[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) U = mfma4(el(tr, i), R[i], U);
+    }
     f32x4 O;
 #pragma unroll
     for (int i = 0; i < 4; ++i) O[i] = el(gm, i) * qs[i];
@@ -918,7 +1011,13 @@ ASCA_DEV float bchain_step(f32x4 (&X)[D::NR], const BChainIn<BF>& ci, const floa
 #pragma unroll
     for (int j = 0; j < 4; ++j) dU[j] = el(gc, j) * acc_sum(kx, j);
     f32x4 Y = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (!MASKED) {
+    if constexpr (!MASKED && D::FINE) {
+        const f32x4 md = mfma_sum(ci.mr, dO);
+        float du[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) du[j] = dU[j] += md[j];
+        Y = dU + mfma_sum(ci.tr, du);
+    } else if constexpr (!MASKED) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) dU = mfma4(el(ci.mr, j), dO[j], dU);
 #pragma unroll
@@ -937,6 +1036,7 @@ ASCA_DEV float bchain_step(f32x4 (&X)[D::NR], const BChainIn<BF>& ci, const floa
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) scr[(4 * g + j) * OTP + n] = dU[j];
+        if constexpr (D::FINE) Y = dU;  // T's diagonal
         wave_sync();
 #pragma unroll 1
         for (int t = 0; t < C; ++t) {
@@ -944,7 +1044,7 @@ ASCA_DEV float bchain_step(f32x4 (&X)[D::NR], const BChainIn<BF>& ci, const floa
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const float y = fmaf(rec[R_T + 4 * (16 * (t >> 2) + 4 * g + j) + (t & 3)], x, Y[j]);
-                Y[j] = t >= 4 * g + j ? y : Y[j];
+                Y[j] = t > 4 * g + j || (!D::FINE && t == 4 * g + j) ? y : Y[j];
             }
         }
         wave_sync();
@@ -960,10 +1060,15 @@ ASCA_DEV float bchain_step(f32x4 (&X)[D::NR], const BChainIn<BF>& ci, const floa
     const float4 do4 = *reinterpret_cast<const float4*>(sb + L::SB_DO + n * D::RV + 16 * w + 4 * g);
     const float4 u4 = *reinterpret_cast<const float4*>(sb + L::SB_U + n * D::RV + 16 * w + 4 * g);
     f32x4 pm = {0.f, 0.f, 0.f, 0.f}, pl = pm;
+    if constexpr (D::FINE) {
+        pm = mfma_sum(do4, u4);
+        pl = mfma_sum(y4, u4);
+    } else {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        pm = mfma4(el(do4, j), el(u4, j), pm);
-        pl = mfma4(el(y4, j), el(u4, j), pl);
+        for (int j = 0; j < 4; ++j) {
+            pm = mfma4(el(do4, j), el(u4, j), pm);
+            pl = mfma4(el(y4, j), el(u4, j), pl);
+        }
     }
     *reinterpret_cast<float4*>(ho + L::HO_DM + (w * 64 + lane) * 4) = make_float4(pm[0], pm[1], pm[2], pm[3]);
     *reinterpret_cast<float4*>(ho + L::HO_DL + (w * 64 + lane) * 4) = make_float4(pl[0], pl[1], pl[2], pl[3]);
@@ -1121,13 +1226,23 @@ ASCA_DEV float bhelp_products(BCarry<D>& cy, const BHelpIn<D>& hi, const float* 
         for (int s = 0; s < KS; ++s) {
             const float4 x4 =
                 *reinterpret_cast<const float4*>(ho + L::HO_DS + (((hw * KS + s) * NV + cc) * 64 + lane) * 4);
+            // (a column split's value tiles apart: their sums are half of what is added)
+            f32x4 f = {0.f, 0.f, 0.f, 0.f}, z = f, d = f;
+            if constexpr (D::VS == 1) {
+                f = F[s];
+                z = Zt[s];
+                d = Dx[s];
+            }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                F[s] = mfma4(el(sk[s][cc], j), el(dO4, j), F[s]);
-                Zt[s] = mfma4(el(sk[s][cc], j), el(y4, j), Zt[s]);
-                Dx[s] = mfma4(el(x4, j), el(u4, j), Dx[s]);
+                f = mfma4(el(sk[s][cc], j), el(dO4, j), f);
+                z = mfma4(el(sk[s][cc], j), el(y4, j), z);
+                d = mfma4(el(x4, j), el(u4, j), d);
                 dss += el(x4, j) * el(sk[s][cc], j);
             }
+            F[s] = D::VS == 1 ? f : F[s] + f;
+            Zt[s] = D::VS == 1 ? z : Zt[s] + z;
+            Dx[s] = D::VS == 1 ? d : Dx[s] + d;
         }
     }
     // dM = tril(dO U^T), dL = -strict_tril(Y U^T) from the chain waves' shares
@@ -1169,7 +1284,13 @@ ASCA_DEV float bhelp_products(BCarry<D>& cy, const BHelpIn<D>& hi, const float* 
             dq[j] = gam * F[s][j];
             dk[j] = gcn * Dx[s][j] - bt * gam * Zt[s][j];
         }
-        if constexpr (!MASKED) {
+        if constexpr (!MASKED && D::FINE) {
+            const float gd[4] = {GdM[0], GdM[1], GdM[2], GdM[3]};
+            const float as[4] = {dA[0] + dat.x, dA[1] + dat.y, dA[2] + dat.z, dA[3] + dat.w};
+            const float gt[4] = {gdmt.x, gdmt.y, gdmt.z, gdmt.w};
+            dq += mfma_sum(kb, gt);
+            dk += mfma_sum(qb, gd) + mfma_sum(kb, as);
+        } else if constexpr (!MASKED) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 dq = mfma4(kb[j], el(gdmt, j), dq);
