@@ -146,16 +146,20 @@ ASCA_DEV void frag_read(float (&f)[4][4], const float* t, int w0, int h, int lan
 // The bf16 MFMA rounds its sums down (towards minus infinity: mean error -2.6e-8
 // of the rms at K = 512, where the f32 MFMA shows none), and a sum over many
 // rows of such a product (a bias gradient over 16384 tokens) adds these up: its
-// error was 3.7e-6 against 1.2e-6.  So odd rows of a tile are multiplied
+// error was 3.7e-6 against 1.2e-6.  So odd rows of the large tiles are multiplied
 // negated and negated back at the end, which makes every second row's error
-// positive.
+// positive, and equal rows of A differ in their last bits between odd and even
+// places.  The 64 x 64 tile negates every second wave's part of the k range instead,
+// so that equal rows of A (a batch of sequences being decoded) give equal rows of C.
+// In the large tiles that cost 3% (the sums negated every four k-tiles), signs by a row's
+// values instead of its place 1 to 5% (routed FFN 777 -> 815 us).
 //
 // The bf16 MFMA takes subnormal inputs as zero, and x1 and x2 lie up to 2^9 and
 // 2^17 below x: unscaled, operands below 2^-110 lost them (a product of rows at
 // 2^-120 had an error of 3.5e-5, at 2^-128 9e-3).  So both operands are split as
 // 2^24 x, where the smallest subnormal float is a normal bf16, and the sums are
 // scaled back by 2^-48: the same bits where nothing under- or overflows.  The
-// odd rows' sign is part of the factor.  The multiplications cost 1 to 2%
+// sign is part of the factor.  The multiplications cost 1 to 2%
 // (16384x512x1536 forward and backward 418 -> 426 us, training step 14.00 -> 14.15 ms).
 //
 // A value that is not finite, or is 2^104 or more, or a sum of 2^80 or more
@@ -425,17 +429,18 @@ ASCA_DEV void split_redo(f32x4 (&acc)[NX][NY], int x0, int y0, const float* A, c
     }
 }
 
-// The sums scaled back, those of the rows that were multiplied negated (odd rows
+// The sums scaled back; ODD: those of the rows that were multiplied negated (odd rows
 // of the tile: row 16 x + 4 (lane / 16) + r, or 4 i + x of an mn-contiguous A)
-// negated back.
-template <bool TA, int NX, int NY>
-ASCA_DEV void split_sign(f32x4 (&acc)[NX][NY], int x0) {
+// negated back.  Plus zero, so that a sum of zeros is not a negative one.
+template <bool ODD, bool TA, int NX, int NY>
+ASCA_DEV void split_unscale(f32x4 (&acc)[NX][NY]) {
 #pragma unroll
     for (int x = 0; x < NX; ++x)
 #pragma unroll
         for (int y = 0; y < NY; ++y)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[x][y][r] *= (TA ? x0 + x : r) & 1 ? -SP_UNSCALE : SP_UNSCALE;
+            for (int r = 0; r < 4; ++r)
+                acc[x][y][r] = fmaf(acc[x][y][r], ODD && ((TA ? x : r) & 1) ? -SP_UNSCALE : SP_UNSCALE, 0.0f);
 }
 
 // Any infinity or NaN among a wave's sums?
@@ -534,7 +539,7 @@ ASCA_DEV void split_mainloop(f32x4 (&acc)[4][4], const float* A, const float* B,
     };
     for (; t + 2 < nw; ++t) step(std::true_type{});
     for (; t < nk; ++t) step(std::false_type{});
-    split_sign<TA>(acc, 0);
+    split_unscale<true, TA>(acc);
     if (split_bad(acc))
         split_redo<TA, TB, 4>(acc, 0, 0, A, B, p, a_off, b_off, m0 + wm, n0 + wn, lim_m - wm, lim_n - wn, K_lo, K_hi, lane);
 }
@@ -783,9 +788,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // Loads are buffer loads (32-bit lane offsets, the k-tile's offset in a scalar
 // register: 64-bit addresses would take the registers the fragments need), so
 // an operand's rows must lie within 4 GB (small_fits).
-// NTL 16-row tiles (mn-contiguous: row NTL i + j is row i of tile j).  NEG: odd
-// rows negated.
-template <bool KC, bool GATHER, bool NEG, int NTL>
+// NTL 16-row tiles (mn-contiguous: row NTL i + j is row i of tile j).
+template <bool KC, bool GATHER, int NTL>
 struct FragTile {
     const float* base;           // KC: k = K_lo of row 0; MC: k = K_lo of the tile's first column
     unsigned vo[KC ? NTL : 1];   // lane's byte offsets: KC: row 16 x + i at its k; MC: its k and column NTL i
@@ -862,15 +866,14 @@ struct FragTile {
             }
         }
     }
-    // the three bf16 fragments of 16-row tile j
-    ASCA_DEV void frag(int j, bf16x8 (&out)[3]) const {
+    // the three bf16 fragments of f times 16-row tile j
+    ASCA_DEV void frag(int j, bf16x8 (&out)[3], float f) const {
         typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
         u32x4 w[3];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             float a = KC ? x[2 * j + e / 2][2 * (e & 1)] : x[2 * e][j];
             float b = KC ? x[2 * j + e / 2][2 * (e & 1) + 1] : x[2 * e + 1][j];
-            const float f = sp_factor(!NEG ? 0 : KC ? col & NTL : j & 1);  // col / NTL = lane % 16: the KC lane's row
             a *= f;
             b *= f;
             unsigned w0, w1, w2;
@@ -901,8 +904,8 @@ ASCA_DEV void small_tile(const T& t, const GemmArgs& p) {
         for (int y = 0; y < NY; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
     const long nk = (t.K_hi - t.K_lo + SP_BK - 1) / SP_BK;
     if (w < nk) {
-        FragTile<!TA, GATHER == 1, true, NX> fa;
-        FragTile<TB, GATHER == 2, false, NY> fb;
+        FragTile<!TA, GATHER == 1, NX> fa;
+        FragTile<TB, GATHER == 2, NY> fb;
         fa.init(t.A, p.lda, p.a_rows, t.a_off, t.m0, t.lim_m, t.K_lo, lane);
         fb.init(t.B, p.ldb, p.b_rows, t.b_off, t.n0, t.lim_n, t.K_lo, lane);
         const bool whole = fa.whole(t.lim_m) && fb.whole(t.lim_n);
@@ -926,7 +929,7 @@ ASCA_DEV void small_tile(const T& t, const GemmArgs& p) {
         for (long kt = w;;) {
             bf16x8 a[NX][3];
 #pragma unroll
-            for (int x = 0; x < NX; ++x) fa.frag(x, a[x]);
+            for (int x = 0; x < NX; ++x) fa.frag(x, a[x], sp_factor(w & 1));
             kt += SM_NW;
             if (kt < nk) load_a(kt);
             // one column tile at a time: its fragments are split beside the
@@ -934,7 +937,7 @@ ASCA_DEV void small_tile(const T& t, const GemmArgs& p) {
 #pragma unroll
             for (int y = 0; y < NY; ++y) {
                 bf16x8 b[3];
-                fb.frag(y, b);
+                fb.frag(y, b, SP_SCALE);
                 constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
                 for (int s = 0; s < 6; ++s)
@@ -962,9 +965,12 @@ ASCA_DEV void small_tile(const T& t, const GemmArgs& p) {
     for (int y = 0; y < PW; ++y) {
         sum[0][y] = part[(NY * x0 + y0 + y) * 64 + lane];
 #pragma unroll
-        for (int v = 1; v < SM_NW; ++v) sum[0][y] += part[(v * TL + NY * x0 + y0 + y) * 64 + lane];
+        for (int v = 1; v < SM_NW; ++v) {
+            const f32x4 pv = part[(v * TL + NY * x0 + y0 + y) * 64 + lane];
+            sum[0][y] = v & 1 ? sum[0][y] - pv : sum[0][y] + pv;  // (sp_factor(w & 1))
+        }
     }
-    split_sign<TA>(sum, x0);
+    split_unscale<false, TA>(sum);
     if (split_bad(sum))
         split_redo<TA, TB, NY>(sum, x0, y0, t.A, t.B, p, t.a_off, t.b_off, t.m0, t.n0, t.lim_m, t.lim_n, t.K_lo, t.K_hi,
                                lane);

@@ -559,3 +559,22 @@ def test_moe_config3_shape_by_token_subsets(orc, g):
         err = orc.rel_err(got, want)
         print(f"[moe]   {name} rel err {err:.2e}", flush=True)
         assert err <= GRAD_TOL, name
+
+
+@pytest.mark.parametrize("M,N,K", [(2, 96, 64), (5, 700, 257), (64, 1536, 512), (33, 100, 1000), (512, 1536, 512)])
+def test_gemm_equal_rows(g, M, N, K):
+    # A batch of equal rows (decoding the same sequence twice): every row of the
+    # product has the same bits, at odd and even places.
+    rng = np.random.default_rng(M + K)
+    a = np.repeat(rng.standard_normal((1, K)).astype(np.float32), M, axis=0)
+    got = g.gemm(a, rng.standard_normal((K, N)).astype(np.float32)).view(np.uint32)
+    np.testing.assert_array_equal(got, np.repeat(got[:1], M, axis=0))
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(7, 130, 40), (4096, 512, 64), (8192, 1024, 96)])
+def test_gemm_of_zeros_is_positive(g, ta, tb, M, N, K):
+    rng = np.random.default_rng(M)
+    b = rng.standard_normal((N, K) if tb else (K, N)).astype(np.float32)
+    got = g.gemm(np.zeros((K, M) if ta else (M, K), np.float32), b, trans_a=bool(ta), trans_b=bool(tb))
+    assert not got.view(np.uint32).any()  # (-0 has its sign bit set)
