@@ -234,6 +234,7 @@ ASCA_DEV float sp_factor(int odd) { return odd ? -SP_SCALE : SP_SCALE; }
 // Rows past the operand's extent repeat a valid one (KC) or read as 0 (MC);
 // k past the range read as 0.
 // Stored as SP_SCALE x; NEG: odd rows negated.
+enum { LD_EDGE, LD_QUADS, LD_WHOLE };
 template <bool KC, bool GATHER, bool NEG, int R, int NT>
 struct SplitTile {
     static constexpr int NI = KC ? R * 4 / NT : 1, W = R * 8 / NT, NF = R * 32 / NT;
@@ -274,9 +275,45 @@ struct SplitTile {
     }
     // Whether every thread's columns of the tile are all valid or all past the extent.
     ASCA_DEV static bool whole(int lim_mn) { return KC || lim_mn >= R || lim_mn % W == 0; }
-    // k-tile at K_lo + k.  WHOLE: all of its k are valid and whole(lim_mn).
-    template <bool WHOLE>
+    // k-tile at K_lo + k.  WHOLE: all of its k are valid and whole(lim_mn).  QUADS:
+    // whole(lim_mn) and lim_k a multiple of 4, so that four k are valid or not together
+    // (one by one, each element a load of its own: 16384 x 1536 x 48 41.5 us instead of
+    // 37.9, its twin with B transposed 51 and 43.6; the f32 kernels took 37.5 and 46.6).
+    template <int MODE>
     ASCA_DEV void load(long k, long lim_k, int lim_mn) {
+        constexpr bool WHOLE = MODE == LD_WHOLE;
+        if constexpr (MODE == LD_QUADS) {
+            const int lk = (int)min(lim_k, (long)SP_BK);
+            if constexpr (KC) {
+#pragma unroll
+                for (int j = 0; j < NI; ++j) {
+                    const float* q = p[j] + k - kofs;
+                    const f32x4u a = *reinterpret_cast<const f32x4u*>(q + min(kofs, lk - 4));
+                    const f32x4u b = *reinterpret_cast<const f32x4u*>(q + min(kofs + 4, lk - 4));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        x[8 * j + e] = kofs < lk ? a[e] : 0.0f;
+                        x[8 * j + 4 + e] = kofs + 4 < lk ? b[e] : 0.0f;
+                    }
+                }
+            } else {
+                const int k0 = min(kofs, lk - 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float* q = GATHER ? p[0] + (long)idx[e] * ld : p[0] + (k + k0 - kofs + e) * ld;
+                    if constexpr (W == 4) {
+                        const f32x4u a = *reinterpret_cast<const f32x4u*>(q);
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) x[4 * e + c] = kofs < lk ? a[c] : 0.0f;
+                    } else {
+                        const f32x2u a = *reinterpret_cast<const f32x2u*>(q);
+                        x[2 * e] = kofs < lk ? a[0] : 0.0f;
+                        x[2 * e + 1] = kofs < lk ? a[1] : 0.0f;
+                    }
+                }
+            }
+            return;
+        }
         if constexpr (KC) {
             if constexpr (WHOLE) {
 #pragma unroll
@@ -480,20 +517,23 @@ ASCA_DEV void split_mainloop(f32x4 (&acc)[4][4], const float* A, const float* B,
     const long nk = (K_hi - K_lo + SP_BK - 1) / SP_BK;  // > 0
     const bool whole = ta.whole(lim_m) && tb.whole(lim_n);
     const long nw = whole ? (K_hi - K_lo) / SP_BK : 0;  // k-tiles that load without checks
-    auto load_as = [&](long kt, auto Whole) {
-        constexpr bool wh = decltype(Whole)::value;
+    const bool quads = whole && (K_hi - K_lo) % 4 == 0;
+    auto load_as = [&](long kt, auto Mode) {
+        constexpr int mode = decltype(Mode)::value;
         const long k = kt * SP_BK, lim_k = K_hi - K_lo - k;
-        ta.template load<wh>(k, lim_k, lim_m);
-        tb.template load<wh>(k, lim_k, lim_n);
+        ta.template load<mode>(k, lim_k, lim_m);
+        tb.template load<mode>(k, lim_k, lim_n);
         const long kn = K_lo + min(kt + 1, nk - 1) * SP_BK;  // the storage rows of the k-tile after it
         if constexpr (GATHER == 1) ta.next_rows(p.a_rows, a_off, kn, K_hi);
         if constexpr (GATHER == 2) tb.next_rows(p.b_rows, b_off, kn, K_hi);
     };
     auto load = [&](long kt) {
         if (kt < nw)
-            load_as(kt, std::true_type{});
+            load_as(kt, std::integral_constant<int, LD_WHOLE>{});
+        else if (kt < nk && quads)
+            load_as(kt, std::integral_constant<int, LD_QUADS>{});
         else if (kt < nk)
-            load_as(kt, std::false_type{});
+            load_as(kt, std::integral_constant<int, LD_EDGE>{});
     };
     load(0);
     ta.store(lds, tid);
@@ -512,7 +552,7 @@ ASCA_DEV void split_mainloop(f32x4 (&acc)[4][4], const float* A, const float* B,
         ta.store(nxt, tid);  // (past the last k-tile: not read)
         tb.store(nxt + sp_tile<RA>(), tid);
         if constexpr (decltype(Whole)::value)
-            load_as(t + 2, Whole);
+            load_as(t + 2, std::integral_constant<int, LD_WHOLE>{});
         else
             load(t + 2);
         if constexpr (DB && decltype(Whole)::value) {

@@ -52,6 +52,8 @@ def _ref_gemm(a, b, ta, tb, alpha, beta, c, bias):
 @pytest.mark.parametrize("M,N,K", [(64, 64, 31), (65, 67, 33), (1, 3, 257), (257, 129, 64), (384, 1030, 1027),
                                    (4096, 512, 96), (4097, 511, 65), (2048, 2052, 128),
                                    (16, 130, 300), (17, 2100, 96), (40, 4097, 64),
+                                   # a last k-tile of whole quads of k, on the large tiles
+                                   (8200, 1030, 12), (4096, 516, 76), (8192, 1024, 36),
                                    # 128 x 256 tiles past whole rounds, done as 64 x 64 tiles: 4 to 10
                                    (16700, 500, 515), (16540, 449, 352), (520, 13300, 384)])
 def test_gemm_split_products(g, ta, tb, M, N, K):
