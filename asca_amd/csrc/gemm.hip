@@ -164,7 +164,7 @@ ASCA_DEV void frag_read(float (&f)[4][4], const float* t, int w0, int h, int lan
 //
 // A value that is not finite, or is 2^104 or more, or a sum of 2^80 or more
 // leaves a non-finite sum wherever it enters: a wave that finds one among its sums
-// computes its tile again with f32 products (split_redo), so infinities and
+// computes its tile again with f32 products (f32_products), so infinities and
 // NaN come out as the f32 products give them.
 //
 // LDS image of one operand tile (R rows x 32 k): three planes (x0, x1, x2) of
@@ -220,6 +220,11 @@ ASCA_DEV void split2(float a, float b, unsigned& w0, unsigned& w1, unsigned& w2)
     w2 = pk_bf16(a, b);
 }
 
+// The longest k range that is not split: one f32 MFMA, each product rounded once,
+// where the six parts' sum of one product is 1.4 times as far off (2.5e-8 -> 3.4e-8, up to
+// 2.7 units of 2^-24 instead of 1; from 4 products on it is the closer one).  Nor is
+// anything staged: 16384 x 1536 x 4 33 -> 22 us, 27 with the f32 kernels.
+constexpr long SP_F32_K = 4;
 constexpr float SP_SCALE = 0x1p24f, SP_UNSCALE = 0x1p-48f;
 // the factor of an operand's values: SP_SCALE, negative where `odd` is not zero
 ASCA_DEV float sp_factor(int odd) { return odd ? -SP_SCALE : SP_SCALE; }
@@ -426,7 +431,7 @@ ASCA_DEV void split_mma(f32x4 (&acc)[4][4], const char* As, const char* Bs, int 
     }
 }
 
-// One operand element (row mn0 + r, k) for split_redo; 0 outside the product
+// One operand element (row mn0 + r, k) for f32_products; 0 outside the product
 template <bool KC>
 ASCA_DEV float split_elem(const float* base, long ld, const int* rows, long off, int mn0, int r, int lim_mn, long k,
                           long K_hi) {
@@ -434,11 +439,16 @@ ASCA_DEV float split_elem(const float* base, long ld, const int* rows, long off,
     return KC ? base[srow(rows, off, mn0 + r) * ld + k] : base[srow(rows, off, k) * ld + mn0 + r];
 }
 
-// The sums of the NX x NY 16 x 16 tiles from (x0, y0) of a wave's 64 x 64 again,
-// as f32 products straight from memory.
+// The sums of the NX x NY 16 x 16 tiles from (x0, y0) of a wave's 64 x 64 as f32
+// products straight from memory: for sums that the split leaves non-finite, and for a k
+// range of at most SP_F32_K.  A product whose sums are all redone takes 4 to 6 times
+// as long (16384 x 1536 x 512 142 -> 624 us, 220 with the f32 kernels; 64 x 1536 x 512
+// 8.8 -> 39); only the waves that find one redo theirs (one NaN row of 16384: 190).
+// Vector loads two steps ahead made that 1.7 times as fast and the finite products 2
+// to 8% slower (registers).
 // (CB: columns of an mn-contiguous B interleaved over so many tiles)
 template <bool TA, bool TB, int CB, int NX, int NY>
-ASCA_DEV void split_redo(f32x4 (&acc)[NX][NY], int x0, int y0, const float* A, const float* B, const GemmArgs& p,
+ASCA_DEV void f32_products(f32x4 (&acc)[NX][NY], int x0, int y0, const float* A, const float* B, const GemmArgs& p,
                          long a_off, long b_off, int m0, int n0, int lim_m, int lim_n, long K_lo, long K_hi,
                          int lane) {
     const int i = lane & 15;
@@ -581,7 +591,7 @@ ASCA_DEV void split_mainloop(f32x4 (&acc)[4][4], const float* A, const float* B,
     for (; t < nk; ++t) step(std::false_type{});
     split_unscale<true, TA>(acc);
     if (split_bad(acc))
-        split_redo<TA, TB, 4>(acc, 0, 0, A, B, p, a_off, b_off, m0 + wm, n0 + wn, lim_m - wm, lim_n - wn, K_lo, K_hi, lane);
+        f32_products<TA, TB, 4>(acc, 0, 0, A, B, p, a_off, b_off, m0 + wm, n0 + wn, lim_m - wm, lim_n - wn, K_lo, K_hi, lane);
 }
 
 // The tile, group and K range of a block.
@@ -796,8 +806,9 @@ ASCA_DEV void gemm_epilogue(const f32x4 (&acc)[NX][NY], int x0, int y0, int m0, 
     }
 }
 
-// Block tile (64 WM) x (64 WN) on WM x WN waves; a wave owns 64 x 64.
-template <bool TA, bool TB, int EPI, int GATHER, int WM, int WN, bool DB, class T>
+// Block tile (64 WM) x (64 WN) on WM x WN waves; a wave owns 64 x 64.  FEW: the k
+// range can be at most SP_F32_K.
+template <bool TA, bool TB, int EPI, int GATHER, int WM, int WN, bool DB, bool FEW, class T>
 ASCA_DEV void gemm_tile(const T& t, const GemmArgs& p) {
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int wm = (w / WN) * 64, wn = (w % WN) * 64;
@@ -806,7 +817,10 @@ ASCA_DEV void gemm_tile(const T& t, const GemmArgs& p) {
     for (int x = 0; x < 4; ++x)
 #pragma unroll
         for (int y = 0; y < 4; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (t.K_hi > t.K_lo)
+    if (FEW && t.K_hi - t.K_lo <= SP_F32_K)
+        f32_products<TA, TB, 4>(acc, 0, 0, t.A, t.B, p, t.a_off, t.b_off, t.m0 + wm, t.n0 + wn, t.lim_m - wm,
+                                t.lim_n - wn, t.K_lo, t.K_hi, lane);
+    else if (t.K_hi > t.K_lo)
         split_mainloop<TA, TB, GATHER, WM, WN, DB>(acc, t.A, t.B, p, t.a_off, t.b_off, t.m0, t.n0, t.lim_m, t.lim_n,
                                                    t.K_lo, t.K_hi, tid, wm, wn);
     gemm_epilogue<TA, TB, EPI, 4>(acc, 0, 0, t.m0 + wm, t.n0 + wn, t, p, lane);
@@ -816,7 +830,7 @@ template <bool TA, bool TB, int EPI, int GATHER>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_k(GemmArgs p) {
     BlockTile<TA, TB, 128, 128> t;
     if (!t.init(p)) return;
-    gemm_tile<TA, TB, EPI, GATHER, 2, 2, false>(t, p);
+    gemm_tile<TA, TB, EPI, GATHER, 2, 2, false, true>(t, p);
 }
 
 // Products too small to fill the chip with the tiles above: one 64 x 64 tile
@@ -942,7 +956,8 @@ ASCA_DEV void small_tile(const T& t, const GemmArgs& p) {
     for (int x = 0; x < NX; ++x)
 #pragma unroll
         for (int y = 0; y < NY; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const long nk = (t.K_hi - t.K_lo + SP_BK - 1) / SP_BK;
+    const bool few = t.K_hi - t.K_lo <= SP_F32_K;
+    const long nk = few ? 0 : (t.K_hi - t.K_lo + SP_BK - 1) / SP_BK;
     if (w < nk) {
         FragTile<!TA, GATHER == 1, NX> fa;
         FragTile<TB, GATHER == 2, NY> fb;
@@ -1011,8 +1026,8 @@ ASCA_DEV void small_tile(const T& t, const GemmArgs& p) {
         }
     }
     split_unscale<false, TA>(sum);
-    if (split_bad(sum))
-        split_redo<TA, TB, NY>(sum, x0, y0, t.A, t.B, p, t.a_off, t.b_off, t.m0, t.n0, t.lim_m, t.lim_n, t.K_lo, t.K_hi,
+    if (few || split_bad(sum))
+        f32_products<TA, TB, NY>(sum, x0, y0, t.A, t.B, p, t.a_off, t.b_off, t.m0, t.n0, t.lim_m, t.lim_n, t.K_lo, t.K_hi,
                                lane);
     gemm_epilogue<TA, TB, EPI, NY>(sum, x0, y0, t.m0, t.n0, t, p, lane);
 }
@@ -1041,7 +1056,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if ((int)blockIdx.x < first) {
         if ((int)blockIdx.x >= cut) return;
         t.init(p, t.of_block(blockIdx.x, cut));
-        gemm_tile<TA, TB, EPI, GATHER, 2, 4, true>(t, p);
+        // (few k: groups of a grouped K; best_tile keeps other products of so few off this tile)
+        gemm_tile<TA, TB, EPI, GATHER, 2, 4, true, TA && !TB>(t, p);
         return;
     }
     for (int i = blockIdx.x - first; i < 8 * (n - cut); i += p.tail_blocks) {
@@ -1386,6 +1402,7 @@ static Tile best_tile(long M, long N, int groups, long mult, long steps, bool sm
     // (one K range: the splits' blocks are not tiles of one launch dimension)
     const bool tail = small_ok && whole_k;
     double t = tile_us(T_WIDE, mult * tile_count(T_WIDE, M, N, groups), steps, tail);
+    if (steps <= 1) t = 1e30;  // (SP_F32_K; and the first loads of two blocks per CU overlap)
     for (Tile c : {T_128, T_SMALL}) {
         if (c == T_SMALL && !small_ok) continue;
         const double u = tile_us(c, mult * tile_count(c, M, N, groups), steps, false);

@@ -580,3 +580,21 @@ def test_gemm_of_zeros_is_positive(g, ta, tb, M, N, K):
     b = rng.standard_normal((N, K) if tb else (K, N)).astype(np.float32)
     got = g.gemm(np.zeros((K, M) if ta else (M, K), np.float32), b, trans_a=bool(ta), trans_b=bool(tb))
     assert not got.view(np.uint32).any()  # (-0 has its sign bit set)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("M,N", [(3, 50), (65, 200), (1000, 1000), (4100, 1030), (16400, 520)])
+def test_gemm_few_k(g, ta, tb, M, N):
+    """Up to four products: one is the correctly rounded f32 product, more are off by
+    at most a rounding each (2^-24 of the running sum, itself at most sum |a||b|)."""
+    for K in (1, 2, 3, 4):
+        rng = np.random.default_rng(M + K)
+        a = rng.standard_normal((K, M) if ta else (M, K)).astype(np.float32)
+        b = rng.standard_normal((N, K) if tb else (K, N)).astype(np.float32)
+        got = g.gemm(a, b, trans_a=bool(ta), trans_b=bool(tb))
+        A, Bm = (a.T if ta else a).astype(np.float64), (b.T if tb else b).astype(np.float64)
+        ref = A @ Bm
+        if K == 1:
+            np.testing.assert_array_equal(got, ref.astype(np.float32))
+        else:
+            assert np.all(np.abs(got - ref) <= K * 2.0**-24 * (np.abs(A) @ np.abs(Bm)))
