@@ -87,10 +87,13 @@ bool ut_fits(int T, int H, int dh, long ld);
 DeltaWs ut_ws_layout(int B, int T, int H, int dh, void* base);
 int launch_ut_fwd(const void* q, const void* k, const void* v, bool bf, const float* alpha, const float* beta,
                   float* o, const DeltaWs& ws, int B, int T, int H, int dh, hipStream_t st);
+// floats of scratch that a backward takes
+size_t ut_bwd_scratch(int B, int T, int H, int dh);
+// `scratch`: ut_bwd_scratch floats, or null: the stream's
 int launch_ut_bwd(bool fused, const void* q, const void* k, const void* v, bool bf, const float* alpha,
-                  const float* beta, const void* d_o, const DeltaWs& ws, const float* qn, const float* kn, float* gq,
-                  float* gk, float* gv, long ldx, float* ga, float* gb, long ldg, int B, int T, int H, int dh,
-                  hipStream_t st);
+                  const float* beta, const void* d_o, const DeltaWs& ws, float* scratch, const float* qn,
+                  const float* kn, float* gq, float* gk, float* gv, long ldx, float* ga, float* gb, long ldg, int B,
+                  int T, int H, int dh, hipStream_t st);
 // Adds the cs column splits' partial dq, dk (part_x: [2][cs][rows][H dh]) and
 // dalpha, dbeta (part_g: [cs][rows][2H]) and, fused, applies the L2-norm and
 // sigmoid backward (delta.hip).

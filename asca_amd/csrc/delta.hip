@@ -1254,8 +1254,8 @@ static int launch_bwd(const float* q, const float* k, const float* v, const floa
                       hipStream_t st) {
     const int dhc = dh_class(dh);
     if (blocked(T, H, dh))
-        return launch_ut_bwd(FUSED, q, k, v, false, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx, ga, gb, ldg, B, T, H,
-                             dh, st);
+        return launch_ut_bwd(FUSED, q, k, v, false, alpha, beta, d_o, ws, nullptr, qn, kn, gq, gk, gv, ldx, ga, gb, ldg,
+                             B, T, H, dh, st);
 #define ASCA_BWD(DHC)                                                                                            \
     if (dhc == DHC)                                                                                              \
         return launch_bwd_t<DHC, FUSED>(q, k, v, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx, ga, gb, ldg, B,   \

@@ -28,10 +28,19 @@ int launch_ut_fwd(const void* q, const void* k, const void* v, bool bf, const fl
     return launch_ut_fwd_other(q, k, v, bf, al, alpha, beta, o, ws, B, T, H, dh, st);
 }
 
+// The gate sums of every block and, for column splits, their partial dq, dk, dalpha, dbeta.
+static size_t gate_sums(int B, int T, int H, int dh) {
+    return ut_bwd_scratch_floats((long)B * H * ut_col_splits(dh), (T + ut64::C - 1) / ut64::C);
+}
+size_t ut_bwd_scratch(int B, int T, int H, int dh) {
+    const size_t vs = ut_col_splits(dh), rows = (size_t)B * T;
+    return gate_sums(B, T, H, dh) + (vs > 1 ? vs * 2 * rows * ((size_t)H * dh + H) : 0);
+}
+
 int launch_ut_bwd(bool fused, const void* q, const void* k, const void* v, bool bf, const float* alpha,
-                  const float* beta, const void* d_o, const DeltaWs& ws, const float* qn, const float* kn, float* gq,
-                  float* gk, float* gv, long ldx, float* ga, float* gb, long ldg, int B, int T, int H, int dh,
-                  hipStream_t st) {
+                  const float* beta, const void* d_o, const DeltaWs& ws, float* scratch, const float* qn,
+                  const float* kn, float* gq, float* gk, float* gv, long ldx, float* ga, float* gb, long ldg, int B,
+                  int T, int H, int dh, hipStream_t st) {
     if (!ws.rec) return fail(ASCA_ERR_INVALID, "ut_bwd: workspace layout mismatch");
     if (!ut_fits(T, H, dh, max(ldx, ldg)))
         return fail(ASCA_ERR_UNSUPPORTED, "ut_bwd: one sequence's rows exceed 32-bit byte offsets");
@@ -42,17 +51,19 @@ int launch_ut_bwd(bool fused, const void* q, const void* k, const void* v, bool 
     a.NC = (T + ut64::C - 1) / ut64::C;
     a.x_vs = a.g_vs = 0;
     a.vs = 0;
-    // scratch of this call on its stream (the forward's workspace is only read):
-    // the gate sums, and for column splits their partial dq, dk, dalpha, dbeta
+    // a caller that lends the forward's workspace only for reading gives no scratch
     const int vs = ut_col_splits(dh);
-    const size_t rows = (size_t)B * T, n = rows * a.d, gs = ut_bwd_scratch_floats((long)B * H * vs, a.NC);
+    const size_t rows = (size_t)B * T, n = rows * a.d, gs = gate_sums(B, T, H, dh);
     StreamScratch sc;
-    int rc = sc.get(gs + (vs > 1 ? vs * (2 * n + rows * 2 * H) : 0), st);
-    if (rc) return rc;
-    a.gsc = sc.ws.p;
+    int rc = ASCA_OK;
+    if (!scratch) {
+        if ((rc = sc.get(ut_bwd_scratch(B, T, H, dh), st))) return rc;
+        scratch = sc.ws.p;
+    }
+    a.gsc = scratch;
     float *px = nullptr, *pg = nullptr;
     if (vs > 1) {
-        px = sc.ws.p + gs;
+        px = scratch + gs;
         pg = px + 2 * vs * n;
         a.gq = px;
         a.gk = px + vs * n;

@@ -393,8 +393,8 @@ ASCA_API int asca_moe_bwd(const float* xn, const float* w1, const float* w2, con
  *   q, k, v, d_o : (B*T, H*dh) bf16 (raw 16-bit patterns); alpha, beta : (B*T, H) f32
  *   o, dq, dk, dv : (B*T, H*dh) f32; dalpha, dbeta : (B*T, H) f32 (raw, not logits)
  *   1 <= C <= 64; dh a multiple of 4, at most 256.
- *   ws : asca_chunk_ws_bytes bytes; the forward leaves in it what the backward
- *   needs: call asca_chunk_bwd with the forward's ws and the same q, k, v (the
+ *   ws : asca_chunk_ws_bytes bytes, all that either call takes; the forward leaves
+ *   in it what the backward needs, and the backward writes to it: call asca_chunk_bwd with the forward's ws and the same q, k, v (the
  *   backward reads the bf16 inputs, as the reference's backward keeps q, k, v
  *   resident in DeltaDev, rust/src/cuda/mod.rs:1386-1397). */
 ASCA_API int asca_chunk_ws_bytes(int B, int T, int H, int dh, int C, size_t* bytes);

@@ -99,3 +99,50 @@ def test_split_k_partials_never_exceed_the_static_scratch():
                         worst = max(worst, wsb.value)
     print(f"[noalloc] largest split-K partials {worst} B of {SCRATCH_BYTES}", flush=True)
     assert 0 < worst <= SCRATCH_BYTES
+
+
+@pytest.mark.parametrize("B,T,H,dh,C_", [(2, 500, 4, 128, 32), (4, 300, 4, 96, 64), (4, 1000, 8, 64, 64), (3, 50, 2, 48, 64),
+                                         (1, 17, 1, 16, 16), (2, 100, 2, 32, 32), (2, 200, 2, 128, 64), (2, 60, 2, 24, 32)])
+def test_chunked_calls_take_their_workspace_and_nothing_else(g, B, T, H, dh, C_):
+    """asca_chunk_fwd and _bwd on a new stream: the device's free memory stays as it
+    is, the bytes behind the workspace too, and a second backward gives the same."""
+    from asca_amd import _lib
+    from asca_amd.gpu import DevBuf, _vp
+
+    rng = np.random.default_rng(dh + T)
+    rows, d = B * T, H * dh
+    bf = lambda a: (np.ascontiguousarray(a, np.float32).view(np.uint32) >> 16).astype(np.uint16)
+    q, k, v, do = (DevBuf.from_host(bf(rng.standard_normal((rows, d)) / np.sqrt(dh))) for _ in range(4))
+    al, be = (DevBuf.from_host(rng.uniform(0.1, 0.9, (rows, H)).astype(np.float32)) for _ in range(2))
+    wsb = C.c_size_t()
+    _lib.call("asca_chunk_ws_bytes", B, T, H, dh, C_, C.byref(wsb))
+    ws = DevBuf(wsb.value + 4096)
+    guard = np.arange(1024, dtype=np.uint32)
+    _lib.call("asca_h2d", C.c_void_p(ws.ptr + wsb.value), guard.ctypes.data_as(C.c_void_p), 4096)
+    outs = [DevBuf(rows * d * 4) for _ in range(4)] + [DevBuf(rows * H * 4) for _ in range(2)]
+    shapes = [(rows, d)] * 4 + [(rows, H)] * 2
+
+    def both(st, fwd, b=B, t=T):
+        if fwd:
+            _lib.call("asca_chunk_fwd", _vp(q), _vp(k), _vp(v), _vp(al), _vp(be), _vp(outs[0]), _vp(ws), b, t, H, dh, C_, st)
+        _lib.call("asca_chunk_bwd", _vp(q), _vp(k), _vp(v), _vp(do), _vp(ws), *[_vp(o) for o in outs[1:]], b, t, H, dh,
+                  C_, st)
+        _lib.call("asca_stream_sync", st)
+        return [o.to_host(s) for o, s in zip(outs, shapes)]
+
+    _lib.call("asca_pool_release")
+    sp = C.c_void_p()
+    _lib.call("asca_stream_create", C.byref(sp))
+    both(sp, True, 1, 1)  # code objects loaded, the stream's hardware queue set up
+    before = _hip_free_bytes()
+    first = both(sp, True)
+    print(f"[no alloc] chunk dh={dh} C={C_} ws {wsb.value} B, free {before} -> {_hip_free_bytes()}", flush=True)
+    assert _hip_free_bytes() == before
+    for a, b in zip(first, both(sp, False)):
+        np.testing.assert_array_equal(a, b)
+    _lib.call("asca_stream_destroy", sp)
+    got = np.zeros(1024, np.uint32)
+    _lib.call("asca_d2h", got.ctypes.data_as(C.c_void_p), C.c_void_p(ws.ptr + wsb.value), 4096)
+    np.testing.assert_array_equal(got, guard)
+    for b in (q, k, v, do, al, be, ws, *outs):
+        b.free()
