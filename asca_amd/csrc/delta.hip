@@ -1126,8 +1126,10 @@ static DeltaWs ws_layout(int B, int T, int H, int dh, void* base) {
     const DeltaWs g = layout(B, T, H, dh, ck_for(dhc), col_split(B, H, dhc), (size_t)T, 0, base);
     if (!blocked(T, H, dh)) return g;
     DeltaWs w = ut_ws_layout(B, T, H, dh, base);
-    // the size callers know for these widths, where the blocked form needs less
-    if (dh != 64) w.bytes = max(w.bytes, g.bytes);
+    // the size callers know for the narrow widths, where the blocked form needs less
+    // (at dh = 128 a tenth: 5.9 floats per element of q instead of 65, which leaves the
+    // column splits' backward room for twice the partials it took)
+    if (dh < 64) w.bytes = max(w.bytes, g.bytes);
     return w;
 }
 

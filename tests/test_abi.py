@@ -113,6 +113,23 @@ def test_workspace_bytes_layout():
     assert ei.value.code == 3
 
 
+@pytest.mark.parametrize("dh", [16, 32, 48, 64, 96, 128])
+@pytest.mark.parametrize("B,T,H", [(8, 1000, 8), (1, 4096, 16), (40, 128, 8)])
+def test_workspace_and_scratch_of_a_backward_are_bounded(B, T, H, dh):
+    # The blocked widths' workspace and scratch together, in floats per element of q:
+    # the u rows, checkpoints and records, the gate sums, and above dh = 64 the
+    # partials of the dh / 32 column splits (the per-step kernels took 53 and 69 there,
+    # 7 to 11 at the narrow widths).
+    from asca_amd import _lib
+
+    out = C.c_size_t()
+    _lib.call("asca_delta_ws_bytes", B, T, H, dh, C.byref(out))
+    S = dh // 32 if dh > 64 else 1
+    scratch = B * H * S * -(-T // 16) * 768 + (2 * S * B * T * H * (dh + 1) if S > 1 else 0)
+    per = (out.value / 4 + scratch) / (B * T * H * dh)
+    assert per <= {16: 10.0, 32: 7.0, 48: 9.0, 64: 6.0, 96: 14.0, 128: 17.0}[dh], per
+
+
 def test_product_rng_equals_oracle_rng(orc):
     from asca_amd import _lib
 
