@@ -47,7 +47,8 @@ struct Ws {
 // reference's operators take none): each stream has one cached device buffer
 // (from the library's stream-ordered pool, grown when a call needs more, the
 // old one freed behind the work queued on that stream), so work on one stream
-// uses it in stream order and calls on different streams never share it.
+// uses it in stream order and calls on different streams never share it.  One that
+// a captured call used stays until the process ends, as its graph can be replayed.
 // get() holds a library lock until release() (or the destructor), so two host
 // threads enqueueing on one stream do not interleave a grow with a launch.
 struct StreamScratch {

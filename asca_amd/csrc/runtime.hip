@@ -102,9 +102,12 @@ static hipMemPool_t g_scratch_pool = nullptr;
 struct ScratchEntry {
     float* p = nullptr;
     size_t floats = 0;
+    bool in_graph = false;  // a captured launch reads or writes p
 };
 static std::mutex g_scratch_mu;
 static std::unordered_map<hipStream_t, ScratchEntry> g_scratch;
+// buffers outgrown during a capture, which cannot free them: freed with the stream
+static std::unordered_map<hipStream_t, std::vector<float*>> g_retired;
 
 int StreamScratch::get(size_t floats, hipStream_t st) {
     ws = Ws{nullptr, 0};
@@ -113,19 +116,37 @@ int StreamScratch::get(size_t floats, hipStream_t st) {
     g_scratch_mu.lock();
     held_ = true;
     ScratchEntry& en = g_scratch[st];
+    // A stream that is being captured: what its graph uses has to stay where it is
+    // for every replay, so it is never freed, and a stream-ordered allocation would
+    // belong to the graph.
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &status) != hipSuccess) (void)hipGetLastError();
+    const bool capturing = status == hipStreamCaptureStatusActive;
     if (en.floats < floats) {
-        if (en.p) (void)hipFreeAsync(en.p, st);   // behind the queued work that still uses it
-        en = ScratchEntry{};
         const size_t want = floats + floats / 4;  // headroom for slightly larger calls
         void* p = nullptr;
-        hipError_t e = hipMallocFromPoolAsync(&p, want * sizeof(float), g_scratch_pool, st);
+        hipError_t e;
+        if (capturing) {
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+            e = hipThreadExchangeStreamCaptureMode(&mode);
+            if (e == hipSuccess) {
+                e = hipMalloc(&p, want * sizeof(float));
+                (void)hipThreadExchangeStreamCaptureMode(&mode);
+            }
+        } else {
+            if (en.p && !en.in_graph) (void)hipFreeAsync(en.p, st);   // behind the queued work that still uses it
+            en = ScratchEntry{};
+            e = hipMallocFromPoolAsync(&p, want * sizeof(float), g_scratch_pool, st);
+        }
         if (e != hipSuccess) {
             held_ = false;
             g_scratch_mu.unlock();
-            return fail(ASCA_ERR_OOM, "hipMallocFromPoolAsync(%zu): %s", want * sizeof(float), hipGetErrorString(e));
+            return fail(ASCA_ERR_OOM, "%zu bytes of scratch: %s", want * sizeof(float), hipGetErrorString(e));
         }
+        if (capturing && en.p && !en.in_graph) g_retired[st].push_back(en.p);
         en = ScratchEntry{reinterpret_cast<float*>(p), want};
     }
+    en.in_graph = en.in_graph || capturing;
     ws = Ws{en.p, floats};
     return ASCA_OK;
 }
@@ -143,9 +164,14 @@ StreamScratch::~StreamScratch() { (void)release(nullptr); }
 
 void stream_scratch_forget(hipStream_t st) {
     std::lock_guard<std::mutex> lk(g_scratch_mu);
+    auto old = g_retired.find(st);
+    if (old != g_retired.end()) {
+        for (float* p : old->second) (void)hipFreeAsync(p, st);
+        g_retired.erase(old);
+    }
     auto it = g_scratch.find(st);
     if (it == g_scratch.end()) return;
-    if (it->second.p) (void)hipFreeAsync(it->second.p, st);
+    if (it->second.p && !it->second.in_graph) (void)hipFreeAsync(it->second.p, st);  // (a graph can outlive its stream)
     g_scratch.erase(it);
 }
 

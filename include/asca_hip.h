@@ -147,7 +147,8 @@ ASCA_API void asca_rng_normal(uint64_t* state, float* out, size_t n, float scale
  * read it, so several backwards may use one forward's workspace at once; what a
  * backward itself needs beside it comes from the scratch that the library keeps
  * for each stream (grown by the first call that needs more, with a quarter to
- * spare): at the blocked widths B*H*S*ceil(T/16)*768 floats, and above dh = 64
+ * spare; a captured call's stays until the process ends, for its replays, which
+ * must not run beside other calls on that stream): at the blocked widths B*H*S*ceil(T/16)*768 floats, and above dh = 64
  * 2*S*B*T*H*(dh + 1) more, S = dh/32 (else 1); at other widths
  * 4*B*T*H*(dh + 1) where B*H <= 128 or dh > 64, else none. */
 ASCA_API int asca_delta_ws_bytes(int B, int T, int H, int dh, size_t* bytes);

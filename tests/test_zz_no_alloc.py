@@ -146,3 +146,68 @@ def test_chunked_calls_take_their_workspace_and_nothing_else(g, B, T, H, dh, C_)
     np.testing.assert_array_equal(got, guard)
     for b in (q, k, v, do, al, be, ws, *outs):
         b.free()
+
+
+@pytest.mark.parametrize("what", ["delta dh32", "delta dh128", "gemm"])
+def test_captured_calls_keep_their_scratch(g, what):
+    """A call captured as the first one on its stream: its replays give the eager
+    call's results, also after larger calls on that stream have grown its scratch."""
+    from asca_amd import _lib
+    from asca_amd.gpu import DevBuf, _vp
+
+    hip = C.CDLL("libamdhip64.so.7")
+    ok = lambda rc: None if rc == 0 else pytest.fail(f"HIP error {rc}")
+    rng = np.random.default_rng(5)
+    f32 = lambda *s: DevBuf.from_host(rng.standard_normal(s).astype(np.float32))
+    bufs = []
+
+    def call(big):
+        if what == "gemm":  # split K
+            M, N, K = (512, 1536, 16384) if big else (256, 256, 8192)
+            A, Bm, o = f32(K, M), f32(K, N), DevBuf(M * N * 4)
+            bufs.extend([A, Bm, o])
+            return (lambda st: _lib.call("asca_gemm", 1, 0, M, N, K, 1.0, _vp(A), M, _vp(Bm), N, 0.0, _vp(o), N, None, st),
+                    [(o, (M, N))])
+        dh = int(what[8:])
+        B, T, H = (17, 80, 8) if big else (17, 40, 8)  # more than 128 units
+        rows, d = B * T, H * dh
+        q, k, v, do = (f32(rows, d) for _ in range(4))
+        al, be = (DevBuf.from_host(rng.uniform(0.1, 0.9, (rows, H)).astype(np.float32)) for _ in range(2))
+        for x in (q, k):
+            h = x.to_host((rows, H, dh))
+            x.upload(h / np.linalg.norm(h, axis=2, keepdims=True))
+        wsb = C.c_size_t()
+        _lib.call("asca_delta_ws_bytes", B, T, H, dh, C.byref(wsb))
+        ws, o = DevBuf(wsb.value), DevBuf(rows * d * 4)
+        outs = [(DevBuf(rows * d * 4), (rows, d)) for _ in range(3)] + [(DevBuf(rows * H * 4), (rows, H)) for _ in range(2)]
+        bufs.extend([q, k, v, do, al, be, ws, o, *(x for x, _ in outs)])
+        _lib.call("asca_delta_fwd", _vp(q), _vp(k), _vp(v), _vp(al), _vp(be), _vp(o), _vp(ws), B, T, H, dh, None)
+        _lib.call("asca_sync")
+        return (lambda st: _lib.call("asca_delta_bwd_raw", _vp(q), _vp(k), _vp(v), _vp(al), _vp(be), _vp(do), _vp(ws),
+                                     *[_vp(x) for x, _ in outs], B, T, H, dh, st), outs)
+
+    run, outs = call(False)
+    larger, _ = call(True)
+    run(None)
+    _lib.call("asca_sync")
+    want = [x.to_host(s) for x, s in outs]
+    sp, graph, exe = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    _lib.call("asca_stream_create", C.byref(sp))
+    ok(hip.hipStreamBeginCapture(sp, 0))
+    run(sp)
+    ok(hip.hipStreamEndCapture(sp, C.byref(graph)))
+    ok(hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)))
+    for i in range(4):
+        for x, s in outs:
+            _lib.call("asca_memset32", _vp(x), 0x7fc00000, int(np.prod(s)), sp)
+        ok(hip.hipGraphLaunch(exe, sp))
+        _lib.call("asca_stream_sync", sp)
+        for (x, s), w in zip(outs, want):
+            np.testing.assert_array_equal(x.to_host(s), w)
+        larger(sp)
+        _lib.call("asca_stream_sync", sp)
+    ok(hip.hipGraphExecDestroy(exe))
+    ok(hip.hipGraphDestroy(graph))
+    _lib.call("asca_stream_destroy", sp)
+    for b in bufs:
+        b.free()
