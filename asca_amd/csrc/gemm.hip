@@ -138,7 +138,8 @@ ASCA_DEV void frag_read(float (&f)[4][4], const float* t, int w0, int h, int lan
 // rounded to nearest; a bf16 holds 8 bits, so the three hold all 24 of x and
 // both subtractions are exact).  A product of two splits is six bf16 products
 // (x2 y0, x0 y2, x1 y1, x1 y0, x0 y1, x0 y0), each exact in f32 and summed in
-// the f32 accumulator; the three left out are below 2^-25 of x y.  Six
+// the f32 accumulator; the three left out come to at most 2^-24 of x y (x1 y2 and x2
+// y1 a half each), over many products to 6e-9 of their sum.  Six
 // v_mfma_f32_16x16x32_bf16 take 96 cycles where eight
 // v_mfma_f32_16x16x4_f32 take 256 (and those hold the SIMD's VALU besides),
 // and a sum is rounded 6 times per 32 terms instead of 8 times.
@@ -154,8 +155,8 @@ ASCA_DEV void frag_read(float (&f)[4][4], const float* t, int w0, int h, int lan
 // In the large tiles that cost 3% (the sums negated every four k-tiles), signs by a row's
 // values instead of its place 1 to 5% (routed FFN 777 -> 815 us).
 //
-// The bf16 MFMA takes subnormal inputs as zero, and x1 and x2 lie up to 2^9 and
-// 2^17 below x: unscaled, operands below 2^-110 lost them (a product of rows at
+// The bf16 MFMA takes subnormal inputs as zero, and x1 and x2 hold the bits of x down
+// to 2^-23 of it: unscaled, operands below 2^-110 lost them (a product of rows at
 // 2^-120 had an error of 3.5e-5, at 2^-128 9e-3).  So both operands are split as
 // 2^24 x, where the smallest subnormal float is a normal bf16, and the sums are
 // scaled back by 2^-48: the same bits where nothing under- or overflows.  The
@@ -507,11 +508,10 @@ ASCA_DEV bool split_bad(const f32x4 (&acc)[NX][NY]) {
 // split and stored to LDS one step ahead.  DB: two LDS stages and one barrier
 // per step (146 KB for 128 x 256, one block per CU); otherwise one stage and
 // two barriers (49 KB for 128 x 128), the CU's other block filling the waits.
-// Bound: power.  At 4096^3 the 128 x 256 tile runs 225 TFLOP/s (f32 products on
+// Bound: power.  At 4096^3 the 128 x 256 tile runs 225 to 232 TFLOP/s (f32 products on
 // the same shape: 139), 1350 TFLOP/s of bf16 products, and 258 on operands of
 // zeros; a plain bf16 product of torch runs 1130 there.  16384x1536x512
-// 208 -> 140 us, its input gradient 210 -> 126, its weight gradient 218 -> 143.
-// (all before the operands' scaling, which costs 1 to 2%)
+// 208 -> 143 us, its input gradient 210 -> 124, its weight gradient 218 -> 133.
 template <bool TA, bool TB, int GATHER, int WM, int WN, bool DB>
 ASCA_DEV void split_mainloop(f32x4 (&acc)[4][4], const float* A, const float* B, const GemmArgs& p, long a_off,
                              long b_off, int m0, int n0, int lim_m, int lim_n, long K_lo, long K_hi, int tid,

@@ -57,8 +57,9 @@ constexpr int C = 16;          // steps per block; a checkpoint every 2 C steps
 // added by delta_combine_k.  Bound: the chain of blocks (forward 1.4-1.9 us, backward
 // 2-6 us per 16 steps from dh = 16 to 128); the per-step kernels these replaced
 // walked the steps one by one: forward and fused backward of B8 T1000 H8 dh128
-// 2627 -> 519 us, B4 T128 H4 dh32 76 -> 32, B32 T512 H8 dh48 667 -> 160, B32 T512
-// H8 dh96 7424 -> 680.
+// 2627 -> 534 us, B4 T128 H4 dh32 76 -> 33, B32 T512 H8 dh48 667 -> 171, B32 T512
+// H8 dh96 7424 -> 700.  Each width is ten kernels with a register allocation of its
+// own to look after; 80 and 112 and the widths between have not been made.
 template <int NR_, int NV_, int NH_>
 struct Dim {
     static constexpr int NR = NR_, NV = NV_, NH = NH_;

@@ -325,7 +325,13 @@ ASCA_API int asca_bucket_keys(const uint32_t* keys, int n, int n_buckets, int32_
  * tiles to fill the device, K is split and the partial products are summed in
  * a fixed order; the partials live in stream-ordered scratch on `stream`
  * (hipMallocAsync / hipFreeAsync), so calls on different streams never share
- * them. */
+ * them.
+ * The products run as sums of bf16 products of three-way split operands, with
+ * the error of f32 sums or less.  Equal rows of A give equal rows of C in
+ * products that do not fill the device (a batch being decoded); in larger ones
+ * a row's last bits depend on its place.  Infinities, NaN and values from 2^104
+ * come out as f32 products give them; a product with such sums takes up to 6
+ * times as long. */
 ASCA_API int asca_gemm(int trans_a, int trans_b, int M, int N, int K, float alpha, const float* A, long lda,
                        const float* B, long ldb, float beta, float* C, long ldc, const float* bias,
                        void* stream);
