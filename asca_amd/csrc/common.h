@@ -99,11 +99,17 @@ ASCA_DEV Rsrc make_rsrc(const void* p, unsigned bytes) {
 ASCA_DEV void buf_store1(Rsrc r, unsigned off, float x, unsigned soff = 0) {
     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), r, (int)off, (int)soff, 0);
 }
-// 16 bytes at byte offset off + soff (the whole store is dropped past the resource's size)
+// 16 bytes at byte offset off + soff (the whole store is dropped past the resource's size).
+// The sum goes into the vector offset, not the store's SGPR offset: the compiler takes a
+// store with an SGPR offset to have read its data registers when the next instruction
+// issues, and leaves out the two wait states that it keeps before their reuse otherwise.
+// They are needed: in the forward of the blocked delta rule at dh = 16,
+//   buffer_store_dwordx4 v[82:85], v33, s[8:11], s2 offen / v_mul_f32 v82, ...
+// now and then stored the new v82 for lanes 12 .. 15 of each 16 (some 10 units of 8192).
 ASCA_DEV void buf_store4(Rsrc r, unsigned off, float4 x, unsigned soff = 0) {
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
     const u32x4 v = {__float_as_uint(x.x), __float_as_uint(x.y), __float_as_uint(x.z), __float_as_uint(x.w)};
-    __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)off, (int)soff, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)(off + soff), 0, 0);
 }
 // Buffer loads at byte offset voff + soff (soff uniform: an SGPR, so a loop's
 // per-lane offset is computed once and a block's offset costs no VALU); past

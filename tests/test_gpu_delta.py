@@ -454,3 +454,58 @@ def test_blocked_widths_are_as_exact_as_the_steps(orc, g, dh):
     off = np.sqrt(sum(np.sum((y - r) ** 2) for y, r in zip(got, ref)) / sum(np.sum(r ** 2) for r in ref))
     print(f"[delta float64] dh={dh} {off:.3e}", [f"{np.linalg.norm(y - r) / np.linalg.norm(r):.2e}" for y, r in zip(got, ref)], flush=True)
     assert off <= 1.33e-7, off
+
+
+def _placed_parity(orc, dh, B, T, H, off, repeats=1):
+    """Forward, raw and fused gradients of rows `off` floats past their alignment against
+    the oracle, and the same bits in every repeat."""
+    import ctypes as C
+    from asca_amd import _lib
+    from asca_amd.gpu import DevBuf, _vp
+
+    x = orc.DeltaInputs(dh + T, B, T, H, dh)
+    x.alpha[np.arange(B * T) % 5 == 3] = 0.0
+    o_ref, dq, dk, dv, da, db = orc.delta_fwd_bwd(x.q, x.k, x.v, x.alpha, x.beta, x.d_o, B, T, H, dh)
+    d_qkv_ref, d_gate_ref = orc.delta_fuse(x.q, x.k, x.qn, x.kn, x.alpha, x.beta, dq, dk, dv, da, db, H, dh)
+    rows, d = B * T, H * dh
+    bufs = []
+
+    def placed(a):
+        bufs.append(DevBuf((a.size + off) * 4))
+        bufs[-1].upload(np.concatenate([np.zeros(off, np.float32), a.ravel()]))
+        return _vp(bufs[-1].ptr + 4 * off)
+
+    q, k, v, al, be, qn, kn, do = (placed(getattr(x, n)) for n in
+                                   ("q", "k", "v", "alpha", "beta", "qn", "kn", "d_o"))
+    wsb = C.c_size_t()
+    _lib.call("asca_delta_ws_bytes", B, T, H, dh, C.byref(wsb))
+    bufs.append(DevBuf(wsb.value))
+    ws = _vp(bufs[-1].ptr)
+    shapes = [(rows, d)] * 4 + [(rows, H)] * 2 + [(rows, 3 * d), (rows, 2 * H)]
+    first = None
+    for _ in range(repeats):
+        outs = [DevBuf(int(np.prod(s)) * 4) for s in shapes]
+        p = [_vp(b.ptr) for b in outs]
+        _lib.call("asca_delta_fwd", q, k, v, al, be, p[0], ws, B, T, H, dh, None)
+        _lib.call("asca_delta_bwd_raw", q, k, v, al, be, do, ws, *p[1:6], B, T, H, dh, None)
+        _lib.call("asca_delta_bwd_fused", q, k, v, al, be, qn, kn, do, ws, *p[6:], B, T, H, dh, None)
+        _lib.call("asca_sync")
+        got = [b.to_host(s) for b, s in zip(outs, shapes)]
+        for b in outs:
+            b.free()
+        for a, ref, tol in zip(got, (o_ref, dq, dk, dv, da, db, d_qkv_ref, d_gate_ref), [FWD_TOL] + [GRAD_TOL] * 7):
+            assert np.max(np.abs(a - ref)) <= tol * max(np.max(np.abs(ref)), 1e-30)
+        first = first or got
+        assert all(np.array_equal(a, b) for a, b in zip(got, first))
+    for b in bufs:
+        b.free()
+
+
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("dh,B,T,H", [(16, 512, 41, 8), (16, 512, 48, 8), (32, 256, 41, 8), (64, 128, 41, 8),
+                                      (96, 64, 41, 8), (128, 64, 41, 8)])
+def test_checkpoints_of_many_units(orc, g, dh, B, T, H, off):
+    # The states that the forward leaves for the backward, the last one before a block
+    # that is not whole: enough units that a store whose registers are overwritten
+    # before it has read them shows (at dh = 16 it did, in each of some twenty calls).
+    _placed_parity(orc, dh, B, T, H, off, repeats=3)
