@@ -7,7 +7,8 @@
 //
 // Design (MI355X-first, not a translation of rust/kernels/asca.cu):
 // These kernels take the head widths that the blocked form on the matrix cores
-// (ut64_kernels.h: 16, 32, 48, 64, 96 and 128) does not.
+// (ut64_kernels.h: 16, 32, 48, 64, 96 and 128) does not, and sequences too short for
+// its blocks of 16 steps (short_steps).
 //  * Column i of S only ever meets k, q, alpha, beta and its own v_i, sk_i, u_i,
 //    so the forward splits each (sequence, head) unit into dh/8 waves of 8 value
 //    columns that never talk to each other (two waves per SIMD at dh = 64).
@@ -56,16 +57,21 @@ ASCA_DEV float4* trash_f4(int i) { return g_trash4 + (i & 1023); }
 ASCA_DEV float readlane_f(float x, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l)); }
 
 // Masked vector helpers: invalid elements read 0 from a valid address.
+template <bool EXACT>
 ASCA_DEV float4 ld4m(const float* __restrict__ p, int col, int dh) {
-    float4 r;
-    float* rr = reinterpret_cast<float*>(&r);
+    if constexpr (EXACT) {
+        return *reinterpret_cast<const float4*>(p + col);
+    } else {
+        float4 r;
+        float* rr = reinterpret_cast<float*>(&r);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const bool ok = col + e < dh;
-        const float x = p[ok ? col + e : 0];
-        rr[e] = ok ? x : 0.0f;
+        for (int e = 0; e < 4; ++e) {
+            const bool ok = col + e < dh;
+            const float x = p[ok ? col + e : 0];
+            rr[e] = ok ? x : 0.0f;
+        }
+        return r;
     }
-    return r;
 }
 
 // ------------------------------------------------------------------ forward
@@ -101,7 +107,7 @@ struct FwdStage {
 
 // Global -> registers for chunk c (steps c*CK .. c*CK+CK-1, clamped to T-1);
 // wg: the wave's index among all waves of the unit (its value columns).
-template <int DH, int CS>
+template <int DH, int CS, bool EXACT>
 ASCA_DEV void fwd_stage_load(FwdStage<DH, CS>& st, int c, const float* __restrict__ q, const float* __restrict__ k,
                              const float* __restrict__ v, long ubase, long d, int T, int dh, int wg, int lane) {
     using L = FS<DH, CS>;
@@ -115,7 +121,7 @@ ASCA_DEV void fwd_stage_load(FwdStage<DH, CS>& st, int c, const float* __restric
         const int fl = f - tsr * (L::KQ_F / 4);
         const int j = fl / (DH / 4), c4 = fl % (DH / 4);
         const long t = min(t0 + j, T - 1);
-        st.kq[i] = ld4m((tsr ? q : k) + ubase + t * d, 4 * c4, dh);
+        st.kq[i] = ld4m<EXACT>((tsr ? q : k) + ubase + t * d, 4 * c4, dh);
     }
 #pragma unroll
     for (int i = 0; i < L::NV; ++i) {
@@ -123,7 +129,7 @@ ASCA_DEV void fwd_stage_load(FwdStage<DH, CS>& st, int c, const float* __restric
         const int f = f0 < CK * 2 ? f0 : 0;
         const int j = f / 2, half = f % 2;
         const long t = min(t0 + j, T - 1);
-        st.v[i] = ld4m(v + ubase + t * d, wg * 8 + half * 4, dh);
+        st.v[i] = ld4m<EXACT>(v + ubase + t * d, wg * 8 + half * 4, dh);
     }
 }
 
@@ -232,11 +238,17 @@ ASCA_DEV void fwd_steps(float (&s)[DH / 8], const float* __restrict__ buf, float
 
 // A lane's rows row0 .. row0+R-1 of column col into a checkpoint slot (S^T,
 // contiguous per column); masked elements go to the trash.
-template <int R>
+template <int R, bool EXACT>
 ASCA_DEV void store_ckpt(float* __restrict__ dst, const float (&s)[R], bool col_ok, int row0, int dh,
                          float* __restrict__ tr) {
+    if constexpr (EXACT && R % 4 == 0) {
 #pragma unroll
-    for (int j = 0; j < R; ++j) *((col_ok && row0 + j < dh) ? dst + j : tr + j) = s[j];
+        for (int j = 0; j < R; j += 4)
+            *reinterpret_cast<float4*>(dst + j) = make_float4(s[j], s[j + 1], s[j + 2], s[j + 3]);
+    } else {
+#pragma unroll
+        for (int j = 0; j < R; ++j) *((col_ok && row0 + j < dh) ? dst + j : tr + j) = s[j];
+    }
 }
 
 // One block per (sequence, head) unit, unit = h*B + b (the reference's s_pre
@@ -244,7 +256,7 @@ ASCA_DEV void store_ckpt(float* __restrict__ dst, const float (&s)[R], bool col_
 // unit, slot j = S^T before step j*CK (element (a, i) of S at [i*dh + a]), the
 // last slot S^T after step T-1.  Steps past T (the tail of the last chunk) run
 // with alpha = 1, beta = 0, which leaves the state unchanged.
-template <int DH, int CS>
+template <int DH, int CS, bool EXACT>
 __global__ __launch_bounds__((FS<DH, CS>::NT)) void delta_fwd_k(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     const float* __restrict__ alpha, const float* __restrict__ beta, float* __restrict__ o,
@@ -269,7 +281,7 @@ __global__ __launch_bounds__((FS<DH, CS>::NT)) void delta_fwd_k(
     float* skb = sk_out + ubase;
     const long gbase = (long)b * T * H + h;
     float* ckb = ckpt + (long)unit * nslots * dh2;
-    const bool col_ok = col < dh;
+    const bool col_ok = EXACT || col < dh;
     float* const tr = trash_f(threadIdx.x * 2);
     const int nchunk = (T + CK - 1) / CK;
 
@@ -283,7 +295,7 @@ __global__ __launch_bounds__((FS<DH, CS>::NT)) void delta_fwd_k(
     for (int j = 0; j < R; ++j) s[j] = 0.0f;
 
     FwdStage<DH, CS> stg;
-    fwd_stage_load<DH, CS>(stg, 0, q, k, v, ubase, d, T, dh, wg, lane);
+    fwd_stage_load<DH, CS, EXACT>(stg, 0, q, k, v, ubase, d, T, dh, wg, lane);
     // a gate of step t (lane-dependent: alpha or beta); past T, alpha = 1 and beta = 0
     const float gpad = gl < CK ? 1.0f : 0.0f;
     auto gate = [&](int t) {
@@ -299,8 +311,8 @@ __global__ __launch_bounds__((FS<DH, CS>::NT)) void delta_fwd_k(
         const float* buf = lds + (ci & 1) * L::BUF_F;
         const float gcur = gnext;
         gnext = gate(t0 + CK + gstep);
-        fwd_stage_load<DH, CS>(stg, min(ci + 1, nchunk - 1), q, k, v, ubase, d, T, dh, wg, lane);
-        store_ckpt<R>(ckb + (long)ci * dh2 + (long)col * dh + row0, s, col_ok, row0, dh, tr);
+        fwd_stage_load<DH, CS, EXACT>(stg, min(ci + 1, nchunk - 1), q, k, v, ubase, d, T, dh, wg, lane);
+        store_ckpt<R, EXACT>(ckb + (long)ci * dh2 + (long)col * dh + row0, s, col_ok, row0, dh, tr);
         // Lanes j < CK of gcur hold the chunk's alpha; when all of them lie in
         // [2^-8, 2^8] the chunk runs on the scaled state (fwd_steps).
         const bool bad = lane < CK && !(gcur >= 0x1p-8f && gcur <= 0x1p8f);
@@ -330,7 +342,7 @@ __global__ __launch_bounds__((FS<DH, CS>::NT)) void delta_fwd_k(
         fwd_stage_store<DH, CS>(stg, lds + ((ci + 1) & 1) * L::BUF_F, w, lane);
         lds_barrier();
     }
-    store_ckpt<R>(ckb + (long)nchunk * dh2 + (long)col * dh + row0, s, col_ok, row0, dh, tr);
+    store_ckpt<R, EXACT>(ckb + (long)nchunk * dh2 + (long)col * dh + row0, s, col_ok, row0, dh, tr);
 }
 
 // Full state history for download_states: S before every step then the final
@@ -432,7 +444,7 @@ struct BStage {
 };
 
 // wg: the wave's index among all waves of the unit (its value columns)
-template <int DH, int CS, bool FUSED>
+template <int DH, int CS, bool EXACT, bool FUSED>
 ASCA_DEV void bstage_load(BStage<DH, CS>& st, int g, const float* __restrict__ q, const float* __restrict__ k,
                           const float* __restrict__ v, const float* __restrict__ d_o,
                           const float* __restrict__ skv, const float* __restrict__ alpha,
@@ -450,7 +462,7 @@ ASCA_DEV void bstage_load(BStage<DH, CS>& st, int g, const float* __restrict__ q
         const int fl = f - tsr * S::QK4;
         const int j = fl / (DH / 4), c4 = fl % (DH / 4);
         const long t = min(t0 + j, T - 1);
-        st.rq[i] = ld4m((tsr ? k : q) + ubase + t * d, 4 * c4, dh);
+        st.rq[i] = ld4m<EXACT>((tsr ? k : q) + ubase + t * d, 4 * c4, dh);
     }
 #pragma unroll
     for (int i = 0; i < S::NW; ++i) {
@@ -461,7 +473,7 @@ ASCA_DEV void bstage_load(BStage<DH, CS>& st, int g, const float* __restrict__ q
         const int j = rem / 2, half = rem % 2;
         const long t = min(t0 + j, T - 1);
         const float* src = tsr == 0 ? d_o : (tsr == 1 ? v : skv);
-        st.rw[i] = ld4m(src + ubase + t * d, wg * 8 + half * 4, dh);
+        st.rw[i] = ld4m<EXACT>(src + ubase + t * d, wg * 8 + half * 4, dh);
     }
     {
         const int gl = lane & (2 * CK - 1);
@@ -473,11 +485,19 @@ ASCA_DEV void bstage_load(BStage<DH, CS>& st, int g, const float* __restrict__ q
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
         const int i = colb + n;
+        if constexpr (EXACT && M % 4 == 0) {
 #pragma unroll
-        for (int m = 0; m < M; ++m) {
-            const bool ok = i < dh && rowb + m < dh;
-            const float x = cks[ok ? (long)i * dh + rowb + m : 0];
-            st.rck[n][m] = ok ? x : 0.0f;
+            for (int m = 0; m < M; m += 4) {
+                const float4 x = *reinterpret_cast<const float4*>(cks + (long)i * dh + rowb + m);
+                st.rck[n][m] = x.x; st.rck[n][m + 1] = x.y; st.rck[n][m + 2] = x.z; st.rck[n][m + 3] = x.w;
+            }
+        } else {
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const bool ok = i < dh && rowb + m < dh;
+                const float x = cks[ok ? (long)i * dh + rowb + m : 0];
+                st.rck[n][m] = ok ? x : 0.0f;
+            }
         }
     }
 }
@@ -589,7 +609,7 @@ ASCA_DEV void bops_read(BOps<DH / 16>& o, const float* __restrict__ st_q, const 
 //     du~ = ds^T k = G_{j+1} du (one FMA per element), and every output term
 //     takes its scale from the step's gate-table row (g1 = G_{j+1}, r1 = 1/G_{j+1},
 //     ia = 1/alpha = G_j / G_{j+1}).
-template <int DH, bool SC>
+template <int DH, bool EXACT, bool SC>
 ASCA_DEV void bwd_step(const BOps<DH / 16>& in, const float (&sm)[DH / 16][2], const float (&sa)[DH / 16][2],
                        float (&ds)[DH / 16][2], float* __restrict__ rq, float* __restrict__ rk, float& pab_out,
                        float* __restrict__ rv, int rg, int cg,
@@ -700,7 +720,7 @@ ASCA_DEV void bwd_step(const BOps<DH / 16>& in, const float (&sm)[DH / 16][2], c
 // LDS buffer nbuf halfway, and reduce the per-step dalpha / dbeta partials.  With SC
 // the stash holds S / G_j and ds is carried as G_{j+1} dS inside the segment
 // (see bwd_step); ds enters and leaves unscaled.
-template <int DH, int CS, bool SC>
+template <int DH, int CS, bool EXACT, bool SC>
 ASCA_DEV void bwd_segment(const float (&s0)[DH / 16][2], float (&ds)[DH / 16][2], const BStage<DH, CS>& stg,
                           float* __restrict__ nbuf, float2* __restrict__ cks, const float* __restrict__ st_q,
                           const float* __restrict__ st_k, const float* __restrict__ st_w,
@@ -760,7 +780,7 @@ ASCA_DEV void bwd_segment(const float (&s0)[DH / 16][2], float (&ds)[DH / 16][2]
 #pragma unroll
     for (int jj = CK - 1; jj >= 0; --jj) {
         if (jj > 0) bops_read<DH>(op[(jj - 1) & 1], st_q, st_k, st_w, st_ab, jj - 1, w, rowb, cg);
-        bwd_step<DH, SC>(op[jj & 1], stash[jj], stash[jj + 1], ds, red_q + (jj * W + w) * DH,
+        bwd_step<DH, EXACT, SC>(op[jj & 1], stash[jj], stash[jj + 1], ds, red_q + (jj * W + w) * DH,
                                 red_k + (jj * W + w) * DH, pab[jj], red_v + jj * DH, rg, cg, rowb, colb, dh);
         if (jj == CK / 2) {
             // the staged operands of the next segment (loads issued at the
@@ -784,7 +804,7 @@ ASCA_DEV void bwd_segment(const float (&s0)[DH / 16][2], float (&ds)[DH / 16][2]
 // With CS = 2 the row sums dq, dk and dalpha, dbeta cover only the block's
 // columns: they go to the partial buffers (part_x [CS][B*T][H*dh], part_g
 // [CS][B*T][2H]) and delta_combine_k finishes them; dv is complete per column.
-template <int DH, int CS, bool FUSED>
+template <int DH, int CS, bool EXACT, bool FUSED>
 __global__ __launch_bounds__((BS<DH, CS>::NT)) void delta_bwd_k(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     const float* __restrict__ alpha, const float* __restrict__ beta, const float* __restrict__ d_o,
@@ -818,7 +838,7 @@ __global__ __launch_bounds__((BS<DH, CS>::NT)) void delta_bwd_k(
     for (int m = 0; m < M; ++m) ds[m][0] = ds[m][1] = 0.0f;
 
     BStage<DH, CS> stg;
-    bstage_load<DH, CS, FUSED>(stg, nseg - 1, q, k, v, d_o, skv, alpha, beta, qnorm, knorm, ckb, ubase,
+    bstage_load<DH, CS, EXACT, FUSED>(stg, nseg - 1, q, k, v, d_o, skv, alpha, beta, qnorm, knorm, ckb, ubase,
                                       gbase, d, dh2, T, H, dh, wg, lane, rowb, colb);
     {
         float* const b0 = lds + ((nseg - 1) & 1) * S::BUF_F + S::ST_OFF;
@@ -845,15 +865,15 @@ __global__ __launch_bounds__((BS<DH, CS>::NT)) void delta_bwd_k(
             s0[m][0] = x.x;
             s0[m][1] = x.y;
         }
-        bstage_load<DH, CS, FUSED>(stg, g > 0 ? g - 1 : 0, q, k, v, d_o, skv, alpha, beta, qnorm, knorm, ckb,
+        bstage_load<DH, CS, EXACT, FUSED>(stg, g > 0 ? g - 1 : 0, q, k, v, d_o, skv, alpha, beta, qnorm, knorm, ckb,
                                           ubase, gbase, d, dh2, T, H, dh, wg, lane, rowb, colb);
         lds_barrier();  // staging of this segment visible to all waves
 
         if (__builtin_amdgcn_readfirstlane(__float_as_int(st_ab[8 * CK])) == __float_as_int(1.0f))
-            bwd_segment<DH, CS, true>(s0, ds, stg, nbuf, cks, st_q, st_k, st_w, st_ab, red_q, red_k,
+            bwd_segment<DH, CS, EXACT, true>(s0, ds, stg, nbuf, cks, st_q, st_k, st_w, st_ab, red_q, red_k,
                                              red_ab, red_v, t0, T, w, lane, rg, cg, rowb, colb, dh);
         else
-            bwd_segment<DH, CS, false>(s0, ds, stg, nbuf, cks, st_q, st_k, st_w, st_ab, red_q, red_k,
+            bwd_segment<DH, CS, EXACT, false>(s0, ds, stg, nbuf, cks, st_q, st_k, st_w, st_ab, red_q, red_k,
                                               red_ab, red_v, t0, T, w, lane, rg, cg, rowb, colb, dh);
         lds_barrier();  // red_* of this segment complete
 
@@ -1116,15 +1136,38 @@ DeltaWs ut_ws_layout(int B, int T, int H, int dh, void* base) {
     return layout(B, T, H, dh, D64_CK, 1, blocks * D64_BLK, blocks * D64_REC, base);
 }
 
-// Shapes on the blocked form: its widths, but for sequences whose rows pass its
-// 32-bit offsets (dh = 64 has no other kernels and refuses those).  A function
-// of the shape only: forward and backward must agree.
-static bool blocked(int T, int H, int dh) { return ut_width(dh) && (dh == 64 || ut_fits(T, H, dh, 3L * H * dh)); }
+// Sequences of a few steps that the per-step kernels do faster, at the widths that
+// they have without masked rows: a block of 16 steps costs the blocked form its
+// whole latency and products whatever the sequence fills of it, and it records
+// what no second block reads.  Forward and fused backward, per-step / blocked (us):
+//   dh 128   64 units T4 21 / 24, T8 32 / 25;  256 units T4 41 / 78, T8 64 / 80, T12 85 / 82
+//   dh 32    128 units T8 15 / 15;  256 units T8 12 / 16, T12 16 / 16;  512 units T12 17 / 21,
+//            T24 24 / 27, T32 29 / 27;  4096 units T40 219 / 241, T48 268 / 249
+//   dh 16    256 units T8 13 / 14, T12 15 / 13;  1024 units T8 14 / 18, T16 18 / 17;
+//            2048 units T16 30 / 30, T24 41 / 47, T32 52 / 50;  8192 units T40 186 / 214,
+//            T48 225 / 228
+// (at 48 and 96, where rows are masked, the blocked form is the faster one from T = 1)
+static bool short_steps(int B, int T, int H, int dh) {
+    const long units = (long)B * H;
+    if (dh == 128) return T <= 4 || (T <= 8 && units >= 128);
+    if (dh != 16 && dh != 32) return false;
+    if (units * dh >= 8192 * 16) return T <= 40;
+    if (units >= (dh == 16 ? 2048 : 512)) return T <= 24;
+    return units >= 256 && T <= 8;
+}
+
+// Shapes on the blocked form: its widths, but for short sequences and for those
+// whose rows pass its 32-bit offsets (dh = 64 has no other kernels: it takes the
+// first and refuses the second).  A function of the shape only: forward and
+// backward must agree.
+static bool blocked(int B, int T, int H, int dh) {
+    return ut_width(dh) && (dh == 64 || (!short_steps(B, T, H, dh) && ut_fits(T, H, dh, 3L * H * dh)));
+}
 
 static DeltaWs ws_layout(int B, int T, int H, int dh, void* base) {
     const int dhc = dh_class(dh);
     const DeltaWs g = layout(B, T, H, dh, ck_for(dhc), col_split(B, H, dhc), (size_t)T, 0, base);
-    if (!blocked(T, H, dh)) return g;
+    if (!blocked(B, T, H, dh)) return g;
     DeltaWs w = ut_ws_layout(B, T, H, dh, base);
     // the size callers know for the narrow widths, where the blocked form needs less
     // (at dh = 128 a tenth: 5.9 floats per element of q instead of 65, which leaves the
@@ -1140,6 +1183,8 @@ static size_t part_floats(int cs, int B, int T, int H, int dh) {
     return (size_t)2 * cs * B * T * H * dh + (size_t)cs * B * T * 2 * H;
 }
 
+static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
 static int check_shape(int B, int T, int H, int dh) {
     if (B < 0 || T < 0 || H < 0) return fail(ASCA_ERR_INVALID, "negative shape B=%d T=%d H=%d", B, T, H);
     if (!dh_class(dh)) return fail(ASCA_ERR_UNSUPPORTED, "dh=%d outside 1..128", dh);
@@ -1147,16 +1192,16 @@ static int check_shape(int B, int T, int H, int dh) {
     return ASCA_OK;
 }
 
-template <int DH>
+template <int DH, bool EXACT>
 static int launch_fwd_t(const float* q, const float* k, const float* v, const float* alpha, const float* beta,
                         float* o, const DeltaWs& ws, int B, int T, int H, int dh, hipStream_t st) {
     int rc = pre_launch("delta_fwd");
     if (rc) return rc;
     if (DH == 128 || ws.cs > 1)
-        hipLaunchKernelGGL((delta_fwd_k<DH, 2>), dim3(B * H * 2), dim3(FS<DH, 2>::NT), 0, st, q, k, v, alpha,
+        hipLaunchKernelGGL((delta_fwd_k<DH, 2, EXACT>), dim3(B * H * 2), dim3(FS<DH, 2>::NT), 0, st, q, k, v, alpha,
                            beta, o, ws.sk, ws.ckpt, B, T, H, dh, ws.nslots);
     else if constexpr (DH < 128)  // dh = 128 always splits its columns
-        hipLaunchKernelGGL((delta_fwd_k<DH, 1>), dim3(B * H), dim3(FS<DH, 1>::NT), 0, st, q, k, v, alpha,
+        hipLaunchKernelGGL((delta_fwd_k<DH, 1, EXACT>), dim3(B * H), dim3(FS<DH, 1>::NT), 0, st, q, k, v, alpha,
                            beta, o, ws.sk, ws.ckpt, B, T, H, dh, ws.nslots);
     return post_launch("delta_fwd");
 }
@@ -1164,10 +1209,12 @@ static int launch_fwd_t(const float* q, const float* k, const float* v, const fl
 static int launch_fwd(const float* q, const float* k, const float* v, const float* alpha, const float* beta,
                       float* o, const DeltaWs& ws, int B, int T, int H, int dh, hipStream_t st) {
     const int dhc = dh_class(dh);
-    if (blocked(T, H, dh)) return launch_ut_fwd(q, k, v, false, alpha, beta, o, ws, B, T, H, dh, st);
+    const bool exact = dh == dhc && aligned16(q) && aligned16(k);
+    if (blocked(B, T, H, dh)) return launch_ut_fwd(q, k, v, false, alpha, beta, o, ws, B, T, H, dh, st);
 #define ASCA_FWD(DHC)                                                                                    \
     if (dhc == DHC)                                                                                      \
-        return launch_fwd_t<DHC>(q, k, v, alpha, beta, o, ws, B, T, H, dh, st);
+        return exact ? launch_fwd_t<DHC, true>(q, k, v, alpha, beta, o, ws, B, T, H, dh, st)             \
+                     : launch_fwd_t<DHC, false>(q, k, v, alpha, beta, o, ws, B, T, H, dh, st);
     ASCA_FWD(16)
     ASCA_FWD(32)
     ASCA_FWD(64)
@@ -1208,13 +1255,13 @@ int launch_delta_combine(bool fused, int cs, const float* part_x, const float* p
     return post_launch("delta_combine");
 }
 
-template <int DH, int CS, bool FUSED>
+template <int DH, int CS, bool EXACT, bool FUSED>
 static int launch_bwd_cs(const float* q, const float* k, const float* v, const float* alpha, const float* beta,
                          const float* d_o, const DeltaWs& ws, const float* qn, const float* kn, float* gq, float* gk,
                          float* gv, long ldx, float* ga, float* gb, long ldg, int B, int T, int H, int dh,
                          hipStream_t st) {
     const size_t lds = BS<DH, CS>::LDS;
-    if (int arc = allow_lds(reinterpret_cast<const void*>(&delta_bwd_k<DH, CS, FUSED>), lds)) return arc;
+    if (int arc = allow_lds(reinterpret_cast<const void*>(&delta_bwd_k<DH, CS, EXACT, FUSED>), lds)) return arc;
     int rc = pre_launch("delta_bwd");
     if (rc) return rc;
     // the column halves' partials: scratch of this call on its stream
@@ -1222,7 +1269,7 @@ static int launch_bwd_cs(const float* q, const float* k, const float* v, const f
     if ((rc = sc.get(part_floats(CS, B, T, H, dh), st))) return rc;
     float* part_x = sc.ws.p;
     float* part_g = CS > 1 ? part_x + (size_t)2 * CS * B * T * H * dh : nullptr;
-    hipLaunchKernelGGL((delta_bwd_k<DH, CS, FUSED>), dim3(B * H * CS), dim3(BS<DH, CS>::NT), lds, st, q, k,
+    hipLaunchKernelGGL((delta_bwd_k<DH, CS, EXACT, FUSED>), dim3(B * H * CS), dim3(BS<DH, CS>::NT), lds, st, q, k,
                        v, alpha, beta, d_o, ws.sk, ws.ckpt, qn, kn, gq, gk, gv, ldx, ga, gb, ldg, part_x, part_g, B,
                        T, H, dh, ws.nslots);
     if ((rc = post_launch("delta_bwd"))) {
@@ -1236,16 +1283,16 @@ static int launch_bwd_cs(const float* q, const float* k, const float* v, const f
     return rc ? rc : rr;
 }
 
-template <int DH, bool FUSED>
+template <int DH, bool EXACT, bool FUSED>
 static int launch_bwd_t(const float* q, const float* k, const float* v, const float* alpha, const float* beta,
                         const float* d_o, const DeltaWs& ws, const float* qn, const float* kn, float* gq, float* gk,
                         float* gv, long ldx, float* ga, float* gb, long ldg, int B, int T, int H, int dh,
                         hipStream_t st) {
     if (DH == 128 || ws.cs > 1)
-        return launch_bwd_cs<DH, 2, FUSED>(q, k, v, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx, ga, gb, ldg,
+        return launch_bwd_cs<DH, 2, EXACT, FUSED>(q, k, v, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx, ga, gb, ldg,
                                                   B, T, H, dh, st);
     if constexpr (DH == 128) return fail(ASCA_ERR_UNSUPPORTED, "dh=128 without column split");
-    else return launch_bwd_cs<DH, 1, FUSED>(q, k, v, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx, ga, gb, ldg, B,
+    else return launch_bwd_cs<DH, 1, EXACT, FUSED>(q, k, v, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx, ga, gb, ldg, B,
                                               T, H, dh, st);
 }
 
@@ -1255,13 +1302,17 @@ static int launch_bwd(const float* q, const float* k, const float* v, const floa
                       float* gv, long ldx, float* ga, float* gb, long ldg, int B, int T, int H, int dh,
                       hipStream_t st) {
     const int dhc = dh_class(dh);
-    if (blocked(T, H, dh))
+    const bool exact = dh == dhc && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(d_o) &&
+                       aligned16(gv) && ((ldx * 4) % 16 == 0);
+    if (blocked(B, T, H, dh))
         return launch_ut_bwd(FUSED, q, k, v, false, alpha, beta, d_o, ws, nullptr, qn, kn, gq, gk, gv, ldx, ga, gb, ldg,
                              B, T, H, dh, st);
 #define ASCA_BWD(DHC)                                                                                            \
     if (dhc == DHC)                                                                                              \
-        return launch_bwd_t<DHC, FUSED>(q, k, v, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx, ga, gb, ldg, B,   \
-                                        T, H, dh, st);
+        return exact ? launch_bwd_t<DHC, true, FUSED>(q, k, v, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx, ga, \
+                                                      gb, ldg, B, T, H, dh, st)                                  \
+                     : launch_bwd_t<DHC, false, FUSED>(q, k, v, alpha, beta, d_o, ws, qn, kn, gq, gk, gv, ldx,   \
+                                                       ga, gb, ldg, B, T, H, dh, st);
     ASCA_BWD(16)
     ASCA_BWD(32)
     ASCA_BWD(64)

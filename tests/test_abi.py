@@ -113,6 +113,18 @@ def test_workspace_bytes_layout():
     assert ei.value.code == 3
 
 
+@pytest.mark.parametrize("B,T,H,dh,C_", [(2048, 1, 8, 128, 2), (1, 4, 1, 128, 2), (256, 8, 1, 16, 8), (1024, 24, 1, 32, 8)])
+def test_short_sequences_keep_the_per_step_workspace(B, T, H, dh, C_):
+    # sk rows and a state every C steps plus the last one: what the per-step kernels
+    # leave, without the blocked ones' records of whole 16-step blocks
+    from asca_amd import _lib
+
+    out = C.c_size_t()
+    _lib.call("asca_delta_ws_bytes", B, T, H, dh, C.byref(out))
+    up = lambda n: (n + 255) // 256 * 256
+    assert out.value == up(B * T * H * dh * 4) + up(B * H * (-(-T // C_) + 1) * dh * dh * 4)
+
+
 @pytest.mark.parametrize("dh", [16, 32, 48, 64, 96, 128])
 @pytest.mark.parametrize("B,T,H", [(8, 1000, 8), (1, 4096, 16), (40, 128, 8)])
 def test_workspace_and_scratch_of_a_backward_are_bounded(B, T, H, dh):

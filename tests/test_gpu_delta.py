@@ -509,3 +509,15 @@ def test_checkpoints_of_many_units(orc, g, dh, B, T, H, off):
     # that is not whole: enough units that a store whose registers are overwritten
     # before it has read them shows (at dh = 16 it did, in each of some twenty calls).
     _placed_parity(orc, dh, B, T, H, off, repeats=3)
+
+
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("dh,B,T,H", [
+    (16, 255, 8, 1), (16, 32, 8, 8), (16, 32, 9, 8), (16, 256, 24, 8), (16, 256, 25, 8), (16, 1024, 40, 8),
+    (16, 1024, 41, 8), (16, 300, 1, 1), (32, 255, 1, 1), (32, 128, 8, 2), (32, 128, 9, 2), (32, 171, 24, 3),
+    (32, 170, 24, 3), (32, 128, 25, 4), (32, 1024, 40, 4), (32, 1024, 41, 4), (128, 1, 1, 1), (128, 3, 4, 1),
+    (128, 2, 5, 2), (128, 127, 8, 1), (128, 16, 8, 8), (128, 16, 9, 8)])
+def test_short_sequences(orc, g, dh, B, T, H, off):
+    # around the lines between the per-step kernels and the blocked ones for sequences
+    # of a few steps
+    _placed_parity(orc, dh, B, T, H, off)
