@@ -1,6 +1,6 @@
 // Internals shared by the delta-rule translation units (delta.hip: the
-// recurrent kernels on eight-lane column groups for the head widths that the
-// blocked form does not take, and the entry points; delta_ut64.hip,
+// recurrent kernels on eight-lane column groups for the head widths and the short
+// sequences that the blocked form does not take, and the entry points; delta_ut64.hip,
 // delta_ut64_b.hip, delta_utn.hip: the blocked form).
 #pragma once
 #include "common.h"

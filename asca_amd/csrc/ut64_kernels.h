@@ -55,8 +55,8 @@ constexpr int C = 16;          // steps per block; a checkpoint every 2 C steps
 // block would leave most CUs idle: NV = 2, the forward with two helper waves (a
 // wave per SIMD), the backward's partial dq, dk, dalpha, dbeta of the splits
 // added by delta_combine_k.  Bound: the chain of blocks (forward 1.4-1.9 us, backward
-// 2-6 us per 16 steps from dh = 16 to 128); the per-step kernels these replaced
-// walked the steps one by one: forward and fused backward of B8 T1000 H8 dh128
+// 2-6 us per 16 steps from dh = 16 to 128); the per-step kernels of these widths
+// (delta.hip: they keep sequences of a few steps) walk the steps one by one: forward and fused backward of B8 T1000 H8 dh128
 // 2627 -> 534 us, B4 T128 H4 dh32 76 -> 33, B32 T512 H8 dh48 667 -> 171, B32 T512
 // H8 dh96 7424 -> 700.  Each width is ten kernels with a register allocation of its
 // own to look after; 80 and 112 and the widths between have not been made.

@@ -140,16 +140,18 @@ ASCA_API void asca_rng_normal(uint64_t* state, float* out, size_t n, float scale
  * those widths also a record of 1344 floats per 16-step block and unit
  * (B*H*ceil(T/16)*1344 floats: the block's Gram products, triangular factors and
  * gate vectors), and at dh = 16, 32 and 48 never less than the other kernels'
- * layout (C = 8) takes.  It replaces the full state history
- * DeltaDev.states of
+ * layout (C = 8) takes.  Sequences of up to 40 steps at dh = 16 and 32 and of up
+ * to 8 at dh = 128 have, depending on B*H, the other widths' layout (C = 8, at
+ * dh = 128 C = 2).  It replaces the full state history DeltaDev.states of
  * rust/src/cuda/mod.rs:1274-1275,1386-1397 ((T+1)*dh*dh floats per unit).
  * dh may be 1..128.  The forward writes the workspace and the backwards only
  * read it, so several backwards may use one forward's workspace at once; what a
  * backward itself needs beside it comes from the scratch that the library keeps
  * for each stream (grown by the first call that needs more, with a quarter to
  * spare; a captured call's stays until the process ends, for its replays, which
- * must not run beside other calls on that stream): at the blocked widths B*H*S*ceil(T/16)*768 floats, and above dh = 64
- * 2*S*B*T*H*(dh + 1) more, S = dh/32 (else 1); at other widths
+ * must not run beside other calls on that stream): on the blocked kernels
+ * B*H*S*ceil(T/16)*768 floats, and above dh = 64 2*S*B*T*H*(dh + 1) more,
+ * S = dh/32 (else 1); at other widths and for those short sequences
  * 4*B*T*H*(dh + 1) where B*H <= 128 or dh > 64, else none. */
 ASCA_API int asca_delta_ws_bytes(int B, int T, int H, int dh, size_t* bytes);
 
